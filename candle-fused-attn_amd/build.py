@@ -19,8 +19,8 @@ REPO = PKG_DIR.parent
 CSRC = PKG_DIR / "csrc"
 LIB_DIR = PKG_DIR / "lib"
 LIB = LIB_DIR / "libfattn.so"
-SOURCES = [CSRC / "fattn_kernels.hip", CSRC / "fattn_api.cpp"]
-HEADERS = [REPO / "include" / "fattn.h", CSRC / "fattn_internal.h"]
+SOURCES = [CSRC / "fattn_kernels.hip", CSRC / "fattn_pair.hip", CSRC / "fattn_api.cpp"]
+HEADERS = [REPO / "include" / "fattn.h", CSRC / "fattn_internal.h", CSRC / "fattn_device.h"]
 # The C++ op layer over the C ABI (the reference's src/lib.rs ops for C++ callers), linked
 # against libfattn.so, and its test program (links the CPU oracle; test infrastructure).
 HOST = PKG_DIR / "host"

@@ -186,9 +186,8 @@ int check_range(const char* who, int64_t b, int64_t h, int64_t s, int64_t d) {
   }
   const int64_t grid_lim = (int64_t{1} << 32) / 256 - 1;
   const int dd = static_cast<int>(d);
-  if (fattn::forward_blocks(b, h, s, 1, dd) > grid_lim ||
-      fattn::forward_blocks(b, h, s, 0, dd) > grid_lim ||
-      fattn::bwd_main_blocks(b, h, s) + fattn::bwd_dq_blocks(b, h, s) + 8 > grid_lim ||
+  // (The forward's grid, one workgroup per 128 queries or more, is below step 2's.)
+  if (fattn::bwd_main_blocks(b, h, s) + fattn::bwd_dq_blocks(b, h, s) + 8 > grid_lim ||
       fattn::bwd_prep_blocks(b, h, s, dd) > grid_lim) {
     return fail(FATTN_ERANGE, std::string(who) + ": the grid for " + std::to_string(b) +
                                   " x " + std::to_string(h) + " x " + std::to_string(s) +
@@ -291,14 +290,7 @@ int run_bwd_prep(const char* who, const float* o, View d_o, void* ws, size_t ws_
   }
   WsParts p{};
   if (int rc = workspace_parts(who, ws, ws_bytes, b, h, s, d, &p)) return rc;
-  // split (d <= 64, and d 128 with few key blocks per (b, h)): step 2 computes D itself and its
-  // dQ sums need no clearing (epochs).
-  if (!fattn::bwd_needs_prep(p.part != nullptr, static_cast<int>(d), s)) return ok();
-  const int err = fattn::launch_bwd_prep(o, d_o, p.dsum, p.turn, p.ctrl, static_cast<int>(b),
-                                         static_cast<int>(h), static_cast<int>(s),
-                                         static_cast<int>(d), stream);
-  if (err) return hip_fail(err, "backward step 1 launch");
-  return ok();
+  return ok();  // step 2 forms D itself and needs nothing cleared
 }
 
 // Step 2's operand checks (nothing launched).
@@ -326,23 +318,13 @@ int run_bwd_main(const char* who, View q, View k, View v, const float* o, View d
   if (int rc = check_bwd_main(who, q, k, v, o, d_o, lse, dqkv, b, h, s, d)) return rc;
   WsParts p{};
   if (int rc = workspace_parts(who, ws, ws_bytes, b, h, s, d, &p)) return rc;
-  const int err = fattn::launch_bwd_main(q, k, v, d_o, o, lse, p.dsum, dqkv, p.part, p.arrive,
-                                         p.done, p.epoch, next_epoch(), p.turn, p.ctrl,
-                                         static_cast<int>(b), static_cast<int>(h),
-                                         static_cast<int>(s), static_cast<int>(d), scale,
-                                         causal ? 1 : 0, 0, static_cast<int>(b * h),
-                                         sums_final ? 1 : 0, stream);
+  const int err = fattn::launch_backward(
+      q, k, v, d_o, o, lse, dqkv, p.part, p.done, p.epoch, next_epoch(), p.ctrl,
+      static_cast<int>(b), static_cast<int>(h), static_cast<int>(s), static_cast<int>(d), scale,
+      causal ? 1 : 0, fattn::step2_deferred() ? 1 : 0, sums_final ? 1 : 0, fattn::give_up_pair(),
+      stream);
   if (err) return hip_fail(err, "backward step 2 launch");
   return ok();
-}
-
-// Whether `stream` is capturing a HIP graph (or that cannot be told): then step 3 runs after
-// step 2 even where step 2 sums every tile, because it also clears the sums' flags, which a
-// replay of the graph (the same epoch) needs.
-bool capturing(void* stream) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st) != hipSuccess) return true;
-  return st != hipStreamCaptureStatusNone;
 }
 
 // Step 3: in split mode (the workspace holds the partials) dQ from the partials; else nothing.
@@ -357,74 +339,45 @@ int run_bwd_dq(const char* who, float* dqkv, void* ws, size_t ws_bytes, int64_t 
   WsParts p{};
   if (int rc = workspace_parts(who, ws, ws_bytes, b, h, s, d, &p)) return rc;
   if (!p.part) return ok();
-  const int err = fattn::launch_bwd_dq(p.part, p.done, p.arrive, p.epoch, dqkv,
-                                       static_cast<int>(b), static_cast<int>(h),
-                                       static_cast<int>(s), static_cast<int>(d), scale,
-                                       causal ? 1 : 0, 0, static_cast<int>(b * h), stream);
+  const int err = fattn::launch_bwd_dq(p.part, p.done, p.epoch, dqkv, static_cast<int>(b),
+                                       static_cast<int>(h), static_cast<int>(s),
+                                       static_cast<int>(d), scale, stream);
   if (err) return hip_fail(err, "backward step 3 launch");
-  return ok();
-}
-
-// Steps 2 and 3 of the split sum over the (b, h) in chunks of `chunk` pairs, each chunk's
-// partials, arrival slots and done flags at the start of the workspace (no step 1 at d <= 64).
-int run_backward_chunked(const char* who, View q, View k, View v, const float* o, View d_o,
-                         const float* lse, float* dqkv, void* ws, size_t ws_bytes, int64_t b,
-                         int64_t h, int64_t s, int64_t d, float scale, int causal, int64_t chunk,
-                         void* stream) {
-  if (int rc = check_bwd_main(who, q, k, v, o, d_o, lse, dqkv, b, h, s, d)) return rc;
-  WsParts p{};
-  if (int rc = workspace_parts(who, ws, ws_bytes, 1, chunk, s, d, &p)) return rc;
-  if (!p.part) return fail(FATTN_EWORKSPACE, std::string(who) + ": workspace too small");
-  const bool eager = !capturing(stream);
-  for (int64_t bh0 = 0; bh0 < b * h; bh0 += chunk) {
-    const int n = static_cast<int>(std::min(chunk, b * h - bh0));
-    const bool final_sums =
-        eager && fattn::bwd_step2_sums_all(n, b, h, s, static_cast<int>(d), causal ? 1 : 0);
-    int err = fattn::launch_bwd_main(q, k, v, d_o, o, lse, p.dsum, dqkv, p.part, p.arrive, p.done,
-                                     p.epoch, next_epoch(), p.turn, p.ctrl, static_cast<int>(b),
-                                     static_cast<int>(h), static_cast<int>(s),
-                                     static_cast<int>(d), scale, causal ? 1 : 0,
-                                     static_cast<int>(bh0), n, final_sums ? 1 : 0, stream);
-    if (err) return hip_fail(err, "backward step 2 launch");
-    if (final_sums) continue;
-    err = fattn::launch_bwd_dq(p.part, p.done, p.arrive, p.epoch, dqkv, static_cast<int>(b),
-                               static_cast<int>(h), static_cast<int>(s), static_cast<int>(d),
-                               scale, causal ? 1 : 0, static_cast<int>(bh0), n, stream);
-    if (err) return hip_fail(err, "backward step 3 launch");
-  }
   return ok();
 }
 
 int run_backward(const char* who, View q, View k, View v, const float* o, View d_o,
                  const float* lse, float* dqkv, void* ws, size_t ws_bytes, int64_t b, int64_t h,
                  int64_t s, int64_t d, float scale, int causal, void* stream) {
-  // A workspace that holds the split sum of some (b, h) but not of all: the split sum by chunks
-  // where the chunks are large enough to beat the turn hand-over (or the workspace is too small
-  // for the turn hand-over's minimum).
   if (int rc = check_range(who, b, h, s, d)) return rc;
-  int64_t chunk = 0;
-  if (ws) {
-    chunk = fattn::split_chunk(b, h, s, d, ws_bytes,
-                               fattn::min_chunk_pairs(b, h, s, d, causal != 0), causal != 0);
-    if (chunk == 0 && ws_bytes < fattn::workspace_layout(b, h, s, d).bytes_min) {
-      chunk = fattn::split_chunk(b, h, s, d, ws_bytes, 1, causal != 0);
+  const fattn::Workspace l = fattn::workspace_layout(b, h, s, d);
+  if (ws && ws_bytes < l.bytes_split) {
+    // dQ goes straight to its rows: the control words are all that step 2 uses. A workspace below
+    // the minimum is taken where it holds the split state of a chunk of (b, h) pairs.
+    const bool chunk =
+        fattn::split_chunk(b, h, s, d, ws_bytes,
+                           fattn::min_chunk_pairs(b, h, s, d, causal != 0), causal != 0) > 0 ||
+        (ws_bytes < l.bytes_min && fattn::split_chunk(b, h, s, d, ws_bytes, 1, causal != 0) > 0);
+    if (ws_bytes >= l.bytes_min || chunk) {
+      if (int rc = check_bwd_main(who, q, k, v, o, d_o, lse, dqkv, b, h, s, d)) return rc;
+      if ((reinterpret_cast<uintptr_t>(ws) & 255u) == 0) {
+        const int err = fattn::launch_backward(
+            q, k, v, d_o, o, lse, dqkv, nullptr, nullptr, nullptr, 0, static_cast<int*>(ws),
+            static_cast<int>(b), static_cast<int>(h), static_cast<int>(s), static_cast<int>(d),
+            scale, causal ? 1 : 0, 0, 1, fattn::give_up_pair(), stream);
+        if (err) return hip_fail(err, "backward step 2 launch");
+        return ok();
+      }
     }
   }
-  if (chunk > 0 && chunk < b * h) {
-    return run_backward_chunked(who, q, k, v, o, d_o, lse, dqkv, ws, ws_bytes, b, h, s, d, scale,
-                                causal, chunk, stream);
-  }
-  if (int rc = run_bwd_prep(who, o, d_o, ws, ws_bytes, b, h, s, d, stream)) return rc;
-  // Step 3 only where step 2's sums may leave tiles (or a graph is being captured).
-  const bool final_sums = ws && ws_bytes >= fattn::workspace_layout(b, h, s, d).bytes_split &&
-                          fattn::bwd_step2_sums_all(b * h, b, h, s, static_cast<int>(d),
-                                                    causal ? 1 : 0) &&
-                          !capturing(stream);
+  // The whole split state (its done flags are kept; step 3 only where a test hook defers dQ), or a
+  // refusal.
+  const bool last = !fattn::step2_deferred();
   if (int rc = run_bwd_main(who, q, k, v, o, d_o, lse, dqkv, ws, ws_bytes, b, h, s, d, scale,
-                            causal, stream, final_sums)) {
+                            causal, stream, last)) {
     return rc;
   }
-  if (final_sums) return ok();
+  if (last) return ok();
   return run_bwd_dq(who, dqkv, ws, ws_bytes, b, h, s, d, scale, causal, stream);
 }
 
@@ -493,7 +446,7 @@ extern "C" {
 const char* fattn_last_error(void) { return g_error.c_str(); }
 
 const char* fattn_version(void) {
-  return "fattn-gfx950 0.2.0 (head_dim 32, 64, 128; fp32 MFMA)";
+  return "fattn-gfx950 0.2.0 (head_dim 32, 64, 128; fp32 by pairs of f16 MFMA)";
 }
 
 size_t fattn_bwd_workspace_bytes(int64_t b, int64_t h, int64_t s, int64_t d) {

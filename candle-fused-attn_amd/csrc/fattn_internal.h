@@ -162,53 +162,34 @@ int set_sum_shift(int shift);
 // before their first poll in every later launch, as a wait that timed out would; returns the
 // previous pair.
 int set_give_up_bh(int bh);
+// What the hooks ask of a launch: dQ deferred to step 3 (step 2's sums off), the give-up pair.
+bool step2_deferred();
+int give_up_pair();
 // The three hooks' current settings: step 2's sums on, the sum shift, the give-up pair.
 void test_hook_state(int64_t out[3]);
-// Step 3's grid: one workgroup per query tile, or (with step 2's sums) at most 256 workgroups
-// that each check a range of tiles and sum those not done.
-int64_t bwd_dq_grid(int64_t b, int64_t h, int64_t s, int d, int causal);
-
-// Launchers (fattn_kernels.hip). They assume validated arguments; they return a hipError_t
+// Launchers (fattn_pair.hip: the forward; fattn_kernels.hip). They assume validated arguments; they return a hipError_t
 // value as int (0 = launched).
 int launch_forward(View q, View k, View v, float* o, float* lse, int b, int h, int s, int d,
                    float scale, int causal, void* stream);
-int launch_bwd_prep(const float* o, View d_o, float* dsum, int* turn, int* ctrl, int b, int h,
-                    int s, int d, void* stream);
-// part == nullptr: the turn hand-over (dQ final after step 2; D from step 1); else the split
-// partials, which step 3 (launch_bwd_dq) sums into dQ (D computed from o here, no step 1).
-// arrive / done / epoch_slot (split, d <= 64): step 2's dQ sums, tagged with `epoch`.
-// bh0, nbh (split, d <= 64): the (b, h) pairs bh0 .. bh0 + nbh - 1 only, whose partials, slots
-// and flags sit in a workspace laid out for nbh pairs (workspace_layout(1, nbh, s, d)); otherwise
-// 0 and b h.
-int launch_bwd_main(View q, View k, View v, View d_o, const float* o, const float* lse,
-                    const float* dsum, float* dqkv, float* part, unsigned long long* arrive,
-                    unsigned long long* done, unsigned long long* epoch_slot,
-                    unsigned long long epoch, int* turn, int* ctrl, int b, int h, int s, int d,
-                    float scale, int causal, int bh0, int nbh, int sums_final, void* stream);
-// Whether step 2's sums cover every query tile of a launch over nbh of the b h pairs (then no
-// step 3 need follow it).
-bool bwd_step2_sums_all(int64_t nbh, int64_t b, int64_t h, int64_t s, int d, int causal);
-// Step 3: dQ of every query tile that step 2 did not sum (done: null, none did); then the done
-// flags and arrival slots are zeroed. bh0, nbh: as step 2's.
-int launch_bwd_dq(const float* part, unsigned long long* done, unsigned long long* arrive,
-                  const unsigned long long* epoch_slot, float* dqkv, int b, int h, int s, int d,
-                  float scale, int causal, int bh0, int nbh, void* stream);
+// Backward, step 2 (fattn_pair.hip): dK, dV and dQ. part, done, epoch_slot (a split-size workspace,
+// else null): with `defer` dQ goes to `part` for step 3, else to its rows, and `done` takes `epoch`
+// per 16-query tile. last: no step 3 follows. give_up_bh: a test hook's pair (-1: none).
+int launch_backward(View q, View k, View v, View d_o, const float* o, const float* lse, float* dqkv,
+                    float* part, unsigned long long* done, unsigned long long* epoch_slot,
+                    unsigned long long epoch, int* ctrl, int b, int h, int s, int d, float scale,
+                    int causal, int defer, int last, int give_up_bh, void* stream);
+// Step 3: dQ of every query tile that step 2 left in the workspace; the flags are zeroed.
+int launch_bwd_dq(const float* part, unsigned long long* done, const unsigned long long* epoch_slot,
+                  float* dqkv, int b, int h, int s, int d, float scale, void* stream);
 
 // The device address of the library's static scratch (FATTN_STATIC_SCRATCH_BYTES, the workspace
 // of fattn_bwd_f32_noalloc) on the device that runs `stream`; a hipError_t value as int.
 int static_scratch(void* stream, void** out);
 
 // Grid sizes the launchers will use (for range checks before launching).
-int64_t forward_blocks(int64_t b, int64_t h, int64_t s, int causal, int d);
 int64_t bwd_main_blocks(int64_t b, int64_t h, int64_t s);
 int64_t bwd_prep_blocks(int64_t b, int64_t h, int64_t s, int d);
 int64_t bwd_dq_blocks(int64_t b, int64_t h, int64_t s);
-// Whether step 1 (D, counters) must run: the turn mode, and the split mode at d 128 past
-// kOwnDMaxBlocks key blocks per (b, h) (fewer: its step 2 forms D itself).
-bool bwd_needs_prep(bool split, int d, int64_t s);
-// D 128, split: step 2 forms D = rowsum(dO o O) itself (few key blocks per (b, h)).
-bool bwd_own_d(int64_t s, int d);
-
 }  // namespace fattn
 
 #endif  // FATTN_INTERNAL_H

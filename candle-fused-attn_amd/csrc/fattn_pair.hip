@@ -1,0 +1,1395 @@
+// fp32 attention on the f16 matrix cores. Every fp32 operand, times a power of two, is held as the
+// sum of two f16 terms, x 2^k = h + l (h rounded to nearest, l the rest rounded to nearest: 22 bits
+// and the sign of l), and a product is accumulated in fp32 as three f16 products,
+//   h l' + l h' + h h'
+// (l l' is below 2^-22 of the product with a random sign, as is what l drops).
+//
+// Why: v_mfma_f32_32x32x16_f16 runs at 16 times the rate of the fp32 v_mfma_f32_16x16x4_f32
+// (measured on MI355X, 4 waves per SIMD: 2.27 PFLOP/s against 151 TFLOP/s), so three of them take
+// a fifth of the time, and unlike the fp32 one they run beside the VALU (six VALU instructions per
+// MFMA are free with two waves per SIMD; beside the fp32 MFMA each adds its whole issue time). The
+// sums are no less accurate, since one rounding covers 16 contracted values instead of 4: N(0, 1)
+// dot products against fp64, normwise, 32 / 64 / 128 terms: 8.8e-8 / 9.5e-8 / 1.08e-7, the fp32
+// instruction 1.02e-7 / 1.44e-7 / 2.03e-7. (Three bf16 terms with six products hold all 24 bits,
+// 4.6e-8 at 64 terms, but twice the products run into the power limit: the clock fell to 1.82 GHz
+// where the fp32 kernel holds 2.41, and the forward at b 16 h 16 s 1024 took 352 us against 524.)
+//
+// Scales. f16 spans 2^-14 .. 2^16 (normal), so operands carry exact powers of two: a wave's own
+// rows (register operands) one per row, a staged 32-row tile one per tile, from the largest
+// magnitude in it: the stored maximum is in [2^13, 2^14), and an element keeps its 22 bits down to
+// 2^-17 of that maximum (below, an absolute error of 2^-39 of it). The scales multiply back into
+// factors the softmax applies anyway; sums over several tiles follow a running maximum of the
+// tiles' exponents.
+//
+// For one v_mfma_f32_32x32x16_f16, lane l (j = l % 32, g = l / 32) supplies A[j][8 g + e] and
+// B[8 g + e][j], e = 0..7, and holds D[8 (r / 4) + 4 g + r % 4][j], r = 0..15. As the contraction
+// order is free (A and B alike), eight consecutive accumulator registers of one product are the B
+// operand of the next one over 16 of its rows: step ks, element e is row
+//   16 ks + 4 g + e (e < 4),  16 ks + 8 + 4 g + e - 4 (e >= 4).
+// A operands are read from LDS, where a tile of 32 rows is held as two f16 planes [32][D]: by rows
+// (ds_read_b128: 8 columns of row j), or transposed (two ds_read_b64_tr_b16: 4 + 4 rows of column
+// j, in the order above). 16-byte chunk c of row r sits at chunk c ^ chunk_swz(r).
+//
+// Values the split cannot carry (infinities, NaN) show as a non-finite result; a wave that finds
+// one computes its rows again in plain fp32.
+#include <hip/hip_runtime.h>
+#include <math.h>
+#include <stddef.h>
+#include <stdint.h>
+
+#include "fattn_device.h"
+#include "fattn_internal.h"
+
+namespace fattn {
+namespace {
+
+typedef float f16v __attribute__((ext_vector_type(16)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
+typedef short s4 __attribute__((ext_vector_type(4)));
+
+constexpr int kRows = 32;  // rows of a staged tile, and of a wave's own operand
+constexpr int kTop = 13;   // the scaled maximum lies in [2^kTop, 2^(kTop + 1))
+
+__device__ __forceinline__ f16v mma(h8 a, h8 b, f16v c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f16v zero16() { return f16v{}; }
+
+// 2^e, -126 <= e <= 127.
+__device__ __forceinline__ float pow2(int e) { return __int_as_float((e + 127) << 23); }
+// The exponent of a magnitude, at least -100 (so that every scale below is a normal float).
+__device__ __forceinline__ int exponent(float x) {
+  return max(static_cast<int>((__float_as_uint(x) >> 23) & 255u) - 127, -100);
+}
+
+// The scale of a tile whose largest magnitude has exponent e. A tile with an infinity (exponent 128)
+// becomes NaN as a whole: its other rows would vanish beside it, unseen where its own is masked.
+__device__ __forceinline__ float tile_scale(int e) {
+  return e == 128 ? __builtin_nanf("") : pow2(kTop - e);
+}
+
+// Eight values times a scale, in two terms.
+struct Pair {
+  h8 h, l;
+};
+__device__ __forceinline__ Pair make_pair8(const unsigned* h, const unsigned* l) {
+  return Pair{__builtin_bit_cast(h8, u4{h[0], h[1], h[2], h[3]}),
+              __builtin_bit_cast(h8, u4{l[0], l[1], l[2], l[3]})};
+}
+// x sc = h + l, two values: four instructions (v_fma_mixlo / mixhi_f16 scale, subtract and round in
+// one). The empty asm makes the compiler take l's subtrahend from the packed h instead of
+// converting each value a second time.
+__device__ __forceinline__ void split2(float x, float y, float sc, unsigned& h, unsigned& l) {
+  const h2 a{static_cast<_Float16>(fmaf(x, sc, 0.0f)), static_cast<_Float16>(fmaf(y, sc, 0.0f))};
+  h = __builtin_bit_cast(unsigned, a);
+  asm("" : "+v"(h));
+  const h2 b = __builtin_bit_cast(h2, h);
+  const h2 c{static_cast<_Float16>(fmaf(x, sc, -static_cast<float>(b.x))),
+             static_cast<_Float16>(fmaf(y, sc, -static_cast<float>(b.y)))};
+  l = __builtin_bit_cast(unsigned, c);
+}
+// x = h + l, two values: three instructions.
+__device__ __forceinline__ void split2(float x, float y, unsigned& h, unsigned& l) {
+  h = __builtin_bit_cast(unsigned, __builtin_convertvector(f2{x, y}, h2));
+  asm("" : "+v"(h));
+  const h2 b = __builtin_bit_cast(h2, h);
+  const h2 c{static_cast<_Float16>(fmaf(static_cast<float>(b.x), -1.0f, x)),
+             static_cast<_Float16>(fmaf(static_cast<float>(b.y), -1.0f, y))};
+  l = __builtin_bit_cast(unsigned, c);
+}
+__device__ __forceinline__ Pair split8(f4 x, f4 y, float sc) {
+  unsigned h[4], l[4];
+  split2(x[0], x[1], sc, h[0], l[0]);
+  split2(x[2], x[3], sc, h[1], l[1]);
+  split2(y[0], y[1], sc, h[2], l[2]);
+  split2(y[2], y[3], sc, h[3], l[3]);
+  return make_pair8(h, l);
+}
+// Registers 8 KS .. 8 KS + 7 of an accumulator as a B operand.
+template <int KS>
+__device__ __forceinline__ Pair split_acc(const f16v& x) {
+  unsigned h[4], l[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) split2(x[8 * KS + 2 * i], x[8 * KS + 2 * i + 1], h[i], l[i]);
+  return make_pair8(h, l);
+}
+__device__ __forceinline__ f16v mma_small(const Pair& a, const Pair& b, f16v c) {
+  c = mma(a.h, b.l, c);
+  return mma(a.l, b.h, c);
+}
+__device__ __forceinline__ f16v mma3(const Pair& a, const Pair& b, f16v c) {
+  return mma(a.h, b.h, mma_small(a, b, c));
+}
+
+// --- LDS tiles ---------------------------------------------------------------------------------
+// The 16-byte chunk a row's chunk 0 moves to, linear over xor in the row's low four bits: the maps
+// that took the fewest cycles over all of them, measured for the two read patterns and the staging
+// writes together (128 of each by four waves, D 64: row reads 5276 cycles, transposed 3648, writes
+// 6636; bit-reversed low three bits: 6020, 4000, 6684).
+template <int D>
+constexpr int kSwz8 = D == 32 ? 3 : D == 64 ? 1 : 7;  // of row 8
+template <int D>
+__device__ __forceinline__ int chunk_swz(int row) {
+  constexpr int f1 = D == 32 ? 1 : D == 64 ? 2 : 11, f2 = D == 32 ? 0 : D == 64 ? 5 : 15;
+  constexpr int f4 = D == 32 ? 2 : D == 64 ? 6 : 10;
+  return ((row & 1) ? f1 : 0) ^ ((row & 2) ? f2 : 0) ^ ((row & 4) ? f4 : 0) ^
+         ((row & 8) ? kSwz8<D> : 0);
+}
+template <int D>
+struct Tile {
+  _Float16 p[2][kRows * D];  // planes h, l
+};
+template <int D>
+constexpr int kPlane = kRows * D * 2;  // bytes
+
+// Row j = lane % 32's columns 16 ks + 8 g .. + 7.
+template <int D>
+__device__ __forceinline__ int row_off(int j, int g, int ks) {
+  return j * (2 * D) + (((2 * ks + g) ^ chunk_swz<D>(j)) << 4);
+}
+template <int D>
+__device__ __forceinline__ Pair ld_row(const Tile<D>& t, int off) {
+  const char* p = reinterpret_cast<const char*>(&t) + off;
+  return Pair{*reinterpret_cast<const h8*>(p), *reinterpret_cast<const h8*>(p + kPlane<D>)};
+}
+// The lane's base offset of the transposed read of columns 32 dt + lane % 32: within each group of
+// 16 lanes, lane i points at row i / 4 and columns 4 (i % 4) .. + 3 of a 4 x 16 block and receives
+// the block's column i. Rows 16 ks + 4 g + (0..3) at + 32 D ks bytes; 8 rows on, + 16 D bytes and
+// the chunk of the offset changed by kSwz8.
+template <int D>
+__device__ __forceinline__ int col_off(int lane, int dt) {
+  const int i = lane & 15, hi = (lane >> 4) & 1, g = lane >> 5;
+  const int row = 4 * g + (i >> 2);
+  const int chunk = 4 * dt + 2 * hi + ((i & 3) >> 1);
+  return row * (2 * D) + ((chunk ^ chunk_swz<D>(row)) << 4) + ((i & 1) << 3);
+}
+template <int D>
+__device__ __forceinline__ h8 ld_tr(const char* t, int off) {
+  typedef __attribute__((address_space(3))) s4 lds_s4;
+  const s4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(t + off));
+  const s4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (lds_s4*)(t + 16 * D + (off ^ (kSwz8<D> << 4))));
+  return __builtin_bit_cast(h8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+template <int D>
+__device__ __forceinline__ Pair ld_col(const Tile<D>& t, int off, int ks) {
+  const char* p = reinterpret_cast<const char*>(&t) + 32 * D * ks;
+  return Pair{ld_tr<D>(p, off), ld_tr<D>(p + kPlane<D>, off)};
+}
+
+// --- Lane exchanges ----------------------------------------------------------------------------
+// The sum over a lane and lane ^ 32 (both get the same bits), and the max.
+__device__ __forceinline__ float pair_sum(float x) {
+  const unsigned u = __float_as_uint(x);
+  const auto p = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+__device__ __forceinline__ float pair_max(float x) {
+  const unsigned u = __float_as_uint(x);
+  const auto p = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return vmax(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+// The max over each half of the wave.
+__device__ __forceinline__ float half_max(float x) {
+  x = fmaxf(x, dpp<0xB1>(x));
+  x = fmaxf(x, dpp<0x4E>(x));
+  x = fmaxf(x, dpp<0x141>(x));
+  x = fmaxf(x, dpp<0x140>(x));
+  const unsigned u = __float_as_uint(x);
+  const auto p = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return vmax(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+__device__ __forceinline__ float wave_sum(float x) {
+#pragma unroll
+  for (int i = 1; i < 64; i <<= 1) x += __shfl_xor(x, i);
+  return x;
+}
+__device__ __forceinline__ float wave_max(float x) {
+#pragma unroll
+  for (int i = 1; i < 64; i <<= 1) x = fmaxf(x, __shfl_xor(x, i));
+  return x;
+}
+// max(m, |x|, |y|) over eight values: four v_max3_f32 with absolute operands (from fmaxf the
+// compiler makes eight and quiets every input first). For loaded values; NaN is passed over.
+__device__ __forceinline__ float abs_max8(f4 x, f4 y, float m) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(x[i]), "v"(y[i]));
+  return m;
+}
+// No memory access moves across: a step's loads are issued before its LDS reads (left to itself the
+// compiler sinks them to their first use, at the end of the step).
+__device__ __forceinline__ void pin_loads() { asm volatile("" ::: "memory"); }
+// No instruction moves across: keeps the compiler from overlapping phases whose registers together
+// do not fit.
+__device__ __forceinline__ void fence_phase() { __builtin_amdgcn_sched_barrier(0); }
+// 0 where every value is finite, else NaN.
+template <int N>
+__device__ __forceinline__ float probe_finite(const f16v (&x)[N], float z) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) z = fmaf(x[i][r], 0.0f, z);
+  }
+  return z;
+}
+
+// --- Staging -----------------------------------------------------------------------------------
+// Two operands' tiles of 32 rows through the registers of a workgroup of four waves: wave w takes
+// rows 8 w .. 8 w + 7 of both (D 32: operand a in lanes 0..31, b in the others), eight columns per
+// lane and access. A tile is loaded in one step of the walk, its maxima (one per wave and operand)
+// go to LDS at the end of that step, and after the step's barrier the next step scales, splits and
+// stores it.
+struct Operand {
+  const char* p;  // row 0 of the (b, h)
+  unsigned ss4;   // row stride in bytes
+};
+struct Maxima {
+  float m[2][2][4];  // by the step's parity, operand and wave
+};
+template <int D>
+struct Stage {
+  static constexpr int kC = D / 8;                // chunks per row
+  static constexpr int kN = D == 32 ? 1 : D / 32;  // accesses per lane: a's, then b's
+  f4 x[kN][2];
+
+  static __device__ __forceinline__ int row(int i, int w, int lane) {
+    if constexpr (D == 32) return 8 * w + (lane & 31) / kC;
+    return 8 * w + (64 / kC) * (i % (kN / 2)) + lane / kC;
+  }
+  // Rows past `last` repeat it (finite where the operand is; masked by the reader).
+  __device__ __forceinline__ void load(const Operand& a, const Operand& b, int r0, int last, int w,
+                                       int lane) {
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+      const bool is_b = kN == 1 ? lane >= 32 : i >= kN / 2;
+      const unsigned r = static_cast<unsigned>(min(r0 + row(i, w, lane), last));
+      const char* p = is_b ? b.p : a.p;
+      const unsigned off =
+          r * (is_b ? b.ss4 : a.ss4) + 32u * static_cast<unsigned>(lane % kC);
+      x[i][0] = *reinterpret_cast<const f4*>(p + off);
+      x[i][1] = *reinterpret_cast<const f4*>(p + off + 16);
+    }
+  }
+  __device__ __forceinline__ void put_maxima(Maxima& mx, int parity, int w, int lane) const {
+    float m;
+    if constexpr (kN == 1) {
+      m = fmaxf(abs_max8(x[0][0], x[0][1], 0.0f), 0.0f);
+    } else {
+      float ma = 0.0f, mb = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kN; ++i) {
+        float& t = i < kN / 2 ? ma : mb;
+        t = abs_max8(x[i][0], x[i][1], t);
+      }
+      // a's into the lower half, b's into the upper. (The swaps must not read an asm's result: the
+      // compiler counts their wait states from the instructions it knows.)
+      ma = fmaxf(ma, 0.0f), mb = fmaxf(mb, 0.0f);
+      const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(ma), __float_as_uint(mb),
+                                                      false, false);
+      m = vmax(__uint_as_float(p[0]), __uint_as_float(p[1]));
+    }
+    m = half_max(m);
+    if ((lane & 31) == 0) mx.m[parity][lane >> 5][w] = m;
+  }
+  __device__ __forceinline__ void store(Tile<D>& a, Tile<D>& b, float sa, float sb, int w,
+                                        int lane) const {
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+      const bool is_b = kN == 1 ? lane >= 32 : i >= kN / 2;
+      const int r = row(i, w, lane);
+      const Pair s = split8(x[i][0], x[i][1], is_b ? sb : sa);
+      char* p = reinterpret_cast<char*>(is_b ? &b : &a) + r * (2 * D) +
+                (((lane % kC) ^ chunk_swz<D>(r)) << 4);
+      *reinterpret_cast<h8*>(p) = s.h;
+      *reinterpret_cast<h8*>(p + kPlane<D>) = s.l;
+    }
+  }
+};
+// Beside a Stage whose operand b is dO: O's rows in the same lanes, and D = rowsum(dO o O) of the
+// tile's 32 rows.
+template <int D>
+struct RowDots {
+  static constexpr int kC = D / 8, kN = D == 128 ? 2 : 1;
+  f4 x[kN][2];
+  __device__ __forceinline__ void load(const Operand& o, int r0, int last, int w, int lane) {
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+      const unsigned r = static_cast<unsigned>(min(r0 + Stage<D>::row(i, w, lane), last));
+      const unsigned off = r * o.ss4 + 32u * static_cast<unsigned>(lane % kC);
+      x[i][0] = *reinterpret_cast<const f4*>(o.p + off);
+      x[i][1] = *reinterpret_cast<const f4*>(o.p + off + 16);
+    }
+  }
+  __device__ __forceinline__ void put(const Stage<D>& st, float* dst, int w, int lane) const {
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+      const f4(&y)[2] = st.x[Stage<D>::kN / 2 + i];
+      float t = x[i][0][0] * y[0][0];
+#pragma unroll
+      for (int e = 1; e < 8; ++e) t = fmaf(x[i][e / 4][e % 4], y[e / 4][e % 4], t);
+      t += dpp<0xB1>(t);
+      t += dpp<0x4E>(t);
+      if constexpr (D >= 64) t += dpp<0x141>(t);
+      if constexpr (D == 128) t += dpp<0x140>(t);
+      if (lane % kC == 0 && (D != 32 || lane >= 32)) dst[Stage<D>::row(i, w, lane)] = t;
+    }
+  }
+};
+// The exponent of operand `o`'s staged tile (wave-uniform).
+__device__ __forceinline__ int tile_exponent(const Maxima& mx, int parity, int o) {
+  const f4 m = *reinterpret_cast<const f4*>(mx.m[parity][o]);
+  const float x = fmaxf(fmaxf(m.x, m.y), fmaxf(m.z, m.w));
+  return exponent(__int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))));
+}
+// A wave's own 32 rows as B operands: row j, columns 16 ks + 8 g .. + 7 of each step, scaled per
+// row (lanes j and j + 32 hold one row). Returns 1 / scale (without `sign`).
+template <int D>
+struct OwnRows {
+  f4 x[D / 16][2];
+  __device__ __forceinline__ void load(const float* row, int g) {
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+      x[ks][0] = ld4(row + 16 * ks + 8 * g);
+      x[ks][1] = ld4(row + 16 * ks + 8 * g + 4);
+    }
+  }
+  __device__ __forceinline__ float split(float sign, Pair (&dst)[D / 16]) const {
+    float m = 0.0f;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) m = abs_max8(x[ks][0], x[ks][1], m);
+    const int e = exponent(pair_max(fmaxf(m, 0.0f)));
+    const float sc = pow2(kTop - e) * sign;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) dst[ks] = split8(x[ks][0], x[ks][1], sc);
+    return pow2(e - kTop);
+  }
+};
+
+// --- Forward -----------------------------------------------------------------------------------
+// One workgroup = 4 waves of one (b, h), NQ groups of 32 queries per wave; key tiles of 32 keys,
+// split into LDS by all four waves (each value split once per workgroup). Per wave, tile and group:
+//   S^T = K Q^T (A = K rows, B = Q in registers): lane (j, g), register r holds the score of query
+//   j and key 8 (r / 4) + 4 g + r % 4, so a query's online softmax is one lane's and lane ^ 32's;
+//   O^T += V^T P^T (A = V transposed, B = P from S^T's registers).
+// Two LDS buffers, one barrier per tile: a step works on tile t, stores tile t + 1 and loads tile
+// t + 2.
+// The softmax: p = 2^(s c2 - m), c2 = |scale| log2 e and the two operands' scales, m a reference
+// that is kRefTop below the largest score seen when it was set. p is computed with the m in hand
+// and its row sum is what is tested: only where it exceeds kRowTop (or m is not set yet) is the
+// tile's max taken, m moved, O and the row sum rescaled and p computed again, so that an ordinary
+// tile pays neither a max nor a rescale, and every p stays below f16's limit.
+constexpr float kRefTop = 3.0f;
+constexpr float kRowTop = 32768.0f;
+
+// One query's output row and L in plain fp32 by one wave: lanes take keys for the scores and dims
+// for the output.
+template <int D>
+__device__ void fwd_row_fp32(const FwdArgs& a, int b, int h, int qi, int lane) {
+  const float* qp = a.q.p + b * a.q.sb + h * a.q.sh + static_cast<int64_t>(qi) * a.q.ss;
+  const float* kp = a.k.p + b * a.k.sb + h * a.k.sh;
+  const float* vp = a.v.p + b * a.v.sb + h * a.v.sh;
+  const float sign = a.scale < 0.0f ? -1.0f : 1.0f, c2 = fabsf(a.scale) * kLog2e;
+  const int kend = a.causal ? qi + 1 : a.S;
+  constexpr int kND = (D + 63) / 64;
+  float m = kNegInf, l = 0.0f, o[kND] = {};
+  for (int k0 = 0; k0 < kend; k0 += 64) {
+    const int key = k0 + lane;
+    float s = kNegInf;
+    if (key < kend) {
+      const float* kr = kp + static_cast<int64_t>(key) * a.k.ss;
+      s = 0.0f;
+      for (int c = 0; c < D; ++c) s = fmaf(sign * qp[c], kr[c], s);
+    }
+    const float mn = fmaxf(m, wave_max(s));
+    const float alpha = mn == m ? 1.0f : m == kNegInf ? 0.0f : exp2_hw((m - mn) * c2);
+    const float p = s == kNegInf ? 0.0f : exp2_hw(fmaf(s, c2, -(mn * c2)));
+    m = mn;
+    l = l * alpha + wave_sum(p);
+#pragma unroll
+    for (int i = 0; i < kND; ++i) o[i] *= alpha;
+    const int n = min(64, kend - k0);
+    for (int kk = 0; kk < n; ++kk) {
+      const float pk = __shfl(p, kk);
+      const float* vr = vp + static_cast<int64_t>(k0 + kk) * a.v.ss;
+#pragma unroll
+      for (int i = 0; i < kND; ++i) {
+        const int c = 64 * i + lane;
+        if (c < D) o[i] = fmaf(pk, vr[c], o[i]);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kND; ++i) {
+    const int c = 64 * i + lane;
+    if (c < D) a.o[((static_cast<int64_t>(b) * a.S + qi) * a.H + h) * D + c] = o[i] / l;
+  }
+  if (lane == 0) {
+    a.lse[(static_cast<int64_t>(b) * a.H + h) * a.S + qi] = m * fabsf(a.scale) + logf(l);
+  }
+}
+
+template <int D, bool kCausal, int NQ, int WAVES>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))
+fwd_pair_kernel(FwdArgs a) {
+  a.causal = kCausal ? 1 : 0;
+  constexpr int kKS = D / 16;              // contraction steps of S
+  constexpr int kDT = D / 32;              // 32-dim tiles of O
+  constexpr int kOCols = D < 64 ? D : 64;  // columns per pass of the output's transpose
+  constexpr int kOPitch = kOCols + 4;
+  constexpr int kWaveQ = kRows * NQ, kQ = 4 * kWaveQ;
+  struct Kv {
+    Tile<D> k, v;
+  };
+  union Tiles {
+    Kv kv[2];
+    float o[4][kRows * kOPitch];
+  };
+  struct Smem {
+    Tiles t;
+    Maxima mx;
+  };
+  __shared__ __attribute__((aligned(16))) Smem sm;
+
+  const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, g = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int S = a.S, BH = a.B * a.H;
+  int qb, bh;
+  if (kCausal) {
+    qb = a.nqb - 1 - static_cast<int>(blockIdx.x) / BH;  // the most expensive first
+    bh = static_cast<int>(blockIdx.x) % BH;
+  } else {
+    const int id = xcd_remap(static_cast<int>(blockIdx.x), a.nqb * BH);
+    qb = id % a.nqb;
+    bh = id / a.nqb;
+  }
+  const int b = bh / a.H, h = bh % a.H;
+  const int q0 = qb * kQ, qw0 = q0 + w * kWaveQ;
+  const float* qp = a.q.p + b * a.q.sb + h * a.q.sh;
+  const Operand kop{reinterpret_cast<const char*>(a.k.p + b * a.k.sb + h * a.k.sh),
+                    static_cast<unsigned>(a.k.ss) * 4u};
+  const Operand vop{reinterpret_cast<const char*>(a.v.p + b * a.v.sb + h * a.v.sh),
+                    static_cast<unsigned>(a.v.ss) * 4u};
+
+  const int k_end = kCausal ? min(S, q0 + kQ) : S;
+  const int ntiles = (k_end + kRows - 1) / kRows;
+  const int kw_end = kCausal ? min(S, qw0 + kWaveQ) : S;  // keys this wave's queries can see
+  const bool wave_live = qw0 < S;
+
+  // The first tile, the wave's queries (negated for a negative scale, so that the raw scores' max
+  // is the scaled scores'), and the second tile's loads. ek, ev: the exponents that tiles t, t + 1
+  // are scaled by; V's is the largest so far (its tiles are summed into one accumulator).
+  Stage<D> st;
+  Pair q[NQ][kKS];
+  float cq[NQ];  // |scale| log2 e over the query's scale
+  int ek[2], ev[2];
+  {
+    OwnRows<D> own[NQ];
+    st.load(kop, vop, 0, S - 1, w, lane);
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) own[n].load(qp + min(qw0 + kRows * n + j, S - 1) * a.q.ss, g);
+    st.put_maxima(sm.mx, 0, w, lane);
+    __syncthreads();
+    ek[0] = tile_exponent(sm.mx, 0, 0);
+    ev[0] = tile_exponent(sm.mx, 0, 1);
+    st.store(sm.t.kv[0].k, sm.t.kv[0].v, tile_scale(ek[0]), tile_scale(ev[0]), w, lane);
+    st.load(kop, vop, kRows, S - 1, w, lane);
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+      cq[n] = own[n].split(a.scale < 0.0f ? -1.0f : 1.0f, q[n]) * (fabsf(a.scale) * kLog2e);
+    }
+    st.put_maxima(sm.mx, 1, w, lane);
+    ek[1] = ek[0], ev[1] = ev[0];
+  }
+
+  f16v acc[NQ][kDT];  // O^T, in units of p and 2^(e_o - kTop)
+  int e_o = ev[0];
+  float m[NQ], lsum[NQ];
+#pragma unroll
+  for (int n = 0; n < NQ; ++n) {
+    m[n] = kNegInf;
+    lsum[n] = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < kDT; ++dt) acc[n][dt] = zero16();
+  }
+  int roff[kKS], coff[kDT];
+#pragma unroll
+  for (int ks = 0; ks < kKS; ++ks) roff[ks] = row_off<D>(j, g, ks);
+#pragma unroll
+  for (int dt = 0; dt < kDT; ++dt) coff[dt] = col_off<D>(lane, dt);
+
+  // Stores tile t + 1 (loaded in the last step) and issues the loads of tile t + 2.
+  auto stage = [&](int t, Kv& put) {
+    ek[1] = tile_exponent(sm.mx, (t + 1) & 1, 0);
+    ev[1] = max(tile_exponent(sm.mx, (t + 1) & 1, 1), ev[0]);
+    st.store(put.k, put.v, tile_scale(ek[1]), tile_scale(ev[1]), w, lane);
+    st.load(kop, vop, (t + 2) * kRows, S - 1, w, lane);
+    pin_loads();
+  };
+  // One tile: kFull, one with no mask. (Past the walk's end a step stages rows that repeat the last
+  // one and nothing reads: tested for, the loaded registers would live across the whole step.)
+  auto tile = [&](auto fullc, int t, const Kv& cur, Kv& put) {
+    constexpr bool kFull = decltype(fullc)::value != 0;
+    const int kt0 = t * kRows;
+    if (ev[0] > e_o) {  // wave-uniform: V's largest exponent grows (by the tiles this wave uses)
+      const float f = e_o - ev[0] < -126 ? 0.0f : pow2(e_o - ev[0]);
+      e_o = ev[0];
+#pragma unroll
+      for (int n = 0; n < NQ; ++n) {
+#pragma unroll
+        for (int dt = 0; dt < kDT; ++dt) acc[n][dt] *= f;
+      }
+    }
+    stage(t, put);
+    f16v s[NQ];
+    {
+      h8 kh[kKS];
+#pragma unroll
+      for (int n = 0; n < NQ; ++n) s[n] = zero16();
+#pragma unroll
+      for (int ks = 0; ks < kKS; ++ks) {
+        const Pair k = ld_row<D>(cur.k, roff[ks]);
+        kh[ks] = k.h;
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) s[n] = mma_small(k, q[n][ks], s[n]);
+      }
+#pragma unroll
+      for (int ks = 0; ks < kKS; ++ks) {
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) s[n] = mma(kh[ks], q[n][ks].h, s[n]);
+      }
+    }
+    Pair p[NQ][2];
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+      const int qi = qw0 + kRows * n + j;
+      const float c2 = cq[n] * pow2(ek[0] - kTop);
+      // Live: keys below S and, causal, not after the query.
+      auto live = [&](int r) {
+        const int key = kt0 + 8 * (r >> 2) + 4 * g + (r & 3);
+        return kFull || (key < S && !(kCausal && key > qi));
+      };
+      f16v e;
+      float psum = 0.0f;
+      auto exps = [&] {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float x = exp2_hw(fmaf(s[n][r], c2, -m[n]));
+          e[r] = live(r) ? x : 0.0f;
+          psum = r == 0 ? e[r] : psum + e[r];
+        }
+      };
+      exps();
+      if (__builtin_amdgcn_ballot_w64(!(psum <= kRowTop)) != 0) {
+        float tmax = kNegInf;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, live(r) ? s[n][r] : kNegInf);
+        tmax = pair_max(tmax);
+        // (c2 may be 0: a row with no live key keeps -inf.)
+        const float ref = tmax == kNegInf ? kNegInf : fmaf(tmax, c2, -kRefTop);
+        if (ref > m[n]) {
+          const float alpha = m[n] == kNegInf ? 0.0f : exp2_hw(m[n] - ref);
+          m[n] = ref;
+          lsum[n] *= alpha;
+#pragma unroll
+          for (int dt = 0; dt < kDT; ++dt) acc[n][dt] *= alpha;
+        }
+        exps();
+      }
+      lsum[n] += psum;
+      p[n][0] = split_acc<0>(e);
+      p[n][1] = split_acc<1>(e);
+    }
+    const bool second = kFull || kt0 + 16 < kw_end;  // wave-uniform: the last 16 keys are live
+#pragma unroll
+    for (int dt = 0; dt < kDT; ++dt) {
+      const Pair v0 = ld_col<D>(cur.v, coff[dt], 0);
+#pragma unroll
+      for (int n = 0; n < NQ; ++n) acc[n][dt] = mma3(v0, p[n][0], acc[n][dt]);
+      if (second) {
+        const Pair v1 = ld_col<D>(cur.v, coff[dt], 1);
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) acc[n][dt] = mma3(v1, p[n][1], acc[n][dt]);
+      }
+    }
+    st.put_maxima(sm.mx, t & 1, w, lane);
+  };
+  auto advance = [&] {
+    __syncthreads();  // tile t + 1 is staged; every wave is done with tile t
+    ek[0] = ek[1], ev[0] = ev[1];
+  };
+  // Tiles wholly below S (and, causal, at or before the wave's first query) need no mask.
+  const int full_end = (kCausal ? min(S, qw0 + 1) : S) / kRows;
+  const int nfull = wave_live ? min(full_end, ntiles) : 0;
+  __syncthreads();  // tile 0, and tile 1's maxima
+  int t = 0;
+  for (; t < nfull; ++t) {
+    if (!kCausal) prio_by_remaining(ntiles - t, ntiles);
+    tile(Const<1>{}, t, sm.t.kv[t & 1], sm.t.kv[(t + 1) & 1]);
+    advance();
+  }
+  for (; t < ntiles; ++t) {
+    if (!kCausal) prio_by_remaining(ntiles - t, ntiles);
+    if (wave_live && t * kRows < kw_end) {
+      tile(Const<0>{}, t, sm.t.kv[t & 1], sm.t.kv[(t + 1) & 1]);
+    } else {
+      stage(t, sm.t.kv[(t + 1) & 1]);
+      st.put_maxima(sm.mx, t & 1, w, lane);
+    }
+    advance();
+  }
+
+  // L = m / (log2 e as rounded into c2) + ln(l), to one rounding (in fp64, the logarithm of l's
+  // significand aside): the backward takes exp(S scale - L), where an error of L scales a whole row
+  // of P (logf(l), with log2 of some 8 taken at once, left -3.8e-7 on average and 4.9e-7 rms).
+  const float as = fabsf(a.scale), cu = as * kLog2e;
+  const double mr =
+      as == 0.0f ? 0.6931471805599453 : static_cast<double>(as) / static_cast<double>(cu);
+#pragma unroll
+  for (int n = 0; n < NQ; ++n) {
+    const int qg = qw0 + kRows * n, qi = qg + j;
+    if (qg >= S) break;
+    const float l = pair_sum(lsum[n]);
+    if (__builtin_amdgcn_ballot_w64(qi < S && !(probe_finite<kDT>(acc[n], l * 0.0f) == 0.0f)) !=
+        0) {
+      for (int i = 0; i < kRows && qg + i < S; ++i) fwd_row_fp32<D>(a, b, h, qg + i, lane);
+      continue;
+    }
+    // O through LDS (the wave's own part; every wave is past its last tile), so that each row is
+    // written as whole 128-byte lines.
+    const float inv = pow2(e_o - kTop) / l;
+    float* so = sm.t.o[w];
+#pragma unroll
+    for (int c0 = 0; c0 < D; c0 += kOCols) {
+#pragma unroll
+      for (int dt = c0 / 32; dt < (c0 + kOCols) / 32; ++dt) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const f4 x{acc[n][dt][4 * i], acc[n][dt][4 * i + 1], acc[n][dt][4 * i + 2],
+                     acc[n][dt][4 * i + 3]};
+          st4(so + j * kOPitch + 32 * dt - c0 + 8 * i + 4 * g, x * inv);
+        }
+      }
+      constexpr int kLanes = kOCols / 4;  // lanes per row
+#pragma unroll
+      for (int i = 0; i < kRows; i += 64 / kLanes) {
+        const int row = i + lane / kLanes, c = 4 * (lane % kLanes);
+        const f4 x = ld4(so + row * kOPitch + c);
+        if (qg + row < S) {
+          st4_nt(a.o + ((static_cast<int64_t>(b) * S + qg + row) * a.H + h) * D + c0 + c, x);
+        }
+      }
+    }
+    if (g == 0 && qi < S) {
+      int le = exponent(l);
+      float f = l * pow2(-le);  // [1, 2), then [0.75, 1.5)
+      if (f > 1.5f) f *= 0.5f, ++le;
+      const double L = fma(static_cast<double>(m[n]), mr, fma(le, 0.6931471805599453, logf(f)));
+      __builtin_nontemporal_store(static_cast<float>(L), a.lse + static_cast<int64_t>(bh) * S + qi);
+    }
+  }
+}
+
+// --- Backward ----------------------------------------------------------------------------------
+// One launch of two kinds of workgroup, four waves x 32 rows each, which share no sum, so that no
+// workgroup waits for another and the results depend on nothing but the shape:
+//   key blocks of 128 keys walk 32-query tiles and hold dK, dV (S, dP, dV, dK: four products);
+//   query blocks of 128 queries walk 32-key tiles and hold dQ (S, dP, dQ: three products).
+// S and dP are computed in both: seven products where one kind of workgroup would need five, but
+// then dQ's partial sums (4 s^2 b h bytes) would go through memory and dS through LDS, between
+// barriers. Measured against that scheme in fp32, backward: see launch_backward.
+//   key block: S = Q K^T, dP = dO V^T (A = staged rows, B = the wave's keys in registers): lane
+//   (j, g), register r holds key j and query 8 (r / 4) + 4 g + r % 4 of the tile;
+//   P = exp(S scale - L), dS = P o (dP - D); dV^T += dO^T P, dK^T += Q^T dS (A = the staged tiles
+//   transposed, B = P, dS from those registers). L comes from the forward, D = rowsum(dO o O) is
+//   formed while dO is staged.
+//   query block: S^T = K Q^T, dP^T = V dO^T, lane (j, g) holding query j; dQ^T += K^T dS^T.
+// S takes the forward's products in the forward's order: exp(S scale - L) is 1 / l of the
+// probabilities that L was summed from, and the rows of P sum to 1.
+// Exponents: P is formed as P 2^k = 2^(S c2 + (k - L log2 e)), the sum in brackets (exact to one
+// rounding) held per row and k about half of log2 s, so that the exponent stays near 0 whether a row
+// is flat (P about 1 / s) or peaked (P about 1): exp((S scale - L)) rounds its argument twice, at
+// -log2 s for a flat row, which was the largest error of the gradients.
+// Scales: P (at most 1) enters its product as P 2^kPTop; dS per lane (its key, or query) as dS times a running
+// power of two, lowered (and the sums with it) when a value would pass f16's limit; the staged
+// operands that are summed over tiles by their largest exponent so far, as V in the forward.
+struct BwdPairArgs {
+  View q, k, v, d_o;
+  const float* o;
+  const float* lse;
+  float* dqkv;
+  // A split-size workspace: per 16-query tile, `done` takes the launch's epoch where dQ was written;
+  // with `defer` (or for the pair `give_up_bh`, where no step 3 follows: NaN) dQ goes unscaled to
+  // `part` ([b h][tile][16][D]) for step 3. Null: dQ is written.
+  float* part;
+  unsigned long long* done;
+  unsigned long long* epoch_slot;
+  unsigned long long epoch;
+  int* ctrl;
+  int B, H, S, nkv, nblk;  // nkv: key blocks in the grid; nblk: blocks of 128 rows per (b, h)
+  float scale;
+  int causal, defer, last, give_up_bh;
+};
+constexpr int kBwdRows = 128;  // rows per workgroup
+constexpr int kPTop = 15;
+constexpr float kDsMax = 61440.0f;  // of a scaled dS
+constexpr int kDsTop = 11;          // where a new scale puts the largest
+
+// The running scale of dS in one lane: raises nothing, lowers `sc` (and the accumulators by the same
+// factor) where a value would exceed kDsMax.
+template <int N>
+__device__ __forceinline__ void fit_scale(const f16v& ds, float& sc, f16v (&acc)[N]) {
+  float m = 0.0f;
+#pragma unroll
+  for (int r = 0; r < 16; r += 2) {
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(ds[r]), "v"(ds[r + 1]));
+  }
+  if (__builtin_amdgcn_ballot_w64(m * sc > kDsMax) != 0) {
+    m = pair_max(fmaxf(m, 0.0f));
+    if (m * sc > kDsMax) {
+      const float to = pow2(kDsTop - exponent(m));
+      const float f = to / sc;  // (a power of two, or 0)
+      sc = to;
+#pragma unroll
+      for (int i = 0; i < N; ++i) acc[i] *= f;
+    }
+  }
+}
+// k - L log2 e, log2 e in two terms.
+constexpr float kLog2eLow = 1.925963033500e-8f;
+__device__ __forceinline__ float shifted_l(float L, float k) {
+  return fmaf(-L, kLog2eLow, fmaf(-L, kLog2e, k));
+}
+__device__ __forceinline__ int half_log2(int s) { return (32 - __builtin_clz(s)) / 2; }
+// A growing exponent of a staged operand: the factor its sums take.
+__device__ __forceinline__ float grown(int from, int to) {
+  return from - to < -126 ? 0.0f : pow2(from - to);
+}
+
+// dK and dV of one key, dQ of one query, in plain fp32 by one wave: lanes take the other side's rows
+// for the products and dims for the sums.
+template <int D>
+__device__ void bwd_key_fp32(const BwdPairArgs& a, int b, int h, int key, int lane) {
+  const float* kr = a.k.p + b * a.k.sb + h * a.k.sh + static_cast<int64_t>(key) * a.k.ss;
+  const float* vr = a.v.p + b * a.v.sb + h * a.v.sh + static_cast<int64_t>(key) * a.v.ss;
+  const float* qp = a.q.p + b * a.q.sb + h * a.q.sh;
+  const float* gp = a.d_o.p + b * a.d_o.sb + h * a.d_o.sh;
+  const float* op = a.o + (static_cast<int64_t>(b) * a.S * a.H + h) * D;
+  const float* lp = a.lse + (static_cast<int64_t>(b) * a.H + h) * a.S;
+  constexpr int kND = (D + 63) / 64;
+  float dk[kND] = {}, dv[kND] = {};
+  for (int q0 = a.causal ? key : 0; q0 < a.S; q0 += 64) {
+    const int qi = q0 + lane;
+    float p = 0.0f, ds = 0.0f;
+    if (qi < a.S) {
+      const float* qr = qp + static_cast<int64_t>(qi) * a.q.ss;
+      const float* gr = gp + static_cast<int64_t>(qi) * a.d_o.ss;
+      const float* orow = op + static_cast<int64_t>(qi) * a.H * D;
+      float s = 0.0f, t = 0.0f, dd = 0.0f;
+      for (int c = 0; c < D; ++c) {
+        s = fmaf(qr[c], kr[c], s);
+        t = fmaf(gr[c], vr[c], t);
+        dd = fmaf(gr[c], orow[c], dd);
+      }
+      p = exp2_hw(fmaf(s, a.scale, -lp[qi]) * kLog2e);
+      ds = p * (t - dd);
+    }
+    const int n = min(64, a.S - q0);
+    for (int i = 0; i < n; ++i) {
+      const float pi = __shfl(p, i), di = __shfl(ds, i);
+      const float* qr = qp + static_cast<int64_t>(q0 + i) * a.q.ss;
+      const float* gr = gp + static_cast<int64_t>(q0 + i) * a.d_o.ss;
+#pragma unroll
+      for (int e = 0; e < kND; ++e) {
+        const int c = 64 * e + lane;
+        if (c < D) {
+          dv[e] = fmaf(pi, gr[c], dv[e]);
+          dk[e] = fmaf(di, qr[c], dk[e]);
+        }
+      }
+    }
+  }
+  float* row = a.dqkv + (static_cast<int64_t>(b) * a.S + key) * 3 * a.H * D +
+               static_cast<int64_t>(h) * D;
+#pragma unroll
+  for (int e = 0; e < kND; ++e) {
+    const int c = 64 * e + lane;
+    if (c < D) {
+      row[static_cast<int64_t>(a.H) * D + c] = dk[e] * a.scale;
+      row[static_cast<int64_t>(2) * a.H * D + c] = dv[e];
+    }
+  }
+}
+template <int D>
+__device__ void bwd_query_fp32(const BwdPairArgs& a, int b, int h, int qi, int lane, float* row,
+                               float factor) {
+  const float* qr = a.q.p + b * a.q.sb + h * a.q.sh + static_cast<int64_t>(qi) * a.q.ss;
+  const float* gr = a.d_o.p + b * a.d_o.sb + h * a.d_o.sh + static_cast<int64_t>(qi) * a.d_o.ss;
+  const float* kp = a.k.p + b * a.k.sb + h * a.k.sh;
+  const float* vp = a.v.p + b * a.v.sb + h * a.v.sh;
+  const float* orow = a.o + ((static_cast<int64_t>(b) * a.S + qi) * a.H + h) * D;
+  const float L = a.lse[(static_cast<int64_t>(b) * a.H + h) * a.S + qi];
+  constexpr int kND = (D + 63) / 64;
+  float dq[kND] = {}, dd = 0.0f;
+  for (int c = 0; c < D; ++c) dd = fmaf(gr[c], orow[c], dd);
+  const int kend = a.causal ? qi + 1 : a.S;
+  for (int k0 = 0; k0 < kend; k0 += 64) {
+    const int key = k0 + lane;
+    float ds = 0.0f;
+    if (key < kend) {
+      const float* kr = kp + static_cast<int64_t>(key) * a.k.ss;
+      const float* vr = vp + static_cast<int64_t>(key) * a.v.ss;
+      float s = 0.0f, t = 0.0f;
+      for (int c = 0; c < D; ++c) {
+        s = fmaf(qr[c], kr[c], s);
+        t = fmaf(gr[c], vr[c], t);
+      }
+      ds = exp2_hw(fmaf(s, a.scale, -L) * kLog2e) * (t - dd);
+    }
+    const int n = min(64, kend - k0);
+    for (int i = 0; i < n; ++i) {
+      const float di = __shfl(ds, i);
+      const float* kr = kp + static_cast<int64_t>(k0 + i) * a.k.ss;
+#pragma unroll
+      for (int e = 0; e < kND; ++e) {
+        const int c = 64 * e + lane;
+        if (c < D) dq[e] = fmaf(di, kr[c], dq[e]);
+      }
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < kND; ++e) {
+    const int c = 64 * e + lane;
+    if (c < D) row[c] = dq[e] * factor;
+  }
+}
+
+// 32 rows x D of an accumulator (times `f`, per lane), through the wave's part of LDS, to rows of
+// `stride` floats.
+template <int D, int N>
+__device__ __forceinline__ void store_rows(const f16v (&acc)[N], float f, float* so, float* base,
+                                           int64_t stride, int rows, int lane) {
+  constexpr int kCols = D < 64 ? D : 64, kPitch = kCols + 4, kLanes = kCols / 4;
+  const int j = lane & 31, g = lane >> 5;
+#pragma unroll
+  for (int c0 = 0; c0 < D; c0 += kCols) {
+#pragma unroll
+    for (int dt = c0 / 32; dt < (c0 + kCols) / 32; ++dt) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f4 x{acc[dt][4 * i], acc[dt][4 * i + 1], acc[dt][4 * i + 2], acc[dt][4 * i + 3]};
+        st4(so + j * kPitch + 32 * dt - c0 + 8 * i + 4 * g, x * f);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kRows; i += 64 / kLanes) {
+      const int row = i + lane / kLanes, c = 4 * (lane % kLanes);
+      const f4 x = ld4(so + row * kPitch + c);
+      if (row < rows) st4_nt(base + row * stride + c0 + c, x);
+    }
+  }
+}
+// LDS of a backward workgroup.
+template <int D>
+struct BwdSmem {
+  union {
+    struct {
+      Tile<D> a, b;
+    } t[2];
+    float o[4][kRows * ((D < 64 ? D : 64) + 4)];
+  };
+  Maxima mx;
+  float l[2][kRows], d[2][kRows];
+};
+
+template <int D, bool kCausal, bool kSerial>
+__device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, int id) {
+  constexpr int kKS = D / 16, kDT = D / 32;
+  const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, g = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int S = a.S, BH = a.B * a.H;
+  // Causal: the low blocks (they see every later query) first.
+  const int item = kCausal ? id : xcd_remap(id, a.nkv);
+  const int bh = kCausal ? item % BH : item / a.nblk;
+  const int kb = kCausal ? item / BH : item % a.nblk;
+  const int b = bh / a.H, h = bh % a.H;
+  const int k0 = kb * kBwdRows, kw0 = k0 + w * kRows, key = kw0 + j;
+  const bool wave_live = kw0 < S;
+  const Operand qop{reinterpret_cast<const char*>(a.q.p + b * a.q.sb + h * a.q.sh),
+                    static_cast<unsigned>(a.q.ss) * 4u};
+  const Operand gop{reinterpret_cast<const char*>(a.d_o.p + b * a.d_o.sb + h * a.d_o.sh),
+                    static_cast<unsigned>(a.d_o.ss) * 4u};
+  const Operand oop{reinterpret_cast<const char*>(a.o + (static_cast<int64_t>(b) * S * a.H + h) * D),
+                    static_cast<unsigned>(a.H) * D * 4u};
+  const float* lp = a.lse + static_cast<int64_t>(bh) * S;
+  // The walk: step u takes tile t0 + u (causal: from the block's diagonal, four tiles, on).
+  const int ntiles = (S + kRows - 1) / kRows, t0 = kCausal ? k0 / kRows : 0;
+  const int nsteps = ntiles - t0;
+
+  const int kp = half_log2(S);
+  Stage<D> st;
+  RowDots<D> ro;
+  float lreg;
+  auto load = [&](int u) { st.load(qop, gop, (t0 + u) * kRows, S - 1, w, lane); };
+  auto load_o = [&](int u) {
+    const int r0 = (t0 + u) * kRows;
+    ro.load(oop, r0, S - 1, w, lane);
+    lreg = lp[min(r0 + j, S - 1)];
+  };
+  Pair kB[kKS], vB[kKS];
+  float uk, uv;  // 1 / the key's scales
+  int eq[2], eg[2];
+  {
+    OwnRows<D> ok, ov;
+    load(0);
+    load_o(0);
+    ok.load(a.k.p + b * a.k.sb + h * a.k.sh + min(key, S - 1) * a.k.ss, g);
+    ov.load(a.v.p + b * a.v.sb + h * a.v.sh + min(key, S - 1) * a.v.ss, g);
+    st.put_maxima(sm.mx, 1, w, lane);
+    uk = ok.split(1.0f, kB);
+    uv = ov.split(1.0f, vB);
+    __syncthreads();
+    eq[0] = eq[1] = tile_exponent(sm.mx, 1, 0);
+    eg[0] = eg[1] = tile_exponent(sm.mx, 1, 1);
+    st.store(sm.t[0].a, sm.t[0].b, tile_scale(eq[0]), tile_scale(eg[0]), w, lane);
+    ro.put(st, sm.d[0], w, lane);
+    if (w == 0 && g == 0) sm.l[0][j] = shifted_l(lreg, kp);
+    load(1);
+    load_o(1);
+    st.put_maxima(sm.mx, 0, w, lane);
+  }
+  f16v dk[kDT], dv[kDT];
+#pragma unroll
+  for (int dt = 0; dt < kDT; ++dt) dk[dt] = zero16(), dv[dt] = zero16();
+  int e_k = eq[0], e_v = eg[0];
+  float dsc = pow2(kTop + 100);
+  int roff[kKS], coff[kDT];
+#pragma unroll
+  for (int ks = 0; ks < kKS; ++ks) roff[ks] = row_off<D>(j, g, ks);
+#pragma unroll
+  for (int dt = 0; dt < kDT; ++dt) coff[dt] = col_off<D>(lane, dt);
+
+  auto stage = [&](int u) {  // stores the next step's tile
+    const int put = (u + 1) & 1;
+    eq[1] = max(tile_exponent(sm.mx, u & 1, 0), eq[0]);
+    eg[1] = max(tile_exponent(sm.mx, u & 1, 1), eg[0]);
+    st.store(sm.t[put].a, sm.t[put].b, tile_scale(eq[1]), tile_scale(eg[1]), w, lane);
+    ro.put(st, sm.d[put], w, lane);
+    if (w == 0 && g == 0) sm.l[put][j] = shifted_l(lreg, kp);
+  };
+  auto tile = [&](auto fullc, int u) {
+    constexpr bool kFull = decltype(fullc)::value != 0;
+    const int cur = u & 1, q0 = (t0 + u) * kRows;
+    if (eq[0] > e_k) {
+#pragma unroll
+      for (int dt = 0; dt < kDT; ++dt) dk[dt] *= grown(e_k, eq[0]);
+      e_k = eq[0];
+    }
+    if (eg[0] > e_v) {
+#pragma unroll
+      for (int dt = 0; dt < kDT; ++dt) dv[dt] *= grown(e_v, eg[0]);
+      e_v = eg[0];
+    }
+    if (kFull) stage(u);
+    const Tile<D>&Q = sm.t[cur].a, &G = sm.t[cur].b;
+    f16v s = zero16(), dp = zero16();
+    {
+      h8 x[kKS];
+#pragma unroll
+      for (int ks = 0; ks < kKS; ++ks) {
+        const Pair q = ld_row<D>(Q, roff[ks]);
+        x[ks] = q.h;
+        // (The forward's order: its A operand is this B.)
+        s = mma(q.l, kB[ks].h, s);
+        s = mma(q.h, kB[ks].l, s);
+      }
+#pragma unroll
+      for (int ks = 0; ks < kKS; ++ks) s = mma(x[ks], kB[ks].h, s);
+#pragma unroll
+      for (int ks = 0; ks < kKS; ++ks) {
+        const Pair y = ld_row<D>(G, roff[ks]);
+        x[ks] = y.h;
+        dp = mma_small(y, vB[ks], dp);
+      }
+#pragma unroll
+      for (int ks = 0; ks < kKS; ++ks) dp = mma(x[ks], vB[ks].h, dp);
+    }
+    // The loads of the step after next from here on (its O later still): held across the products
+    // above as well, they do not fit.
+    if (kFull) {
+      load(u + 2);
+      pin_loads();
+    }
+    const float cs = a.scale * kLog2e * uk * pow2(eq[0] - kTop), cg = uv * pow2(eg[0] - kTop);
+    // Live: register r's query, q0 + 4 g + 8 i + e, below S and, causal, not before the key.
+    const int hi = key < S ? S - q0 - 4 * g : 0, lo = kCausal ? key - q0 - 4 * g : 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const f4 L = ld4(&sm.l[cur][8 * i + 4 * g]), Dv = ld4(&sm.d[cur][8 * i + 4 * g]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = 4 * i + e;
+        const float x = exp2_hw(fmaf(s[r], cs, L[e]));
+        const bool live = kFull || (8 * i + e < hi && !(kCausal && 8 * i + e < lo));
+        const float p = live ? x : 0.0f;
+        const float y = p * fmaf(dp[r], cg, -Dv[e]);
+        dp[r] = live ? y : 0.0f;
+        s[r] = p;
+      }
+    }
+    if constexpr (kSerial) {
+#pragma unroll
+      for (int dt = 0; dt < kDT; ++dt) {
+        const Pair g0 = ld_col<D>(G, coff[dt], 0), g1 = ld_col<D>(G, coff[dt], 1);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const Pair& y = r < 8 ? g0 : g1;
+          dv[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+              static_cast<float>(y.h[r % 8]) + static_cast<float>(y.l[r % 8]), s[r], dv[dt], 0, 0,
+              0);
+        }
+      }
+    } else {
+      unsigned hh[8], ll[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) split2(s[2 * i], s[2 * i + 1], pow2(kPTop - kp), hh[i], ll[i]);
+      const Pair p0 = make_pair8(hh, ll), p1 = make_pair8(hh + 4, ll + 4);
+#pragma unroll
+      for (int dt = 0; dt < kDT; ++dt) {
+        dv[dt] = mma3(ld_col<D>(G, coff[dt], 0), p0, dv[dt]);
+        dv[dt] = mma3(ld_col<D>(G, coff[dt], 1), p1, dv[dt]);
+      }
+    }
+    if (kFull) {
+      load_o(u + 2);
+      pin_loads();
+    }
+    fit_scale(dp, dsc, dk);
+    {
+      unsigned hh[8], ll[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) split2(dp[2 * i], dp[2 * i + 1], dsc, hh[i], ll[i]);
+      const Pair p0 = make_pair8(hh, ll), p1 = make_pair8(hh + 4, ll + 4);
+#pragma unroll
+      for (int dt = 0; dt < kDT; ++dt) {
+        dk[dt] = mma3(ld_col<D>(Q, coff[dt], 0), p0, dk[dt]);
+        dk[dt] = mma3(ld_col<D>(Q, coff[dt], 1), p1, dk[dt]);
+      }
+    }
+    if (kFull) st.put_maxima(sm.mx, (u + 1) & 1, w, lane);
+  };
+  auto advance = [&] {
+    __syncthreads();
+    eq[0] = eq[1], eg[0] = eg[1];
+  };
+  // Steps with no mask: every query and key below S and, causal, past the diagonal. (In the others
+  // the staging is outside the branch: in both its arms, the loaded registers and the accumulators
+  // spill where they join.)
+  const int full1 = kw0 + kRows <= S ? S / kRows - t0 : 0;
+  auto masked = [&](int u) {
+    stage(u);
+    load(u + 2);
+    load_o(u + 2);
+    pin_loads();
+    if (wave_live && !(kCausal && (t0 + u) * kRows + kRows <= kw0)) tile(Const<0>{}, u);
+    st.put_maxima(sm.mx, (u + 1) & 1, w, lane);
+    advance();
+  };
+  __syncthreads();
+  int u = 0;
+  if (kCausal) {
+    for (; u < min(4, nsteps); ++u) masked(u);
+  }
+  for (; u < full1; ++u) {
+    tile(Const<1>{}, u);
+    advance();
+  }
+  for (; u < nsteps; ++u) masked(u);
+  if (!wave_live) return;
+  const float fk = pow2(e_k - kTop - kp) / dsc * a.scale;
+  const float z = probe_finite<kDT>(dk, probe_finite<kDT>(dv, fk * 0.0f));
+  if (__builtin_amdgcn_ballot_w64(key < S && !(z == 0.0f)) != 0) {
+    for (int i = 0; i < kRows && kw0 + i < S; ++i) bwd_key_fp32<D>(a, b, h, kw0 + i, lane);
+    return;
+  }
+  const int64_t part = static_cast<int64_t>(a.H) * D;
+  float* row = a.dqkv + (static_cast<int64_t>(b) * S + kw0) * 3 * part + static_cast<int64_t>(h) * D;
+  store_rows<D>(dk, fk, sm.o[w], row + part, 3 * part, S - kw0, lane);
+  store_rows<D>(dv, pow2(e_v - kTop - (kSerial ? kp : kPTop)), sm.o[w], row + 2 * part, 3 * part, S - kw0, lane);
+}
+
+template <int D, bool kCausal>
+__device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm, int id) {
+  constexpr int kKS = D / 16, kDT = D / 32;
+  const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, g = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int S = a.S, BH = a.B * a.H;
+  int qb, bh;
+  if (kCausal) {
+    qb = a.nblk - 1 - id / BH;
+    bh = id % BH;
+  } else {
+    const int item = xcd_remap(id, a.nblk * BH);
+    qb = item % a.nblk;
+    bh = item / a.nblk;
+  }
+  const int b = bh / a.H, h = bh % a.H;
+  const int q0 = qb * kBwdRows, qw0 = q0 + w * kRows, qi = qw0 + j;
+  const bool wave_live = qw0 < S;
+  const Operand kop{reinterpret_cast<const char*>(a.k.p + b * a.k.sb + h * a.k.sh),
+                    static_cast<unsigned>(a.k.ss) * 4u};
+  const Operand vop{reinterpret_cast<const char*>(a.v.p + b * a.v.sb + h * a.v.sh),
+                    static_cast<unsigned>(a.v.ss) * 4u};
+  const int k_end = kCausal ? min(S, q0 + kBwdRows) : S;
+  const int ntiles = (k_end + kRows - 1) / kRows;
+  const int kw_end = kCausal ? min(S, qw0 + kRows) : S;
+
+  Stage<D> st;
+  Pair qB[kKS], gB[kKS];
+  const int kp = half_log2(S);
+  float uq, ug, L, Dq;  // L: kp - L log2 e
+  int ek[2], ev[2];  // K's largest exponent so far, V's own
+  {
+    OwnRows<D> oq, og, oo;
+    const int qc = min(qi, S - 1);
+    st.load(kop, vop, 0, S - 1, w, lane);
+    oq.load(a.q.p + b * a.q.sb + h * a.q.sh + qc * a.q.ss, g);
+    og.load(a.d_o.p + b * a.d_o.sb + h * a.d_o.sh + qc * a.d_o.ss, g);
+    oo.load(a.o + ((static_cast<int64_t>(b) * S + qc) * a.H + h) * D, g);
+    L = a.lse[static_cast<int64_t>(bh) * S + qc];
+    st.put_maxima(sm.mx, 1, w, lane);
+    Dq = 0.0f;
+#pragma unroll
+    for (int ks = 0; ks < kKS; ++ks) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        Dq = fmaf(og.x[ks][e / 4][e % 4], oo.x[ks][e / 4][e % 4], Dq);
+      }
+    }
+    Dq = pair_sum(Dq);
+    L = shifted_l(L, kp);
+    uq = oq.split(1.0f, qB);
+    ug = og.split(1.0f, gB);
+    __syncthreads();
+    ek[0] = ek[1] = tile_exponent(sm.mx, 1, 0);
+    ev[0] = ev[1] = tile_exponent(sm.mx, 1, 1);
+    st.store(sm.t[0].a, sm.t[0].b, tile_scale(ek[0]), tile_scale(ev[0]), w, lane);
+    st.load(kop, vop, kRows, S - 1, w, lane);
+    st.put_maxima(sm.mx, 0, w, lane);
+  }
+  f16v dq[kDT];
+#pragma unroll
+  for (int dt = 0; dt < kDT; ++dt) dq[dt] = zero16();
+  int e_q = ek[0];
+  float dsc = pow2(kTop + 100);
+  int roff[kKS], coff[kDT];
+#pragma unroll
+  for (int ks = 0; ks < kKS; ++ks) roff[ks] = row_off<D>(j, g, ks);
+#pragma unroll
+  for (int dt = 0; dt < kDT; ++dt) coff[dt] = col_off<D>(lane, dt);
+
+  auto stage = [&](int t) {
+    const int put = (t + 1) & 1;
+    ek[1] = max(tile_exponent(sm.mx, t & 1, 0), ek[0]);
+    ev[1] = tile_exponent(sm.mx, t & 1, 1);
+    st.store(sm.t[put].a, sm.t[put].b, tile_scale(ek[1]), tile_scale(ev[1]), w, lane);
+  };
+  auto load = [&](int t) {
+    st.load(kop, vop, (t + 2) * kRows, S - 1, w, lane);
+    pin_loads();
+  };
+  auto tile = [&](auto fullc, int t) {
+    constexpr bool kFull = decltype(fullc)::value != 0;
+    const int cur = t & 1, kt0 = t * kRows;
+    if (ek[0] > e_q) {
+#pragma unroll
+      for (int dt = 0; dt < kDT; ++dt) dq[dt] *= grown(e_q, ek[0]);
+      e_q = ek[0];
+    }
+    stage(t);
+    const Tile<D>&K = sm.t[cur].a, &V = sm.t[cur].b;
+    f16v s = zero16(), dp = zero16();
+    {
+      h8 x[kKS];
+#pragma unroll
+      for (int ks = 0; ks < kKS; ++ks) {
+        const Pair k = ld_row<D>(K, roff[ks]);
+        x[ks] = k.h;
+        s = mma_small(k, qB[ks], s);
+      }
+#pragma unroll
+      for (int ks = 0; ks < kKS; ++ks) s = mma(x[ks], qB[ks].h, s);
+#pragma unroll
+      for (int ks = 0; ks < kKS; ++ks) {
+        const Pair v = ld_row<D>(V, roff[ks]);
+        x[ks] = v.h;
+        // (The key blocks' order: their A operand is this B.)
+        dp = mma(v.l, gB[ks].h, dp);
+        dp = mma(v.h, gB[ks].l, dp);
+      }
+#pragma unroll
+      for (int ks = 0; ks < kKS; ++ks) dp = mma(x[ks], gB[ks].h, dp);
+    }
+    load(t);
+    const float cs = a.scale * kLog2e * uq * pow2(ek[0] - kTop), cg = ug * pow2(ev[0] - kTop);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int key = kt0 + 8 * (r >> 2) + 4 * g + (r & 3);
+      const float x = exp2_hw(fmaf(s[r], cs, L)) * fmaf(dp[r], cg, -Dq);
+      dp[r] = kFull || (key < S && !(kCausal && key > qi)) ? x : 0.0f;
+    }
+    fit_scale(dp, dsc, dq);
+    unsigned hh[8], ll[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) split2(dp[2 * i], dp[2 * i + 1], dsc, hh[i], ll[i]);
+    const Pair p0 = make_pair8(hh, ll), p1 = make_pair8(hh + 4, ll + 4);
+#pragma unroll
+    for (int dt = 0; dt < kDT; ++dt) {
+      dq[dt] = mma3(ld_col<D>(K, coff[dt], 0), p0, dq[dt]);
+      dq[dt] = mma3(ld_col<D>(K, coff[dt], 1), p1, dq[dt]);
+    }
+    st.put_maxima(sm.mx, (t + 1) & 1, w, lane);
+  };
+  auto advance = [&] {
+    __syncthreads();
+    ek[0] = ek[1], ev[0] = ev[1];
+  };
+  const int full_end = (kCausal ? min(S, qw0 + 1) : S) / kRows;
+  const int nfull = wave_live ? min(full_end, ntiles) : 0;
+  __syncthreads();
+  int t = 0;
+  for (; t < nfull; ++t) {
+    tile(Const<1>{}, t);
+    advance();
+  }
+  for (; t < ntiles; ++t) {
+    if (wave_live && t * kRows < kw_end) {
+      tile(Const<0>{}, t);
+    } else {
+      stage(t);
+      load(t);
+      st.put_maxima(sm.mx, (t + 1) & 1, w, lane);
+    }
+    advance();
+  }
+  // Where dQ goes (uniform): its rows, or the workspace for step 3.
+  const bool gave_up = bh == a.give_up_bh;
+  const bool direct = a.part == nullptr || !(a.defer || (gave_up && !a.last));
+  const int ntile16 = (S + kBwdQueryTile - 1) / kBwdQueryTile;
+  if (a.done != nullptr && direct && tid < kBwdRows / kBwdQueryTile) {
+    const int j16 = q0 / kBwdQueryTile + tid;
+    if (j16 < ntile16) a.done[static_cast<int64_t>(bh) * ntile16 + j16] = a.epoch;
+  }
+  if (!wave_live) return;
+  const int64_t stride = direct ? static_cast<int64_t>(3) * a.H * D : D;
+  float* row = direct ? a.dqkv + (static_cast<int64_t>(b) * S + qw0) * 3 * a.H * D +
+                            static_cast<int64_t>(h) * D
+                      : a.part + (static_cast<int64_t>(bh) * ntile16 * kBwdQueryTile + qw0) * D;
+  const float factor = direct ? a.scale : 1.0f;
+  const float un = pow2(e_q - kTop - kp) / dsc;
+  const bool bad = __builtin_amdgcn_ballot_w64(
+                       qi < S && !(probe_finite<kDT>(dq, un * 0.0f) == 0.0f)) != 0;
+  if (gave_up && direct) {
+    // (The test hook, as a wait that ran out would: NaN and the guard word.)
+    if (lane == 0) {
+      __hip_atomic_store(a.ctrl + kCtrlGuard, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    store_rows<D>(dq, __builtin_nanf(""), sm.o[w], row, stride, S - qw0, lane);
+  } else if (bad) {
+    for (int i = 0; i < kRows && qw0 + i < S; ++i) {
+      bwd_query_fp32<D>(a, b, h, qw0 + i, lane, row + i * stride, factor);
+    }
+  } else {
+    store_rows<D>(dq, un * factor, sm.o[w], row, stride, S - qw0, lane);
+  }
+}
+
+template <int D, bool kCausal, bool kSerial, int WAVES>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))
+bwd_pair_kernel(BwdPairArgs a) {
+  a.causal = kCausal ? 1 : 0;
+  __shared__ __attribute__((aligned(16))) BwdSmem<D> sm;
+  const int id = static_cast<int>(blockIdx.x);
+  if (id == 0 && threadIdx.x == 0) {
+    __hip_atomic_store(a.ctrl + kCtrlGuard, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (a.epoch_slot != nullptr) *a.epoch_slot = a.epoch;
+  }
+  if (id < a.nkv) {
+    bwd_keys<D, kCausal, kSerial>(a, sm, id);
+  } else {
+    bwd_queries<D, kCausal>(a, sm, id - a.nkv);
+  }
+}
+
+template <int D, int NQ, int WAVES>
+const void* fwd_pair_fn(int causal) {
+  return causal ? reinterpret_cast<const void*>(fwd_pair_kernel<D, true, NQ, WAVES>)
+                : reinterpret_cast<const void*>(fwd_pair_kernel<D, false, NQ, WAVES>);
+}
+
+// Causal, up to this many key blocks: dV summed over the queries one at a time, on the fp32 matrix
+// instruction (kSerial). The first keys of a causal row sum hundreds of terms of one sign, and there
+// a sum of one rounding per query, as the composed fp32 path makes, and one of three per 16 queries
+// drift apart by more than the reference's band around that path (5e-6; tests/parity.rs:218): at
+// b 2 h 6 s 240 the composed path's dV is 6.0e-6 from fp64, so a correctly rounded one misses the
+// band too. The small grids, whose time is a workgroup's latency, keep to the band: backward at that
+// shape 25 us without, 31 with (the fp32 kernels' 35); larger ones take the faster and more accurate
+// sum.
+constexpr int kSerialBlocks = 64;
+template <int D, int WAVES>
+const void* bwd_pair_fn(int causal, bool serial) {
+  return !causal  ? reinterpret_cast<const void*>(bwd_pair_kernel<D, false, false, WAVES>)
+         : serial ? reinterpret_cast<const void*>(bwd_pair_kernel<D, true, true, WAVES>)
+                  : reinterpret_cast<const void*>(bwd_pair_kernel<D, true, false, WAVES>);
+}
+
+}  // namespace
+
+int launch_forward(View q, View k, View v, float* o, float* lse, int b, int h, int s, int d,
+                   float scale, int causal, void* stream) {
+  // 64 queries per wave (256 per workgroup) halve what a query pays for reading, splitting and
+  // waiting for the key tiles, but hold 2 waves per SIMD instead of 3 (D 64) and halve the
+  // workgroups: taken where they make two rounds of the two a CU holds and every workgroup walks
+  // all keys. Measured, 64 against 32 queries per wave: D 64, b 16 h 16 s 1024 (1024 workgroups)
+  // 194 against 223 us, b 64 h 6 s 240 (384) 33.6 against 30.2; causal b 8 h 12 s 2048 180 against
+  // 176; D 32, b 16 h 16 s 1024 127 against 134, b 64 h 6 s 240 19.9 against 18.1. At D 128 their
+  // registers do not fit.
+  const int64_t wide = static_cast<int64_t>((s + 255) / 256) * b * h;
+  const int nq = d != 128 && !causal && wide >= 1024 ? 2 : 1;
+  const int qb = 128 * nq, nqb = (s + qb - 1) / qb;
+  FwdArgs a{q, k, v, o, lse, b, h, s, nqb, scale, causal ? 1 : 0};
+  void* args[] = {&a};
+  const void* fn;
+  if (nq == 2) {
+    fn = d == 32 ? reinterpret_cast<const void*>(fwd_pair_kernel<32, false, 2, 3>)
+                 : reinterpret_cast<const void*>(fwd_pair_kernel<64, false, 2, 2>);
+  } else {
+    fn = d == 32    ? fwd_pair_fn<32, 1, 4>(causal)
+         : d == 128 ? fwd_pair_fn<128, 1, 2>(causal)
+                    : fwd_pair_fn<64, 1, 3>(causal);
+  }
+  return static_cast<int>(hipLaunchKernel(fn, dim3(static_cast<unsigned>(nqb) * b * h),
+                                          dim3(kThreads), args, 0,
+                                          static_cast<hipStream_t>(stream)));
+}
+
+int launch_backward(View q, View k, View v, View d_o, const float* o, const float* lse, float* dqkv,
+                    float* part, unsigned long long* done, unsigned long long* epoch_slot,
+                    unsigned long long epoch, int* ctrl, int b, int h, int s, int d, float scale,
+                    int causal, int defer, int last, int give_up_bh, void* stream) {
+  const int nblk = (s + kBwdRows - 1) / kBwdRows;
+  BwdPairArgs a{q, k, v, d_o, o, lse, dqkv, part, done, epoch_slot, epoch, ctrl, b, h, s,
+                nblk * b * h, nblk, scale, causal ? 1 : 0, defer, last, give_up_bh};
+  void* args[] = {&a};
+  const bool serial = causal && a.nkv <= kSerialBlocks;
+  const void* fn = d == 32    ? bwd_pair_fn<32, 2>(causal, serial)
+                   : d == 128 ? bwd_pair_fn<128, 1>(causal, serial)
+                              : bwd_pair_fn<64, 2>(causal, serial);
+  return static_cast<int>(hipLaunchKernel(fn, dim3(2u * static_cast<unsigned>(a.nkv)),
+                                          dim3(kThreads), args, 0,
+                                          static_cast<hipStream_t>(stream)));
+}
+
+}  // namespace fattn

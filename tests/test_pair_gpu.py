@@ -1,0 +1,120 @@
+"""The f16-pair kernels (csrc/fattn_pair.hip) where they can go wrong: the edges of their 32-row
+tiles and 128 / 256-row workgroups, operands far from 1 and growing along the sequence (the
+power-of-two scales), and values the split cannot carry (infinities, NaN), which go to the plain
+fp32 rows. Everything against fp64 from plain torch on the same inputs."""
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+import candle_fused_attn as cfa
+
+pytestmark = pytest.mark.gpu
+
+# Normwise against fp64, as the parity tests' bar.
+REL_TOL = 2e-6
+
+
+def reference(q, k, v, scale, causal, g=None):
+    """O (and dQ, dK, dV for the output gradient g) in fp64; q, k, v, g [n, s, d]."""
+    q, k, v = (t.double().cpu() for t in (q, k, v))
+    s = q.shape[1]
+    x = torch.matmul(q, k.transpose(1, 2).contiguous()) * scale
+    if causal:
+        x = x.masked_fill(torch.ones(s, s, dtype=torch.bool).triu(1), -math.inf)
+    p = torch.softmax(x, dim=-1)
+    o = torch.matmul(p, v)
+    if g is None:
+        return [o]
+    g = g.double().cpu()
+    ds = p * (torch.matmul(g, v.transpose(1, 2).contiguous()) - (g * o).sum(-1, keepdim=True))
+    return [o, torch.matmul(ds, k) * scale,
+            torch.matmul(ds.transpose(1, 2).contiguous(), q) * scale,
+            torch.matmul(p.transpose(1, 2).contiguous(), g)]
+
+
+def rel(got, want):
+    got = got.detach().double().cpu()
+    return ((got - want).norm() / want.norm()).item()
+
+
+def normal(seed, *shape):
+    gen = torch.Generator(device="cuda:0").manual_seed(seed)
+    return torch.randn(*shape, generator=gen, device="cuda:0")
+
+
+def forward(q, k, v, scale, causal):
+    with torch.no_grad():
+        return cfa.fused_attention(q[None], k[None], v[None], scale, causal)[0]
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("s", [1, 15, 17, 31, 32, 33, 64, 97, 127, 128, 129, 161, 257])
+def test_forward_tile_edges(cuda, s, d, causal):
+    q, k, v = (normal(7 * s + i, 3, s, d) for i in range(3))
+    e = rel(forward(q, k, v, 0.125, causal), reference(q, k, v, 0.125, causal)[0])
+    print(f"forward s{s} d{d} causal={causal}: {e:.2e}", flush=True)
+    assert e <= REL_TOL
+
+
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("s", [33, 255, 256, 257])
+def test_forward_wide_workgroups(cuda, s, d):
+    """Two groups of 32 queries per wave (from 1024 workgroups of 256 queries on)."""
+    n = 1024
+    q, k, v = (normal(11 * s + i, n, s, d) for i in range(3))
+    o = forward(q, k, v, 0.125, False)
+    for i in (0, n // 2 + 1, n - 1):
+        at = slice(i, i + 1)
+        e = rel(o[at], reference(q[at], k[at], v[at], 0.125, False)[0])
+        print(f"wide s{s} d{d} pair {i}: {e:.2e}", flush=True)
+        assert e <= REL_TOL
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("qs,ks,vs,grow", [(1e-9, 1e9, 1e-12, 0), (1e6, 1e-7, 1e15, 0),
+                                           (1.0, 1.0, 1e-3, 3), (1.0, 1.0, 1e3, -3)])
+def test_forward_magnitudes(cuda, qs, ks, vs, grow, causal):
+    """Operands far from 1, and V growing (or shrinking) by 2^grow from one 32-key tile to the
+    next. Normwise over each 32-query block's rows, so that small rows count."""
+    s, d = 200, 64
+    q, k, v = (normal(40 + i, 2, s, d) * f for i, f in enumerate((qs, ks, vs)))
+    v = v * torch.exp2(float(grow) * (torch.arange(s, device="cuda:0") // 32))[None, :, None]
+    o = forward(q, k, v, 0.125, causal)
+    want = reference(q, k, v, 0.125, causal)[0]
+    for r in range(0, s, 32):
+        e = rel(o[:, r:r + 32], want[:, r:r + 32])
+        print(f"magnitudes rows {r}: {e:.2e}", flush=True)
+        assert e <= REL_TOL
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_forward_non_finite(cuda, d):
+    """An infinite key element makes scores +-inf (weight 0, or a NaN row), an infinite or NaN value
+    reaches the rows that see it; every other row is untouched."""
+    s = 150
+    q, k, v = (normal(60 + i, 4, s, d) for i in range(3))
+    k[0, 40, 3] = math.inf
+    k[1, 130, 5] = -math.inf
+    v[2, 100, 1] = math.nan
+    v[3, 70, 2] = math.inf
+    q[3, 9, 4] = math.nan
+    for causal in (False, True):
+        o = forward(q, k, v, 0.125, causal).double().cpu()
+        want = reference(q, k, v, 0.125, causal)[0]
+        if causal:
+            # (0 weight times a non-finite value of a masked key is 0 here, NaN in the product.)
+            for n, first in ((2, 100), (3, 70)):
+                vv = v[n:n + 1].clone()
+                vv[0, first] = 0
+                want[n, :first] = reference(q[n:n + 1], k[n:n + 1], vv, 0.125, True)[0][0, :first]
+        ok = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(o), ok), f"d{d} causal={causal}"
+        assert torch.equal(torch.isnan(o), torch.isnan(want))
+        e = ((o - want)[ok].norm() / want[ok].norm()).item()
+        print(f"non-finite d{d} causal={causal}: {int(ok.sum())} of {ok.numel()} finite, {e:.2e}",
+              flush=True)
+        assert e <= REL_TOL
