@@ -24,7 +24,7 @@ import ctypes
 import torch
 
 from . import _lib
-from ._lib import FusedAttentionError, arr, check
+from ._lib import FusedAttentionError, check
 
 # The reference's head dimension (src/lib.rs:91, CUDA_HEAD_DIM), and those the kernels here are
 # built for.
@@ -33,17 +33,26 @@ HIP_HEAD_DIMS = (32, 64, 128)
 HIP_HEAD_DIM = CUDA_HEAD_DIM
 
 
-def _stream(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+# What a call passes is plain ints and ctypes arrays built in one step: on the small shapes the host
+# is the whole time of a call. Of a forward's 15.8 us (no gradient, b 1 h 2 s 33), 2.0 went to
+# torch.cuda.current_stream, 1 to the arrays and the rest of the difference to wrapping pointers:
+# 12.0 us now.
+_A3, _A4 = ctypes.c_int64 * 3, ctypes.c_int64 * 4
+_raw_stream = torch._C._cuda_getCurrentRawStream
 
 
-def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr())
+def _a4(values) -> ctypes.Array:
+    return _A4(*values[:4])  # (an operand of another rank is refused by its shape or strides)
+
+
+def _stream(t: torch.Tensor) -> int:
+    """torch's current HIP stream of the tensor's device, as a hipStream_t."""
+    return _raw_stream(t.get_device())
 
 
 def _storage(t: torch.Tensor):
     """(storage base pointer, element offset): a candle Layout's start_offset view."""
-    return ctypes.c_void_p(t.untyped_storage().data_ptr()), int(t.storage_offset())
+    return t.untyped_storage().data_ptr(), t.storage_offset()
 
 
 def _require(who: str, name: str, t: torch.Tensor, device: torch.device | None = None) -> None:
@@ -112,15 +121,11 @@ _dq_sum = "auto"
 
 
 def set_dq_sum(mode: str) -> str:
-    """How the backward sums dQ over key blocks; returns the previous setting. Both ways are
-    deterministic (a fixed order per query tile):
-      "split": each key block writes its partials to the workspace (about 4 s^2 b h bytes) and a
-               third kernel sums them -- no workgroup waits on another;
-      "turns": key blocks add into dQ in place under turn counters (minimum workspace);
-      "auto" (default): "split" unless its workspace exceeds the library's FATTN_SPLIT_MAX_BYTES;
-               then, at head_dim <= 64, "split" by chunks of (b, h) pairs (each chunk's state in
-               a workspace within that size; the same results) where the chunks fill the chip,
-               else "turns".
+    """The backward's workspace; returns the previous setting. dQ is summed by its own query
+    blocks, in a fixed order, whatever the workspace, so the results do not depend on it:
+      "auto" (default), "turns": the minimum (control words, per-row and per-tile state);
+      "split": the split size (about 4 s^2 b h bytes), in which the backward also records per query
+               tile that its dQ was written (what the kernel-level step 3 reads).
     """
     global _dq_sum
     if mode not in _DQ_SUM_MODES:
@@ -131,10 +136,9 @@ def set_dq_sum(mode: str) -> str:
 
 def _workspace(b: int, h: int, s: int, d: int, device: torch.device) -> torch.Tensor:
     L = _lib.lib()
-    size = {"auto": L.fattn_bwd_workspace_bytes, "split": L.fattn_bwd_workspace_split_bytes,
-            "turns": L.fattn_bwd_workspace_min_bytes}[_dq_sum]
-    nbytes = int(size(b, h, s, d))
-    return torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
+    size = (L.fattn_bwd_workspace_split_bytes if _dq_sum == "split"
+            else L.fattn_bwd_workspace_min_bytes)
+    return torch.empty(max(size(b, h, s, d), 256), dtype=torch.uint8, device=device)
 
 
 class _FusedAttentionQkv(torch.autograd.Function):
@@ -151,11 +155,13 @@ class _FusedAttentionQkv(torch.autograd.Function):
         out = torch.empty((b, s, three_hd // 3), dtype=torch.float32, device=qkv.device)
         lse = torch.empty((b, max(int(heads), 0), s), dtype=torch.float32, device=qkv.device)
         base, off = _storage(qkv)
-        check(L.fattn_qkv_forward(base, off, arr(qkv.shape), arr(qkv.stride()), int(heads),
-                                  float(scale), int(bool(causal)), _ptr(out), _ptr(lse),
-                                  _stream(qkv)))
+        heads, scale, causal = int(heads), float(scale), bool(causal)
+        rc = L.fattn_qkv_forward(base, off, _A3(b, s, three_hd), _A3(*qkv.stride()), heads, scale,
+                                 causal, out.data_ptr(), lse.data_ptr(), _stream(qkv))
+        if rc:
+            check(rc)
         ctx.save_for_backward(qkv, out, lse)
-        ctx.heads, ctx.scale, ctx.causal = int(heads), float(scale), bool(causal)
+        ctx.heads, ctx.scale, ctx.causal = heads, scale, causal
         return out
 
     @staticmethod
@@ -169,10 +175,12 @@ class _FusedAttentionQkv(torch.autograd.Function):
         ws = _workspace(b, ctx.heads, s, three_hd // 3 // max(ctx.heads, 1), qkv.device)
         base, off = _storage(qkv)
         gbase, goff = _storage(grad)
-        check(_lib.lib().fattn_qkv_backward(
-            base, off, arr(qkv.shape), arr(qkv.stride()), ctx.heads, ctx.scale,
-            int(ctx.causal), _ptr(out), _ptr(lse), gbase, goff, arr(grad.shape),
-            arr(grad.stride()), _ptr(dqkv), _ptr(ws), ws.numel(), _stream(qkv)))
+        rc = _lib.lib().fattn_qkv_backward(
+            base, off, _A3(b, s, three_hd), _A3(*qkv.stride()), ctx.heads, ctx.scale, ctx.causal,
+            out.data_ptr(), lse.data_ptr(), gbase, goff, _A3(*grad.shape), _A3(*grad.stride()),
+            dqkv.data_ptr(), ws.data_ptr(), ws.numel(), _stream(qkv))
+        if rc:
+            check(rc)
         return dqkv, None, None, None
 
 
@@ -191,13 +199,14 @@ class _FusedAttention(torch.autograd.Function):
         out = torch.empty((b, s, h, d), dtype=torch.float32, device=q.device)
         lse = torch.empty((b, h, s), dtype=torch.float32, device=q.device)
         (qb, qo), (kb, ko), (vb, vo) = _storage(q), _storage(k), _storage(v)
-        check(L.fattn_forward(qb, qo, arr(q.shape), arr(q.stride()),
-                              kb, ko, arr(k.shape), arr(k.stride()),
-                              vb, vo, arr(v.shape), arr(v.stride()),
-                              float(scale), int(bool(causal)), _ptr(out), _ptr(lse),
-                              _stream(q)))
+        scale, causal = float(scale), bool(causal)
+        rc = L.fattn_forward(qb, qo, _a4(q.shape), _A4(*q.stride()), kb, ko, _a4(k.shape),
+                             _a4(k.stride()), vb, vo, _a4(v.shape), _a4(v.stride()), scale, causal,
+                             out.data_ptr(), lse.data_ptr(), _stream(q))
+        if rc:
+            check(rc)
         ctx.save_for_backward(q, k, v, out, lse)
-        ctx.scale, ctx.causal = float(scale), bool(causal)
+        ctx.scale, ctx.causal = scale, causal
         return out
 
     @staticmethod
@@ -211,11 +220,14 @@ class _FusedAttention(torch.autograd.Function):
         ws = _workspace(b, h, s, d, q.device)
         (qb, qo), (kb, ko), (vb, vo) = _storage(q), _storage(k), _storage(v)
         gbase, goff = _storage(grad)
-        check(_lib.lib().fattn_backward(
-            qb, qo, arr(q.shape), arr(q.stride()), kb, ko, arr(k.shape), arr(k.stride()),
-            vb, vo, arr(v.shape), arr(v.stride()), ctx.scale, int(ctx.causal), _ptr(out),
-            _ptr(lse), gbase, goff, arr(grad.shape), arr(grad.stride()), _ptr(dqkv), _ptr(ws),
-            ws.numel(), _stream(q)))
+        sh = _a4(q.shape)
+        rc = _lib.lib().fattn_backward(
+            qb, qo, sh, _A4(*q.stride()), kb, ko, sh, _A4(*k.stride()), vb, vo, sh,
+            _A4(*v.stride()), ctx.scale, ctx.causal, out.data_ptr(), lse.data_ptr(), gbase, goff,
+            _A4(*grad.shape), _A4(*grad.stride()), dqkv.data_ptr(), ws.data_ptr(), ws.numel(),
+            _stream(q))
+        if rc:
+            check(rc)
         # dQ, dK, dV: narrow views of the one buffer, each [b, h, s, d] (src/lib.rs:484-485).
         return (dqkv[:, :, 0].transpose(1, 2), dqkv[:, :, 1].transpose(1, 2),
                 dqkv[:, :, 2].transpose(1, 2), None, None)
