@@ -401,6 +401,7 @@ __device__ void fwd_row_fp32(const FwdArgs& a, int b, int h, int qi, int lane) {
     if (key < kend) {
       const float* kr = kp + static_cast<int64_t>(key) * a.k.ss;
       s = 0.0f;
+#pragma clang loop unroll(disable)
       for (int c = 0; c < D; ++c) s = fmaf(sign * qp[c], kr[c], s);
     }
     const float mn = fmaxf(m, wave_max(s));
@@ -411,6 +412,7 @@ __device__ void fwd_row_fp32(const FwdArgs& a, int b, int h, int qi, int lane) {
 #pragma unroll
     for (int i = 0; i < kND; ++i) o[i] *= alpha;
     const int n = min(64, kend - k0);
+#pragma clang loop unroll(disable)
     for (int kk = 0; kk < n; ++kk) {
       const float pk = __shfl(p, kk);
       const float* vr = vp + static_cast<int64_t>(k0 + kk) * a.v.ss;
@@ -788,6 +790,7 @@ __device__ void bwd_key_fp32(const BwdPairArgs& a, int b, int h, int key, int la
       const float* gr = gp + static_cast<int64_t>(qi) * a.d_o.ss;
       const float* orow = op + static_cast<int64_t>(qi) * a.H * D;
       float s = 0.0f, t = 0.0f, dd = 0.0f;
+#pragma clang loop unroll(disable)
       for (int c = 0; c < D; ++c) {
         s = fmaf(qr[c], kr[c], s);
         t = fmaf(gr[c], vr[c], t);
@@ -797,6 +800,7 @@ __device__ void bwd_key_fp32(const BwdPairArgs& a, int b, int h, int key, int la
       ds = p * (t - dd);
     }
     const int n = min(64, a.S - q0);
+#pragma clang loop unroll(disable)
     for (int i = 0; i < n; ++i) {
       const float pi = __shfl(p, i), di = __shfl(ds, i);
       const float* qr = qp + static_cast<int64_t>(q0 + i) * a.q.ss;
@@ -833,6 +837,7 @@ __device__ void bwd_query_fp32(const BwdPairArgs& a, int b, int h, int qi, int l
   const float L = a.lse[(static_cast<int64_t>(b) * a.H + h) * a.S + qi];
   constexpr int kND = (D + 63) / 64;
   float dq[kND] = {}, dd = 0.0f;
+#pragma clang loop unroll(disable)
   for (int c = 0; c < D; ++c) dd = fmaf(gr[c], orow[c], dd);
   const int kend = a.causal ? qi + 1 : a.S;
   for (int k0 = 0; k0 < kend; k0 += 64) {
@@ -842,6 +847,7 @@ __device__ void bwd_query_fp32(const BwdPairArgs& a, int b, int h, int qi, int l
       const float* kr = kp + static_cast<int64_t>(key) * a.k.ss;
       const float* vr = vp + static_cast<int64_t>(key) * a.v.ss;
       float s = 0.0f, t = 0.0f;
+#pragma clang loop unroll(disable)
       for (int c = 0; c < D; ++c) {
         s = fmaf(qr[c], kr[c], s);
         t = fmaf(gr[c], vr[c], t);
@@ -849,6 +855,7 @@ __device__ void bwd_query_fp32(const BwdPairArgs& a, int b, int h, int qi, int l
       ds = exp2_hw(fmaf(s, a.scale, -L) * kLog2e) * (t - dd);
     }
     const int n = min(64, kend - k0);
+#pragma clang loop unroll(disable)
     for (int i = 0; i < n; ++i) {
       const float di = __shfl(ds, i);
       const float* kr = kp + static_cast<int64_t>(k0 + i) * a.k.ss;
@@ -1384,7 +1391,10 @@ int launch_backward(View q, View k, View v, View d_o, const float* o, const floa
                 nblk * b * h, nblk, scale, causal ? 1 : 0, defer, last, give_up_bh};
   void* args[] = {&a};
   const bool serial = causal && a.nkv <= kSerialBlocks;
-  const void* fn = d == 32    ? bwd_pair_fn<32, 2>(causal, serial)
+  // Waves per SIMD: what the registers allow without spills to the loop. At d 32 the third fits once
+  // the fp32 fallback's loops are not unrolled (they set the register count); with it b64 h6 s240
+  // takes 63 us (67 with two), causal b8 h12 s2048 352 (375).
+  const void* fn = d == 32    ? bwd_pair_fn<32, 3>(causal, serial)
                    : d == 128 ? bwd_pair_fn<128, 1>(causal, serial)
                               : bwd_pair_fn<64, 2>(causal, serial);
   return static_cast<int>(hipLaunchKernel(fn, dim3(2u * static_cast<unsigned>(a.nkv)),

@@ -118,3 +118,75 @@ def test_forward_non_finite(cuda, d):
         print(f"non-finite d{d} causal={causal}: {int(ok.sum())} of {ok.numel()} finite, {e:.2e}",
               flush=True)
         assert e <= REL_TOL
+
+
+def gradients(q, k, v, g, scale, causal):
+    """dQ, dK, dV [n, s, d] through the op."""
+    q, k, v = (t[None].detach().requires_grad_() for t in (q, k, v))
+    return [t[0] for t in torch.autograd.grad(cfa.fused_attention(q, k, v, scale, causal),
+                                              (q, k, v), g[None])]
+
+
+def check_gradients(got, want, what, tol=REL_TOL):
+    for name, a, w in zip(("dq", "dk", "dv"), got, want):
+        # (One key: P is 1 and dQ, dK are zero but for dP and D rounding apart.)
+        e = rel(a, w) if w.shape[1] > 1 or name == "dv" else a.abs().max().item()
+        print(f"{what} {name}: {e:.2e}", flush=True)
+        assert e <= tol, (what, name)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("s", [1, 15, 17, 31, 32, 33, 64, 97, 127, 128, 129, 161, 257])
+def test_backward_tile_edges(cuda, s, d, causal):
+    q, k, v, g = (normal(13 * s + i, 3, s, d) for i in range(4))
+    check_gradients(gradients(q, k, v, g, 0.125, causal),
+                    reference(q, k, v, 0.125, causal, g)[1:], f"s{s} d{d} causal={causal}")
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("n", [32, 33])
+def test_backward_serial_boundary(cuda, n, d):
+    """Causal dV on either side of 64 key blocks, up to which it is summed in key order on the fp32
+    matrix cores."""
+    s = 256
+    q, k, v, g = (normal(17 * n + i, n, s, d) for i in range(4))
+    check_gradients(gradients(q, k, v, g, 0.125, True),
+                    reference(q, k, v, 0.125, True, g)[1:], f"{n} pairs d{d}")
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("qs,ks,vs,gs,grow", [(1e-9, 1e9, 1e-12, 1e6, 0), (1e6, 1e-7, 1e9, 1e-9, 0),
+                                              (1.0, 1.0, 1.0, 1.0, 3), (1.0, 1.0, 1.0, 1.0, -3)])
+def test_backward_magnitudes(cuda, qs, ks, vs, gs, grow, causal):
+    """Operands far from 1, and the output gradient growing (or shrinking) by 2^grow from one
+    32-query tile to the next: dQ over each tile's rows, dK and dV normwise."""
+    s, d = 200, 64
+    q, k, v, g = (normal(80 + i, 2, s, d) * f for i, f in enumerate((qs, ks, vs, gs)))
+    g = g * torch.exp2(float(grow) * (torch.arange(s, device="cuda:0") // 32))[None, :, None]
+    got, want = gradients(q, k, v, g, 0.125, causal), reference(q, k, v, 0.125, causal, g)[1:]
+    check_gradients(got, want, f"causal={causal}")
+    for r in range(0, s, 32):
+        check_gradients([got[0][:, r:r + 32]], [want[0][:, r:r + 32]], f"rows {r}")
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_backward_non_finite(cuda, d):
+    """A NaN or infinite operand: non-finite gradients where the product has them, the values
+    elsewhere, and the pairs that hold none untouched to the bit."""
+    s = 150
+    q, k, v, g = (normal(100 + i, 5, s, d) for i in range(4))
+    clean = gradients(q, k, v, g, 0.125, False)
+    k[0, 40, 3] = math.nan
+    v[1, 100, 1] = math.inf
+    q[2, 9, 4] = math.nan
+    g[3, 149, 2] = -math.inf
+    got, want = gradients(q, k, v, g, 0.125, False), reference(q, k, v, 0.125, False, g)[1:]
+    for name, a, c, w in zip(("dq", "dk", "dv"), got, clean, want):
+        a = a.double().cpu()
+        assert torch.equal(a[4], c[4].double().cpu()), name
+        ok = torch.isfinite(w)
+        assert torch.equal(torch.isfinite(a), ok), name
+        e = ((a - w)[ok].norm() / w[ok].norm()).item()
+        print(f"non-finite d{d} {name}: {int(ok.sum())} of {ok.numel()} finite, {e:.2e}", flush=True)
+        assert e <= REL_TOL, name
