@@ -309,18 +309,20 @@ struct Stage {
   }
 };
 // Beside a Stage whose operand b is dO: O's rows in the same lanes, and D = rowsum(dO o O) of the
-// tile's 32 rows.
+// tile's 32 rows. O's offsets are in elements: its rows of one (b, h) may span more than 4 GiB (the
+// views' may not).
 template <int D>
 struct RowDots {
   static constexpr int kC = D / 8, kN = D == 128 ? 2 : 1;
   f4 x[kN][2];
-  __device__ __forceinline__ void load(const Operand& o, int r0, int last, int w, int lane) {
+  __device__ __forceinline__ void load(const float* o, unsigned ss, int r0, int last, int w,
+                                       int lane) {
 #pragma unroll
     for (int i = 0; i < kN; ++i) {
       const unsigned r = static_cast<unsigned>(min(r0 + Stage<D>::row(i, w, lane), last));
-      const unsigned off = r * o.ss4 + 32u * static_cast<unsigned>(lane % kC);
-      x[i][0] = *reinterpret_cast<const f4*>(o.p + off);
-      x[i][1] = *reinterpret_cast<const f4*>(o.p + off + 16);
+      const unsigned off = r * ss + 8u * static_cast<unsigned>(lane % kC);
+      x[i][0] = ld4(o + off);
+      x[i][1] = ld4(o + off + 4);
     }
   }
   __device__ __forceinline__ void put(const Stage<D>& st, float* dst, int w, int lane) const {
@@ -928,8 +930,7 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
                     static_cast<unsigned>(a.q.ss) * 4u};
   const Operand gop{reinterpret_cast<const char*>(a.d_o.p + b * a.d_o.sb + h * a.d_o.sh),
                     static_cast<unsigned>(a.d_o.ss) * 4u};
-  const Operand oop{reinterpret_cast<const char*>(a.o + (static_cast<int64_t>(b) * S * a.H + h) * D),
-                    static_cast<unsigned>(a.H) * D * 4u};
+  const float* op = a.o + (static_cast<int64_t>(b) * S * a.H + h) * D;
   const float* lp = a.lse + static_cast<int64_t>(bh) * S;
   // The walk: step u takes tile t0 + u (causal: from the block's diagonal, four tiles, on).
   const int ntiles = (S + kRows - 1) / kRows, t0 = kCausal ? k0 / kRows : 0;
@@ -942,7 +943,7 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
   auto load = [&](int u) { st.load(qop, gop, (t0 + u) * kRows, S - 1, w, lane); };
   auto load_o = [&](int u) {
     const int r0 = (t0 + u) * kRows;
-    ro.load(oop, r0, S - 1, w, lane);
+    ro.load(op, static_cast<unsigned>(a.H) * D, r0, S - 1, w, lane);
     lreg = lp[min(r0 + j, S - 1)];
   };
   Pair kB[kKS], vB[kKS];

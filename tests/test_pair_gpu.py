@@ -190,3 +190,15 @@ def test_backward_non_finite(cuda, d):
         e = ((a - w)[ok].norm() / w[ok].norm()).item()
         print(f"non-finite d{d} {name}: {int(ok.sum())} of {ok.numel()} finite, {e:.2e}", flush=True)
         assert e <= REL_TOL, name
+
+
+def test_backward_output_over_4gib(cuda):
+    """One (b, h)'s rows of O spanning more than 4 GiB (the operands' rows do not)."""
+    h, s, d = 8192, 1040, 128
+    gen = torch.Generator(device="cuda:0").manual_seed(3)
+    q, k, v, g = (torch.randn(h, s, d, generator=gen, device="cuda:0") for _ in range(4))
+    got = gradients(q, k, v, g, 0.1, False)
+    for i in (0, h - 1):
+        at = slice(i, i + 1)
+        check_gradients([t[at] for t in got], reference(q[at], k[at], v[at], 0.1, False, g[at])[1:],
+                        f"head {i}")
