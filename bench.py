@@ -60,9 +60,12 @@ SCALE = 0.125
 TRAFFIC = REPO / "profiles" / "traffic.json"
 LIB = REPO / "candle-fused-attn_amd" / "lib" / "libfattn.so"
 COPY_KIB = 256 * 1024            # the --calibrate-copy kernel moves 256 MiB each way
-KERNEL_NAMES = {"fwd": "fwd_kernel<64, 128, 32, 3, false>",
-                "bwd_main": "bwd_split_kernel<64, 1, false>", "bwd_dq": "dq_kernel<64>"}
-CAUSAL_FWD_NAME = "fwd_kernel<64, 64, 32, 3, true>"   # config 3's forward
+KERNEL_NAMES = {"fwd": "fwd_pair_kernel<64, false, 1, 3>",
+                "bwd_main": "bwd_pair_kernel<64, false, false, 2>", "bwd_dq": "dq_kernel<64>"}
+CAUSAL_FWD_NAME = "fwd_pair_kernel<64, true, 1, 3>"   # config 3's forward
+# (The second names: traces of libraries with the fp32-instruction kernels.)
+FWD_PREFIXES = ("fwd_pair_kernel", "fwd_kernel")
+MAIN_PREFIXES = ("bwd_pair_kernel", "bwd_split_kernel", "bwd_kernel")
 
 # The BASELINE.json configurations this bench times: (name, kind, b, h, s, causal, seed, std).
 CONFIGS = {
@@ -189,8 +192,7 @@ class Workload:
             _lib.check(kl["bwd_dq"](P(dqkv), P(ws), ws_bytes, b, h, s, d, SCALE, ci, sp))
 
         self.fwd, self.bwd = fwd, bwd
-        # With a split workspace at d 64 step 1 launches nothing (step 2 computes D itself, and
-        # its last workgroups sum dQ tiles); step 3 sums the tiles those left.
+        # Step 1 launches nothing; with a split workspace step 3 reads the tiles' flags.
         self.kernels = [("fwd", fwd_k), ("bwd_prep", prep_k), ("bwd_main", main_k)]
         if self.split:
             self.kernels.append(("bwd_dq", dq_k))
@@ -271,9 +273,8 @@ def traffic_path(cfg: int) -> Path:
 
 
 # Kernel roles by name prefix (the traffic summary's keys).
-KERNEL_ROLES = (("fwd", "fwd_kernel"), ("bwd_prep", "prep_kernel"),
-                ("bwd_main", "bwd_split_kernel"), ("bwd_main", "bwd_kernel"),
-                ("bwd_dq", "dq_kernel"))
+KERNEL_ROLES = (("fwd", FWD_PREFIXES), ("bwd_prep", "prep_kernel"),
+                ("bwd_main", MAIN_PREFIXES), ("bwd_dq", "dq_kernel"))
 
 
 def summarize_traffic(fetch_csv: str, write_csv: str, cfg: int = 2) -> int:
@@ -339,10 +340,10 @@ def _headline_windows(rows: list, warmup: int, steps: int, cfg: int) -> dict | N
     steps_seq: list[list] = []
 
     def step2(name):
-        return name.startswith(("bwd_split_kernel", "bwd_kernel"))
+        return name.startswith(MAIN_PREFIXES)
 
     for _, name, wgs, payload in rows:
-        if (name.startswith("fwd_kernel") or not steps_seq
+        if (name.startswith(FWD_PREFIXES) or not steps_seq
                 or (step2(name) and any(step2(n) for n, _, _ in steps_seq[-1]))):
             steps_seq.append([])
         steps_seq[-1].append((name, wgs, payload))
@@ -424,7 +425,7 @@ def summarize_trace(trace_csv: str, warmup: int, steps: int, cfg: int = 2) -> in
 
 
 # Counters per dispatch that the summary derives figures from (any subset may be present).
-MFMA_CYCLES = 32            # v_mfma_f32_16x16x4_f32: 8 passes of 4 cycles on one SIMD
+MFMA_CYCLES = 32            # v_mfma_f32_32x32x16_f16: 8 passes of 4 cycles on one SIMD
 N_SIMDS, N_CUS, N_XCDS = 1024, 256, 8
 
 
@@ -715,15 +716,12 @@ def main() -> int:
         f"dq sum {dq_us:.1f} us ({'split' if w.split else 'turns'}); step {kus['step']:.1f} us")
 
     # The op-level backward alone, K calls back to back with events only at the window's ends.
-    # With a split workspace at d <= 64 a call is one launch of step 2 (step 1 launches nothing,
-    # and step 2 sums every dQ tile), so the window's mean is step 2's average launch duration
-    # plus one dispatch gap; the forward window (`fwd_ms`) is the forward kernel's likewise.
+    # A call is one launch of step 2, so the window's mean is step 2's average launch duration plus
+    # one dispatch gap; the forward window (`fwd_ms`) is the forward kernel's likewise.
     torch.cuda.nvtx.range_push("fattn timed bwd")
     bwd_ms, _, _ = event_steps(torch, w.stream, w.bwd, K)
     torch.cuda.nvtx.range_pop()
-    one_launch = w.split and D <= 64
-    log(f"bench: op-level bwd {bwd_ms:.4f} ms"
-        + (" (one step-2 launch per call)" if one_launch else ""))
+    log(f"bench: op-level bwd {bwd_ms:.4f} ms (one step-2 launch per call)")
 
     if not args.no_extra:
         # The other head dims the kernels are built for, at the headline's shape: after the
@@ -756,7 +754,7 @@ def main() -> int:
     bwd_tflops = f_bwd / (bwd_ms * 1e-3) / 1e12
     # Step 2's rate: from the op-level backward window where a call is that one launch, else from
     # the kernel-level events around it.
-    step2_tflops = bwd_tflops if one_launch else main_tflops
+    step2_tflops = bwd_tflops
     traffic = traffic_entry()
 
     result = {
@@ -802,9 +800,7 @@ def main() -> int:
                        "step": round(kus["step"], 2)},
         "dq_sum": "split" if w.split else "turns",
         "roofline": {
-            "kernel": ("bwd_split_kernel<64, 1, false> (fattn_bwd_main_f32_d64, split; its last "
-                       "workgroups sum dQ tiles)" if w.split
-                       else "bwd_kernel<false, 64> (fattn_bwd_main_f32_d64, turns)"),
+            "kernel": "bwd_pair_kernel<64, false, false, 2> (fattn_bwd_main_f32_d64)",
             "bound": "mfma",
             "achieved": round(step2_tflops, 3),
             "peak": PEAK_FP32_MFMA_TFLOPS,
@@ -813,8 +809,7 @@ def main() -> int:
             **traffic,
             "flops_per_launch": f_bwd,
             "achieved_from": (f"bwd_ms: {K} op-level backwards back to back, one step-2 launch "
-                              "each, HIP events at the window's ends" if one_launch
-                              else "kernels_us.bwd_main: kernel-level events"),
+                              "each, HIP events at the window's ends"),
             "kernel_level_achieved": round(main_tflops, 3),
             "kernel_level_frac": round(main_tflops / PEAK_FP32_MFMA_TFLOPS, 4),
             "bwd_steps_1_3_achieved": round(bwd_steps_tflops, 3),

@@ -1,5 +1,5 @@
 // The C ABI (include/fattn.h): argument validation with the reference's conditions and
-// messages, operand views, workspace layout, and the launches (fattn_kernels.hip).
+// messages, operand views, workspace layout, and the launches.
 //
 // Validation runs before any HIP call, so a rejected call touches no device and needs none.
 #include <hip/hip_runtime.h>
@@ -28,7 +28,7 @@ Workspace workspace_layout(int64_t b, int64_t h, int64_t s, int64_t d) {
   const size_t rows = static_cast<size_t>(b * h * s);
   const size_t tiles = static_cast<size_t>(b * h * ((s + kBwdQueryTile - 1) / kBwdQueryTile));
   const size_t nkb = static_cast<size_t>((s + kBwdKeys - 1) / kBwdKeys);
-  // The control words (ticket, guard word) first: their place is the same for every shape, so
+  // The control words (the guard word) first: their place is the same for every shape, so
   // fattn_bwd_status finds the guard word whichever way the workspace was used.
   w.ctrl_off = 0;
   w.d_off = up(64 * sizeof(int));
@@ -43,8 +43,9 @@ Workspace workspace_layout(int64_t b, int64_t h, int64_t s, int64_t d) {
   return w;
 }
 
-// The split step 2's workgroup slots on gfx950 (256 CUs): 3 per CU, 2 with 128-key blocks at
-// d 64.
+// The rules below size the chunks that a workspace below the split size is taken as: part of the
+// ABI's size queries (callers' plans and saved sizes hold their answers), no longer of a launch.
+// The workgroup slots they count: 3 per CU (256 CUs), 2 with 128-key blocks at d 64.
 int64_t split_slots(int keys, int64_t d) {
   return (keys > kBwdKeys && d > 32 ? 2 : 3) * int64_t{256};
 }
@@ -57,8 +58,7 @@ int64_t split_slots(int keys, int64_t d) {
 //   non-causal: the most pairs whose key blocks fill whole rounds of the chip's workgroup slots
 //     (every key block walks all query tiles, so a partial round idles slots; the last chunk
 //     takes the rest);
-// 0 when that is fewer than min_pairs. Steps 2 and 3 then run per chunk, each chunk's state at
-// the start of the workspace (workspace_layout(1, chunk, s, d)).
+// 0 when that is fewer than min_pairs. A chunk's size is workspace_layout(1, chunk, s, d).
 int64_t split_chunk(int64_t b, int64_t h, int64_t s, int64_t d, size_t ws_bytes,
                     int64_t min_pairs, bool causal) {
   const int64_t total = b * h;
@@ -86,13 +86,8 @@ int64_t split_chunk(int64_t b, int64_t h, int64_t s, int64_t d, size_t ws_bytes,
   return (total + chunks - 1) / chunks;
 }
 
-// The fewest (b, h) pairs a chunk should hold. A chunk is one launch of step 2: with too few key
-// blocks it runs at a fraction of the chip, so chunks of fewer pairs than this lose to the turn
-// hand-over over all pairs (measured: b 4 h 16 s 8192 causal, chunks of 8 pairs 15.1 ms against
-// 13.8 with turns). Non-causal: the chunk's key blocks fill the chip's workgroup slots at least
-// once. Causal: the key blocks' walks shrink with the block index, so the slots' average work must
-// be at least twice the longest walk (block 0's, all query tiles): four times the slots in key
-// blocks.
+// The fewest (b, h) pairs a chunk should hold: non-causal, key blocks for all slots; causal (the key
+// blocks' walks shrink with the block index) for four times as many.
 int64_t min_chunk_pairs(int64_t b, int64_t h, int64_t s, int64_t d, bool causal) {
   const int keys = bwd_split_keys(b, h, s, static_cast<int>(d), causal ? 1 : 0);
   const int64_t nkb = (s + keys - 1) / keys;
@@ -121,8 +116,8 @@ using fattn::View;
 
 thread_local std::string g_error;
 
-// A 64-bit value unique to each step 2 launch of this process (low 3 bits zero, for the XCD), the
-// sequence starting at a random point: step 2's dQ sums tag their workspace state with it.
+// A 64-bit value unique to each step 2 launch of this process, the sequence starting at a random
+// point: step 2 tags its flags in the workspace with it.
 unsigned long long next_epoch() {
   static std::atomic<unsigned long long> counter{[] {
     std::random_device rd;
@@ -252,12 +247,9 @@ int run_forward(const char* who, View q, View k, View v, float* o, float* lse, i
 }
 
 struct WsParts {
-  float* dsum;
-  float* part;  // null: the workspace is too small for the split partials (turn hand-over)
-  unsigned long long* arrive;  // split: step 2's dQ sums
+  float* part;  // null: the workspace is below the split size
   unsigned long long* done;
   unsigned long long* epoch;
-  int* turn;
   int* ctrl;
 };
 
@@ -270,13 +262,9 @@ int workspace_parts(const char* who, void* ws, size_t ws_bytes, int64_t b, int64
                                       " bytes");
   }
   char* base = static_cast<char*>(ws);
-  out->dsum = reinterpret_cast<float*>(base + l.d_off);
   out->part = ws_bytes >= l.bytes_split ? reinterpret_cast<float*>(base + l.part_off) : nullptr;
-  out->arrive =
-      out->part ? reinterpret_cast<unsigned long long*>(base + l.arrive_off) : nullptr;
   out->done = out->part ? reinterpret_cast<unsigned long long*>(base + l.done_off) : nullptr;
   out->epoch = out->part ? reinterpret_cast<unsigned long long*>(base + l.epoch_off) : nullptr;
-  out->turn = reinterpret_cast<int*>(base + l.turn_off);
   out->ctrl = reinterpret_cast<int*>(base + l.ctrl_off);
   return 0;
 }
@@ -721,8 +709,8 @@ int fattn_backward(const float* q, int64_t q_offset, const int64_t q_shape[4],
 }
 
 // Test hook (not declared in include/fattn.h; tests/test_boundary.py calls it without a GPU): an
-// audit of step 2's dQ-sum schedule for one shape, on the host, with the scheduling functions the
-// kernel runs (fattn_internal.h). A summing unit is a workgroup appended to step 2's grid
+// audit of the dQ-sum plan for one shape, on the host, with the plan's functions
+// (fattn_internal.h). A summing unit is a workgroup appended to step 2's grid
 // (non-causal) or a key block's own workgroup summing its diagonal tiles (causal). out[0]:
 // workgroups appended to step 2's grid; out[1]: summing units with tiles to sum; out[2]:
 // violations -- a causal unit waits for a key block later in the grid or sums a tile it is not
@@ -817,27 +805,25 @@ int fattn_internal_sum_audit(int64_t b, int64_t h, int64_t s, int64_t d, int cau
 // process that opted in before the library loaded (FATTN_TEST_HOOKS=1 in its environment, read
 // once, at load); otherwise they change nothing and return FATTN_EINVAL.
 
-// Test hook (not declared in include/fattn.h): step 2's dQ sums on (1, the default) or off (0:
-// step 3 sums every tile) for every later backward of the process. Returns the previous setting.
+// Test hook (not declared in include/fattn.h): step 2 writes dQ (1, the default) or leaves every
+// tile of a split-size workspace to step 3 (0) for every later backward of the process. Returns the
+// previous setting.
 int fattn_internal_step2_sums(int on) {
   if (!g_test_hooks) return hooks_refused("fattn_internal_step2_sums");
   return fattn::set_step2_sums(on != 0) ? 1 : 0;
 }
 
-// Test hook (not declared in include/fattn.h): step 2's non-causal summing workgroups of XCD x
-// sum the (b, h)s whose key blocks ran on XCD x + shift (mod 8) in every later backward of the
-// process (0, the default: their own XCD's), so that a test can make every sum read partials
-// written on another XCD. Returns the previous shift.
+// Test hook (not declared in include/fattn.h): a shift of the plan's XCDs (0, the default). Kept and
+// returned; the kernels sum nothing across workgroups and do not read it. Returns the previous shift.
 int fattn_internal_sum_shift(int shift) {
   if (!g_test_hooks) return hooks_refused("fattn_internal_sum_shift");
   return fattn::set_sum_shift(shift);
 }
 
-// Test hook (not declared in include/fattn.h): the dQ sums of (b, h) pair `bh` (index b * h_count
-// + h; -1, the default: none) give up before their first poll in every later backward of the
-// process, as a wait that timed out would: where no step 3 follows they raise the guard word (3)
-// and write NaN into that pair's dQ rows; where step 3 follows it sums them. Returns the previous
-// pair.
+// Test hook (not declared in include/fattn.h): step 2 gives up the dQ of (b, h) pair `bh` (index
+// b * h_count + h; -1, the default: none) in every later backward of the process: where no step 3
+// follows it raises the guard word (3) and writes NaN into that pair's dQ rows; where step 3 follows
+// it leaves them to it. Returns the previous pair.
 int fattn_internal_sum_give_up(int bh) {
   if (!g_test_hooks) return hooks_refused("fattn_internal_sum_give_up");
   return fattn::set_give_up_bh(bh);

@@ -1,6 +1,5 @@
 // Internal interface between the C-ABI layer (fattn_api.cpp) and the gfx950 kernels
-// (fattn_kernels.hip), both compiled by hipcc. The scheduling functions below are __host__
-// __device__: the kernels and the host's grid sizes use the same code.
+// (fattn_pair.hip, fattn_kernels.hip), all compiled by hipcc.
 #ifndef FATTN_INTERNAL_H
 #define FATTN_INTERNAL_H
 
@@ -14,9 +13,8 @@ namespace fattn {
 constexpr int kHeadDim = 64;
 bool head_dim_supported(int64_t d);
 
-// Backward tiling: a workgroup owns kBwdKeys keys of one (batch, head) and walks query tiles of
-// kBwdQueryTile; per query tile one dQ partial slot per key block (split) or one dQ turn counter
-// (turns).
+// The units of the workspace's sizes (what callers plan with and saved plans hold), not of the
+// kernels: key blocks of kBwdKeys, query tiles of kBwdQueryTile.
 constexpr int kBwdKeys = 64;
 #ifndef BWD_QT
 #define BWD_QT 16
@@ -31,33 +29,25 @@ struct View {
 };
 
 // Workspace of the backward, in this order, each part 256-byte aligned:
-//   ctrl   64 i32                           [0] key-block ticket, [32] guard word (first, so
-//                                           that its place does not depend on the shape)
-//   D      [b, h, s] f32                    rowsum(dO o O)
-//   turn   [b, h, ntile] i32                dQ turn counter per query tile (turn hand-over)
-//   part   [nkb, b, h, ntile, kQT * d] f32 dQ partial per key block and query tile (split only)
-//   arrive [b, h, nkb] u64                  per key block: the epoch of the launch that finished
-//                                           it, or'ed with its XCD (split)
-//   done   [b, h, ntile] u64                the epoch of the launch whose step 2 summed the tile
+//   ctrl   64 i32                           [32] guard word (first, so that its place does not
+//                                           depend on the shape)
+//   D      [b, h, s] f32                    (unused)
+//   turn   [b, h, ntile] i32                (unused)
+//   part   [nkb, b, h, ntile, kQT * d] f32  the first [b, h, ntile, kQT * d]: dQ left to step 3
+//   arrive [b, h, nkb] u64                  (unused)
+//   done   [b, h, ntile] u64                the epoch of the launch that wrote the tile's dQ rows
 //   epoch  u64 (256 bytes)                  the epoch of the last step 2 launch on the workspace
-// with ntile = ceil(s / kBwdQueryTile), nkb = ceil(s / kBwdKeys). `bytes_min` covers ctrl, D and
-// turn (the turn hand-over), `bytes_split` all seven.
+// with ntile = ceil(s / kBwdQueryTile), nkb = ceil(s / kBwdKeys). The layout and its sizes are those
+// of the ABI's size queries: `bytes_min` covers ctrl, D and turn, `bytes_split` all seven.
 struct Workspace {
   size_t d_off, turn_off, ctrl_off, part_off, arrive_off, done_off, epoch_off, bytes_min,
       bytes_split;
 };
 Workspace workspace_layout(int64_t b, int64_t h, int64_t s, int64_t d);
-constexpr int kCtrlTicket = 0;
 constexpr int kCtrlGuard = 32;
-// dQ sums inside step 2 (split mode): a query tile is summed in step 2 once every key block it
-// needs has finished, from partials stored and read at device scope (so whatever XCDs the key
-// blocks ran on); step 3, where it runs, sums what step 2 left. Non-causal, workgroups appended to
-// step 2's grid do the sums; causal, each key block's own workgroup sums, after its walk, the
-// tiles whose last contributor it is. Every step 2 launch carries its own epoch (a 64-bit value
-// unique to the launch, low 3 bits zero): the key blocks' arrivals and the done flags hold it, so
-// nothing needs clearing between launches and no stale or uninitialised value passes for a
-// current one (but with a 2^-64 chance). The summing workgroups poll at most kSumMaxBlocks
-// arrival slots.
+// The schedule of dQ sums over key blocks, as the ABI's schedule queries describe it for a shape and
+// a workspace (a plan over the units above). The kernels keep dQ in registers and sum nothing across
+// workgroups; the queries keep their answers.
 constexpr int kSumMaxBlocks = 256;
 constexpr int kSumTiles = 3;  // query tiles per summing workgroup
 // Causal: the query tiles whose last contributor is key block kb of `keys` keys (its diagonal
@@ -83,15 +73,10 @@ __host__ __device__ inline int item_xcd(int item, int total) {
   return item >= full ? (item & 7) : item / (full >> 3);
 }
 
-// The dQ sums in step 2 (split). Non-causal: workgroups appended to step 2's grid; workgroup
-// n_main + 8 m + x runs on XCD x (workgroups go to the XCDs round robin on MI355X). xcd_remap
-// gives XCD x the (b, h)-major key blocks [x F, (x + 1) F), F = floor(nkb b h / 8), and deals the
-// rest (fewer than 8) round robin. Summing workgroup m < mc nchunk of XCD x takes chunk
-// m % nchunk of the (m / nchunk)-th (b, h) whose last key block is among XCD x's, so that the
-// sums dispatched first wait for the key blocks dispatched first; the workgroups after those take,
-// in (b, h) order, the (b, h)s whose last key block is among the rest. Causal: every key block
-// sums the tiles it completes. The partials are read at device scope, so the XCDs order the waits
-// but are not needed for correctness. on = 0: no sums (step 3 sums every tile).
+// The plan: non-causal, summing units after the key blocks of the grid; unit m < mc nchunk of XCD x
+// takes chunk m % nchunk of the (m / nchunk)-th (b, h) whose last key block is among XCD x's, the
+// units after those take, in (b, h) order, the (b, h)s whose last key block is among the rest.
+// Causal: every key block sums the tiles it completes. on = 0: no sums (step 3 takes every tile).
 struct SumPlan {
   int on;
   int nchunk;  // chunks of kSumTiles query tiles per (b, h)
@@ -117,7 +102,7 @@ __host__ __device__ inline SumPlan sum_plan(int BH, int nkb, int ntile, int d, i
   }
   return p;
 }
-// Workgroups appended to step 2's grid for the non-causal sums (a multiple of 8).
+// Units of the non-causal plan (a multiple of 8).
 __host__ __device__ inline int sum_blocks(SumPlan p, int BH, int causal) {
   if (causal || !p.on) return 0;
   const int left = BH - 8 * (p.nkb * BH / 8) / p.nkb;
@@ -143,32 +128,29 @@ __host__ __device__ inline bool sum_target(SumPlan p, int x, int m, int BH, int 
   *j0 = idx % p.nchunk * kSumTiles;
   return *bh < BH;
 }
-// Keys per key block of the split step 2 (d <= 64): kBwdKeys, or twice that (each wave owning two
-// groups of 16 keys) for long non-causal sequences at d 64. The sums' plan, step 3 and the
-// workspace's slots (sized for kBwdKeys) follow it.
+// Keys per key block of the plan: kBwdKeys, or twice that for large non-causal launches.
 int bwd_split_keys(int64_t b, int64_t h, int64_t s, int d, int causal);
-// Whether step 2 sums dQ tiles for this shape (the plan has (b, h)s to sum and the sums are on).
+// Whether the plan has sums for this shape (and the hook has not turned them off).
 bool bwd_step2_sums(int64_t b, int64_t h, int64_t s, int d, int causal);
-// Workgroups appended to step 2's grid for the non-causal sums (0 when causal or without sums).
+// Units of the non-causal plan (0 when causal or without sums).
 int64_t bwd_sum_blocks(int64_t b, int64_t h, int64_t s, int d, int causal);
-// Test hooks (the C ABI lets a process use them only when it opted in at load). Step 2's sums on
-// (the default) or off for every later backward of the process, so that a test can compare both;
-// returns the previous setting.
+// Test hooks (the C ABI lets a process use them only when it opted in at load). Off: step 2 leaves
+// every dQ tile of a split-size workspace to step 3, in every later backward of the process; returns
+// the previous setting (1, the default: on).
 bool set_step2_sums(bool on);
-// The non-causal summing workgroups of XCD x sum the (b, h)s of XCD x + shift (mod 8) in every
-// later launch, so that their partials come from another XCD; returns the previous shift.
+// A setting of the plan's XCDs; kept and returned, the kernels do not read it.
 int set_sum_shift(int shift);
-// Step 2's dQ sums of (b, h) pair `bh` (of the whole backward; -1: none, the default) give up
-// before their first poll in every later launch, as a wait that timed out would; returns the
-// previous pair.
+// Step 2 gives up the dQ of (b, h) pair `bh` (of the whole backward; -1: none, the default) in every
+// later launch: NaN and guard word 3 where no step 3 follows, else left to it; returns the previous
+// pair.
 int set_give_up_bh(int bh);
 // What the hooks ask of a launch: dQ deferred to step 3 (step 2's sums off), the give-up pair.
 bool step2_deferred();
 int give_up_pair();
 // The three hooks' current settings: step 2's sums on, the sum shift, the give-up pair.
 void test_hook_state(int64_t out[3]);
-// Launchers (fattn_pair.hip: the forward; fattn_kernels.hip). They assume validated arguments; they return a hipError_t
-// value as int (0 = launched).
+// Launchers (step 3: fattn_kernels.hip, the others fattn_pair.hip). They assume validated arguments
+// and return a hipError_t value as int (0 = launched).
 int launch_forward(View q, View k, View v, float* o, float* lse, int b, int h, int s, int d,
                    float scale, int causal, void* stream);
 // Backward, step 2 (fattn_pair.hip): dK, dV and dQ. part, done, epoch_slot (a split-size workspace,

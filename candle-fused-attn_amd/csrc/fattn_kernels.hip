@@ -82,14 +82,8 @@ void test_hook_state(int64_t out[3]) {
 }
 
 int bwd_split_keys(int64_t b, int64_t h, int64_t s, int d, int causal) {
-  // 128-key blocks (two 16-key groups per wave): half the dQ partials and half the per-tile
-  // staging and barriers per product. At d 64 they hold 2 waves per SIMD instead of 3. Measured
-  // (step 2, non-causal, d 64): s 384 +3.9 %, 512 -4.8 %, 768 -4.1 %, 1024 -6.7 %, 2048 -6.9 %,
-  // 4096 -3.6 %; causal +1 to +31 % (the diagonal blocks' masked work doubles). They need two
-  // workgroups per CU to fill the chip. At d 32 they keep 3 waves per SIMD and pay where the
-  // halved workgroup count leaves fewer than two rounds of them (b h s 256 +8 %, 512 +60 %,
-  // config 2's shape -2 %); from two rounds on (1536 workgroups) they gain: b16 h16 s768 -3.4 %,
-  // s1024 -5.0 %, b8 h16 s2048 -4.4 %, b4 h16 s4096 -4.2 %.
+  // (The rule of the size queries: 128-key blocks for non-causal launches that fill the chip with
+  // them. The kernels' own blocks are 128 rows at every shape.)
   const int64_t blocks128 = (s + 2 * kBwdKeys - 1) / (2 * kBwdKeys) * b * h;
   if (causal) return kBwdKeys;
   if (d == 32) return blocks128 >= 1536 ? 2 * kBwdKeys : kBwdKeys;
@@ -97,8 +91,7 @@ int bwd_split_keys(int64_t b, int64_t h, int64_t s, int d, int causal) {
   return blocks128 >= 512 ? 2 * kBwdKeys : kBwdKeys;
 }
 namespace {
-// The schedule of a launch over nbh (b, h) pairs with key blocks of `keys` keys (a chunk's keys
-// come from the whole launch's pair count: every chunk has the whole's arithmetic).
+// The plan of nbh (b, h) pairs with key blocks of `keys` keys.
 bool step2_sums_of(int64_t nbh, int64_t s, int d, int causal, int keys) {
   if (g_step2_sums.load(std::memory_order_relaxed) == 0) return false;
   // The range check keeps b h s (hence every count below) inside int32.

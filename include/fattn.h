@@ -28,7 +28,11 @@
  *     a message of this thread prefixed like the reference's (`fused_attention:` or
  *     `fused_attention_qkv:`);
  *   - empty inputs (batch, heads or seq 0) are a successful no-op (empty outputs);
- *   - all arithmetic is fp32; backward results are bit-identical from run to run.
+ *   - operands, sums and results are fp32: the products run on the f16 matrix cores with every
+ *     fp32 operand held as the sum of two f16 under a power-of-two scale (22 bits or more of each
+ *     value above 2^-17 of the largest of its 32-row tile, below that 2^-39 of that largest), and
+ *     are summed in fp32; a 32-row group whose result is not finite is computed again in plain
+ *     fp32. Results are bit-identical from run to run.
  */
 #ifndef FATTN_H
 #define FATTN_H
@@ -67,42 +71,35 @@ int fattn_fwd_f32(const float* q, const float* k, const float* v, float* o, floa
                   const int64_t v_strides[3], void* stream);
 
 /* Backward workspace (256-byte aligned). Replaces the temporaries cuda::backward allocates
- * (dsum and turn, src/cuda.rs:200-209). Its size picks how dQ is summed over key blocks:
- *   >= fattn_bwd_workspace_split_bytes: "split" -- every key block writes its dQ partials to the
- *      workspace (about s * s * b * h * d / 16 bytes); they are summed in key-block order by the
- *      last workgroups of step 2 (which wait, boundedly, only for key blocks dispatched before
- *      them) or by a third kernel; no key block waits on another (the faster way);
- *   below that, d <= 64, in fattn_bwd_f32 and the op-level backwards: "split by chunks" when the
- *      workspace holds the split state of enough (b, h) pairs for a chunk to fill the chip (a
- *      chunk of c pairs needs fattn_bwd_workspace_split_bytes(1, c, s, d)) -- steps 2 and 3 run
- *      per chunk of pairs, with the same results as the whole split, bit for bit;
- *   >= fattn_bwd_workspace_min_bytes, otherwise: "turns" -- key blocks add into dQ in place,
- *      in key-block order, under per-query-tile turn counters; D, counters and ticket only.
- * All are deterministic. fattn_bwd_workspace_bytes is the split size when that is at most
- * FATTN_SPLIT_MAX_BYTES, else the split of the largest worthwhile chunk within it (d <= 64),
- * else the minimum. All three return 0 for a negative size or an unsupported d. */
+ * (dsum and turn, src/cuda.rs:200-209). dQ is summed in registers by the workgroup that owns its
+ * rows, so only the control words at the start of the workspace are used, whatever its size; the
+ * sizes are those that callers already plan with, and every size that was accepted still is:
+ *   >= fattn_bwd_workspace_split_bytes: step 2 also keeps a flag per 16-query tile and the launch's
+ *      epoch in it, and the space of the tiles' dQ, which step 3 reads;
+ *   below that, d <= 64, in fattn_bwd_f32 and the op-level backwards: the split size of a chunk of
+ *      (b, h) pairs, fattn_bwd_workspace_split_bytes(1, c, s, d), also where that is below the
+ *      minimum;
+ *   >= fattn_bwd_workspace_min_bytes, otherwise.
+ * The results are the same, bit for bit. fattn_bwd_workspace_bytes is the split size when that is
+ * at most FATTN_SPLIT_MAX_BYTES, else the split of the largest worthwhile chunk within it
+ * (d <= 64), else the minimum; a caller that allocates per call does best with the minimum. All
+ * three return 0 for a negative size or an unsupported d. */
 #define FATTN_SPLIT_MAX_BYTES ((size_t)4 << 30)
 size_t fattn_bwd_workspace_bytes(int64_t b, int64_t h, int64_t s, int64_t d);
 size_t fattn_bwd_workspace_min_bytes(int64_t b, int64_t h, int64_t s, int64_t d);
 size_t fattn_bwd_workspace_split_bytes(int64_t b, int64_t h, int64_t s, int64_t d);
 
-/* Backward step 1: D[b, h, i] = sum_c dO[b, i, h, c] * O[b, i, h, c] (fixed order) and the
- * counters of step 2 cleared. O is [b, s, h, d] contiguous; dO is read through do_strides. With
- * a split-size workspace at d <= 64, and at d 128 with s <= 256, there is nothing to do (step 2
- * computes D itself, and tags the state of its own dQ sums with a value unique to its launch;
- * returns 0 after the checks).
+/* Backward step 1: the checks of its arguments. D[b, h, i] = sum_c dO[b, i, h, c] * O[b, i, h, c] is
+ * formed where step 2 reads dO, and no counter needs clearing, so nothing is launched.
  * Replaces the fattn_bwd_dot_f32_d64 launch (src/cuda.rs:215-231). */
 int fattn_bwd_prep_f32(const float* o, const float* d_o, const int64_t do_strides[3],
                        void* workspace, size_t workspace_bytes, int64_t b, int64_t h, int64_t s,
                        int64_t d, void* stream);
 
-/* Backward step 2: dK and dV into ONE [b, s, 3, h, d] buffer (the fused qkv projection's
- * gradient layout); dQ summed over key blocks in a fixed order, so every rerun is bit-identical:
- * with a split-size workspace its partials go to the workspace (this step sums some query
- * tiles, step 3 the rest) and, for d <= 64, D is computed here from O (the forward's
- * [b, s, h, d] output); else dQ is complete after this step. Where D is not computed here it
- * comes from step 1, which must run first on the same workspace (running step 1 first is always
- * correct). Replaces the fattn_bwd_f32_d64 launch (src/cuda.rs:233-258), which takes no O. */
+/* Backward step 2: dQ, dK and dV into ONE [b, s, 3, h, d] buffer (the fused qkv projection's
+ * gradient layout), each row summed by one workgroup in a fixed order, so every rerun is
+ * bit-identical. O is the forward's [b, s, h, d] output. Replaces the fattn_bwd_f32_d64 launch
+ * (src/cuda.rs:233-258), which takes no O. */
 int fattn_bwd_main_f32(const float* q, const float* k, const float* v, const float* o,
                        const float* d_o, const float* lse, float* dqkv, void* workspace,
                        size_t workspace_bytes, int64_t b, int64_t h, int64_t s, int64_t d,
@@ -110,17 +107,14 @@ int fattn_bwd_main_f32(const float* q, const float* k, const float* v, const flo
                        const int64_t k_strides[3], const int64_t v_strides[3],
                        const int64_t do_strides[3], void* stream);
 
-/* Backward step 3: with a split-size workspace, dQ = scale * (sum of step 2's partials in
- * key-block order) into part 0 of dqkv, for every query tile the last step 2 launch on this
- * workspace did not sum itself (its last workgroups sum the tiles the schedule gives them; the
- * same operations in the same order, so the result does not depend on which kernel summed a
- * tile), then it clears the sums' flags; with a smaller workspace nothing to do (returns 0). Has
- * no counterpart launch in the reference (its dQ is summed in place, as the turn mode here). */
+/* Backward step 3: with a split-size workspace, dQ = scale * the workspace's tile into part 0 of
+ * dqkv for every query tile that the last step 2 launch on this workspace left there (none, unless
+ * a test hook asks for it); then it clears the tiles' flags. With a smaller workspace nothing to do
+ * (returns 0). Has no counterpart launch in the reference. */
 int fattn_bwd_dq_f32(float* dqkv, void* workspace, size_t workspace_bytes, int64_t b, int64_t h,
                      int64_t s, int64_t d, float scale, int causal, void* stream);
 
-/* All backward steps. Replaces cuda::backward (src/cuda.rs:187-260). Step 3 is launched only
- * where step 2 has no dQ sums, or while `stream` is capturing a HIP graph. */
+/* All backward steps: one launch. Replaces cuda::backward (src/cuda.rs:187-260). */
 int fattn_bwd_f32(const float* q, const float* k, const float* v, const float* o,
                   const float* d_o, const float* lse, float* dqkv, void* workspace,
                   size_t workspace_bytes, int64_t b, int64_t h, int64_t s, int64_t d,
@@ -132,10 +126,9 @@ int fattn_bwd_f32(const float* q, const float* k, const float* v, const float* o
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). It has no
  * counterpart in the reference. It calls no allocating routine: the workspace is the library's
  * static scratch, FATTN_STATIC_SCRATCH_BYTES of device memory per GPU, held until the process
- * ends. dQ is summed as fattn_bwd_f32 sums it with a workspace of that size (the same kernels
- * and results): the split way when its workspace fits in the scratch, else at d <= 64 split by
- * chunks of (b, h) pairs where such chunks fit and fill the chip, else by turns; a shape whose minimum
- * workspace exceeds the scratch is refused with FATTN_EWORKSPACE before any launch. Every call on
+ * ends. The launch is fattn_bwd_f32's with a workspace of that size, with its results; a shape
+ * that fattn_bwd_f32 refuses for a workspace of that size (its minimum exceeds the scratch and no
+ * chunk fits) is refused with FATTN_EWORKSPACE before any launch. Every call on
  * one GPU shares that GPU's scratch: calls that overlap on one GPU (two streams, two threads)
  * race and must be ordered by the caller. */
 #define FATTN_STATIC_SCRATCH_BYTES ((size_t)64 << 20)
@@ -225,10 +218,9 @@ const char* fattn_last_error(void);
 const char* fattn_version(void);
 
 /* Synchronises `stream`, then reads the backward's guard word from `workspace` into *status:
- * 0 = every dQ wait ended normally; nonzero = results are invalid: 1, a turn wait of the turn
- * hand-over hit its spin bound; 2, a ticket out of range (step 1 did not run on this
- * workspace); 3, a dQ sum of step 2 with no step 3 after it gave up waiting (the dQ rows
- * concerned hold NaN). For tests and debugging; any head_dim. */
+ * 0 = the last backward on the workspace was normal (its kernels wait for nothing, so it is);
+ * 3, a test hook made it give up a (b, h) pair with no step 3 after it (the dQ rows concerned hold
+ * NaN). 1 and 2 are not used any more. For tests and debugging; any head_dim. */
 int fattn_bwd_status(const void* workspace, size_t workspace_bytes, int64_t b, int64_t h,
                      int64_t s, void* stream, int* status);
 
