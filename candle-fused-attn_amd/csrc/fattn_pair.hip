@@ -60,9 +60,11 @@ __device__ __forceinline__ f16v zero16() { return f16v{}; }
 
 // 2^e, -126 <= e <= 127.
 __device__ __forceinline__ float pow2(int e) { return __int_as_float((e + 127) << 23); }
-// The exponent of a magnitude, at least -100 (so that every scale below is a normal float).
+// The exponent of a magnitude, at least kMinExp: 2^(kTop - e) and its inverse are normal floats, and
+// the smallest normal float is still scaled to 1, where both its terms are whole.
+constexpr int kMinExp = kTop - 126;
 __device__ __forceinline__ int exponent(float x) {
-  return max(static_cast<int>((__float_as_uint(x) >> 23) & 255u) - 127, -100);
+  return max(static_cast<int>((__float_as_uint(x) >> 23) & 255u) - 127, kMinExp);
 }
 
 // The scale of a tile whose largest magnitude has exponent e. A tile with an infinity (exponent 128)
@@ -487,7 +489,7 @@ fwd_pair_kernel(FwdArgs a) {
   // are scaled by; V's is the largest so far (its tiles are summed into one accumulator).
   Stage<D> st;
   Pair q[NQ][kKS];
-  float cq[NQ];  // |scale| log2 e over the query's scale
+  float uq[NQ];  // 1 / the query's scale
   int ek[2], ev[2];
   {
     OwnRows<D> own[NQ];
@@ -502,7 +504,7 @@ fwd_pair_kernel(FwdArgs a) {
     st.load(kop, vop, kRows, S - 1, w, lane);
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
-      cq[n] = own[n].split(a.scale < 0.0f ? -1.0f : 1.0f, q[n]) * (fabsf(a.scale) * kLog2e);
+      uq[n] = own[n].split(a.scale < 0.0f ? -1.0f : 1.0f, q[n]);
     }
     st.put_maxima(sm.mx, 1, w, lane);
     ek[1] = ek[0], ev[1] = ev[0];
@@ -569,7 +571,7 @@ fwd_pair_kernel(FwdArgs a) {
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
       const int qi = qw0 + kRows * n + j;
-      const float c2 = cq[n] * pow2(ek[0] - kTop);
+      const float c2 = fabsf(a.scale) * kLog2e * (uq[n] * pow2(ek[0] - kTop));
       // Live: keys below S and, causal, not after the query.
       auto live = [&](int r) {
         const int key = kt0 + 8 * (r >> 2) + 4 * g + (r & 3);
@@ -663,7 +665,7 @@ fwd_pair_kernel(FwdArgs a) {
     }
     // O through LDS (the wave's own part; every wave is past its last tile), so that each row is
     // written as whole 128-byte lines.
-    const float inv = pow2(e_o - kTop) / l;
+    const float inv = 1.0f / l, unit = pow2(e_o - kTop);  // (apart: inv unit may be subnormal)
     float* so = sm.t.o[w];
 #pragma unroll
     for (int c0 = 0; c0 < D; c0 += kOCols) {
@@ -673,7 +675,7 @@ fwd_pair_kernel(FwdArgs a) {
         for (int i = 0; i < 4; ++i) {
           const f4 x{acc[n][dt][4 * i], acc[n][dt][4 * i + 1], acc[n][dt][4 * i + 2],
                      acc[n][dt][4 * i + 3]};
-          st4(so + j * kOPitch + 32 * dt - c0 + 8 * i + 4 * g, x * inv);
+          st4(so + j * kOPitch + 32 * dt - c0 + 8 * i + 4 * g, x * inv * unit);
         }
       }
       constexpr int kLanes = kOCols / 4;  // lanes per row
@@ -882,11 +884,12 @@ __device__ void bwd_query_fp32(const BwdPairArgs& a, int b, int h, int qi, int l
   }
 }
 
-// 32 rows x D of an accumulator (times `f`, per lane), through the wave's part of LDS, to rows of
-// `stride` floats.
+// 32 rows x D of an accumulator (times f f2, per lane), through the wave's part of LDS, to rows of
+// `stride` floats. Two factors: their product may be below the least float, where it is 0 or, as a
+// pow2() out of range, anything, while a sum times it is not.
 template <int D, int N>
-__device__ __forceinline__ void store_rows(const f16v (&acc)[N], float f, float* so, float* base,
-                                           int64_t stride, int rows, int lane) {
+__device__ __forceinline__ void store_rows(const f16v (&acc)[N], float f, float f2, float* so,
+                                           float* base, int64_t stride, int rows, int lane) {
   constexpr int kCols = D < 64 ? D : 64, kPitch = kCols + 4, kLanes = kCols / 4;
   const int j = lane & 31, g = lane >> 5;
 #pragma unroll
@@ -896,7 +899,7 @@ __device__ __forceinline__ void store_rows(const f16v (&acc)[N], float f, float*
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const f4 x{acc[dt][4 * i], acc[dt][4 * i + 1], acc[dt][4 * i + 2], acc[dt][4 * i + 3]};
-        st4(so + j * kPitch + 32 * dt - c0 + 8 * i + 4 * g, x * f);
+        st4(so + j * kPitch + 32 * dt - c0 + 8 * i + 4 * g, x * f * f2);
       }
     }
 #pragma unroll
@@ -1037,7 +1040,7 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
       load(u + 2);
       pin_loads();
     }
-    const float cs = a.scale * kLog2e * uk * pow2(eq[0] - kTop), cg = uv * pow2(eg[0] - kTop);
+    const float cs = a.scale * kLog2e * (uk * pow2(eq[0] - kTop)), cg = uv * pow2(eg[0] - kTop);
     // Live: register r's query, q0 + 4 g + 8 i + e, below S and, causal, not before the key.
     const int hi = key < S ? S - q0 - 4 * g : 0, lo = kCausal ? key - q0 - 4 * g : 0;
 #pragma unroll
@@ -1123,7 +1126,7 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
   }
   for (; u < nsteps; ++u) masked(u);
   if (!wave_live) return;
-  const float fk = pow2(e_k - kTop - kp) / dsc * a.scale;
+  const float fk = pow2(-kp) / dsc * a.scale;
   const float z = probe_finite<kDT>(dk, probe_finite<kDT>(dv, fk * 0.0f));
   if (__builtin_amdgcn_ballot_w64(key < S && !(z == 0.0f)) != 0) {
     for (int i = 0; i < kRows && kw0 + i < S; ++i) bwd_key_fp32<D>(a, b, h, kw0 + i, lane);
@@ -1131,9 +1134,9 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
   }
   const int64_t part = static_cast<int64_t>(a.H) * D;
   float* row = a.dqkv + (static_cast<int64_t>(b) * S + kw0) * 3 * part + static_cast<int64_t>(h) * D;
-  store_rows<D>(dk, fk, sm.o[w], row + part, 3 * part, S - kw0, lane);
-  store_rows<D>(dv, pow2(e_v - kTop - (kSerial ? kp : kPTop)), sm.o[w], row + 2 * part, 3 * part,
-                S - kw0, lane);
+  store_rows<D>(dk, pow2(e_k - kTop), fk, sm.o[w], row + part, 3 * part, S - kw0, lane);
+  store_rows<D>(dv, pow2(e_v - kTop), pow2(kSerial ? -kp : -kPTop), sm.o[w], row + 2 * part,
+                3 * part, S - kw0, lane);
 }
 
 template <int D, bool kCausal>
@@ -1249,7 +1252,7 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
       for (int ks = 0; ks < kKS; ++ks) dp = mma(x[ks], gB[ks].h, dp);
     }
     load(t);
-    const float cs = a.scale * kLog2e * uq * pow2(ek[0] - kTop), cg = ug * pow2(ev[0] - kTop);
+    const float cs = a.scale * kLog2e * (uq * pow2(ek[0] - kTop)), cg = ug * pow2(ev[0] - kTop);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int key = kt0 + 8 * (r >> 2) + 4 * g + (r & 3);
@@ -1304,7 +1307,7 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
                             static_cast<int64_t>(h) * D
                       : a.part + (static_cast<int64_t>(bh) * ntile16 * kBwdQueryTile + qw0) * D;
   const float factor = direct ? a.scale : 1.0f;
-  const float un = pow2(e_q - kTop - kp) / dsc;
+  const float un = pow2(-kp) / dsc;
   const bool bad = __builtin_amdgcn_ballot_w64(
                        qi < S && !(probe_finite<kDT>(dq, un * 0.0f) == 0.0f)) != 0;
   if (gave_up && direct) {
@@ -1312,13 +1315,13 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
     if (lane == 0) {
       __hip_atomic_store(a.ctrl + kCtrlGuard, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    store_rows<D>(dq, __builtin_nanf(""), sm.o[w], row, stride, S - qw0, lane);
+    store_rows<D>(dq, __builtin_nanf(""), 1.0f, sm.o[w], row, stride, S - qw0, lane);
   } else if (bad) {
     for (int i = 0; i < kRows && qw0 + i < S; ++i) {
       bwd_query_fp32<D>(a, b, h, qw0 + i, lane, row + i * stride, factor);
     }
   } else {
-    store_rows<D>(dq, un * factor, sm.o[w], row, stride, S - qw0, lane);
+    store_rows<D>(dq, pow2(e_q - kTop), un * factor, sm.o[w], row, stride, S - qw0, lane);
   }
 }
 

@@ -202,3 +202,64 @@ def test_backward_output_over_4gib(cuda):
         at = slice(i, i + 1)
         check_gradients([t[at] for t in got], reference(q[at], k[at], v[at], 0.1, False, g[at])[1:],
                         f"head {i}")
+
+
+@pytest.mark.parametrize("n", [3, 33])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_backward_zero_gradient(cuda, d, causal, n):
+    """The output gradient zero for a whole pair, from a query on (a padded tail: whole key blocks
+    see only zeros), and everywhere: gradients of exactly 0 where the products have nothing else.
+    Causal, 3 and 33 pairs lie on either side of the serial dV rule."""
+    s, tail = 256, 120
+    q, k, v, g = (normal(120 + i, n, s, d) for i in range(4))
+    g[0] = 0
+    g[1, tail:] = 0
+    got, want = gradients(q, k, v, g, 0.125, causal), reference(q, k, v, 0.125, causal, g)[1:]
+    for a in got:
+        assert torch.equal(a[0], torch.zeros_like(a[0]))
+        if causal:
+            assert torch.equal(a[1, tail:], torch.zeros_like(a[1, tail:]))
+    check_gradients(got, want, f"zero gradient d{d} causal={causal}")
+    for a in gradients(q, k, v, torch.zeros_like(g), 0.125, causal):
+        assert torch.equal(a, torch.zeros_like(a))
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_zero_operands(cuda, d, causal):
+    """Each of q, k, v zero in turn: uniform weights, a zero output, and the gradients that are 0."""
+    s = 130
+    for which in range(3):
+        q, k, v, g = (normal(140 + i, 2, s, d) for i in range(4))
+        (q, k, v)[which].zero_()
+        want = reference(q, k, v, 0.125, causal, g)
+        got = [forward(q, k, v, 0.125, causal), *gradients(q, k, v, g, 0.125, causal)]
+        for name, a, w in zip(("o", "dq", "dk", "dv"), got, want):
+            if not w.any():
+                assert torch.equal(a, torch.zeros_like(a)), (which, name)
+                continue
+            e = rel(a, w)
+            print(f"operand {which} zero, d{d} causal={causal} {name}: {e:.2e}", flush=True)
+            assert e <= REL_TOL, (which, name)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("f", [1e-28, 1e-30, 1e-32, 1e-35])
+def test_tiny_magnitudes(cuda, f, causal):
+    """Output gradients and values near the least normal float. Each result within the bar of its
+    norm, or within one least subnormal (2^-149) per element where it is that small; dQ and dK of
+    tiny values take the scale's bits off the bottom of that range."""
+    s, d = 200, 64
+    q, k, v, g = (normal(160 + i, 2, s, d) for i in range(4))
+
+    def check(name, got, want):
+        diff = (got.detach().double().cpu() - want).norm().item()
+        floor = 2.0 ** -149 * math.sqrt(want.numel())
+        print(f"{f:g} causal={causal} {name}: {diff / want.norm().item():.2e}", flush=True)
+        assert diff <= REL_TOL * want.norm().item() + floor, name
+
+    got, want = gradients(q, k, v, g * f, 0.125, causal), reference(q, k, v, 0.125, causal, g * f)
+    for name, a, w in zip(("dq", "dk", "dv"), got, want[1:]):
+        check(name, a, w)
+    check("o", forward(q, k, v * f, 0.125, causal), reference(q, k, v * f, 0.125, causal)[0])
