@@ -14,12 +14,17 @@
 // 4.6e-8 at 64 terms, but twice the products run into the power limit: the clock fell to 1.82 GHz
 // where the fp32 kernel holds 2.41, and the forward at b 16 h 16 s 1024 took 352 us against 524.)
 //
-// Scales. f16 spans 2^-14 .. 2^16 (normal), so operands carry exact powers of two: a wave's own
-// rows (register operands) one per row, a staged 32-row tile one per tile, from the largest
-// magnitude in it: the stored maximum is in [2^13, 2^14), and an element keeps its 22 bits down to
-// 2^-17 of that maximum (below, an absolute error of 2^-39 of it). The scales multiply back into
-// factors the softmax applies anyway; sums over several tiles follow a running maximum of the
-// tiles' exponents.
+// Scales. f16 spans 2^-14 .. 2^16 (normal), so every row of an operand carries its own exact power
+// of two, from the largest magnitude in it: that is stored in [2^kTop, 2^(kTop + 1)), and an element
+// keeps its 22 bits down to 2^-17 of its row's largest (below, an absolute error of 2^-39 of it). A
+// wave's own rows hold theirs in a register; a staged row's is in LDS beside the tile (`unit`, 2^e)
+// and multiplies back per accumulator row: into the scores' factor, and, where the product sums over
+// the staged rows, into the weights (P, dS). The weights of a lane's own row follow a power of two
+// of their own, so that they keep 22 bits down to about 2^-17 of the largest term of the sum, and no
+// term's error depends on a row that has no part in it. (One scale per tile, or the largest so far,
+// costs less: forward b64 h6 s240 33.5 us against 35.5, b16 h16 s1024 204 against 231, backward 104
+// against 106 and 787 against 807, d 128 227 against 248. But one large row, masked or not, or one
+// key of large weight, takes the bits of all the others.)
 //
 // For one v_mfma_f32_32x32x16_f16, lane l (j = l % 32, g = l / 32) supplies A[j][8 g + e] and
 // B[8 g + e][j], e = 0..7, and holds D[8 (r / 4) + 4 g + r % 4][j], r = 0..15. As the contraction
@@ -60,17 +65,11 @@ __device__ __forceinline__ f16v zero16() { return f16v{}; }
 
 // 2^e, -126 <= e <= 127.
 __device__ __forceinline__ float pow2(int e) { return __int_as_float((e + 127) << 23); }
-// The exponent of a magnitude, at least kMinExp: 2^(kTop - e) and its inverse are normal floats, and
-// the smallest normal float is still scaled to 1, where both its terms are whole.
-constexpr int kMinExp = kTop - 126;
+// The exponent of a magnitude, within [kMinExp, kMaxExp] (0, subnormals, infinities): every 2^e,
+// 2^-e and 2^(kTop - e) is a normal float, and the smallest normal one is still scaled to 1.
+constexpr int kMinExp = kTop - 126, kMaxExp = 126;
 __device__ __forceinline__ int exponent(float x) {
-  return max(static_cast<int>((__float_as_uint(x) >> 23) & 255u) - 127, kMinExp);
-}
-
-// The scale of a tile whose largest magnitude has exponent e. A tile with an infinity (exponent 128)
-// becomes NaN as a whole: its other rows would vanish beside it, unseen where its own is masked.
-__device__ __forceinline__ float tile_scale(int e) {
-  return e == 128 ? __builtin_nanf("") : pow2(kTop - e);
+  return min(max(static_cast<int>(__float_as_uint(x) >> 23) - 127, kMinExp), kMaxExp);
 }
 
 // Eight values times a scale, in two terms.
@@ -93,15 +92,6 @@ __device__ __forceinline__ void split2(float x, float y, float sc, unsigned& h, 
              static_cast<_Float16>(fmaf(y, sc, -static_cast<float>(b.y)))};
   l = __builtin_bit_cast(unsigned, c);
 }
-// x = h + l, two values: three instructions.
-__device__ __forceinline__ void split2(float x, float y, unsigned& h, unsigned& l) {
-  h = __builtin_bit_cast(unsigned, __builtin_convertvector(f2{x, y}, h2));
-  asm("" : "+v"(h));
-  const h2 b = __builtin_bit_cast(h2, h);
-  const h2 c{static_cast<_Float16>(fmaf(static_cast<float>(b.x), -1.0f, x)),
-             static_cast<_Float16>(fmaf(static_cast<float>(b.y), -1.0f, y))};
-  l = __builtin_bit_cast(unsigned, c);
-}
 __device__ __forceinline__ Pair split8(f4 x, f4 y, float sc) {
   unsigned h[4], l[4];
   split2(x[0], x[1], sc, h[0], l[0]);
@@ -110,12 +100,12 @@ __device__ __forceinline__ Pair split8(f4 x, f4 y, float sc) {
   split2(y[2], y[3], sc, h[3], l[3]);
   return make_pair8(h, l);
 }
-// Registers 8 KS .. 8 KS + 7 of an accumulator as a B operand.
+// Registers 8 KS .. 8 KS + 7 of an accumulator, times a scale, as a B operand.
 template <int KS>
-__device__ __forceinline__ Pair split_acc(const f16v& x) {
+__device__ __forceinline__ Pair split_acc(const f16v& x, float sc) {
   unsigned h[4], l[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) split2(x[8 * KS + 2 * i], x[8 * KS + 2 * i + 1], h[i], l[i]);
+  for (int i = 0; i < 4; ++i) split2(x[8 * KS + 2 * i], x[8 * KS + 2 * i + 1], sc, h[i], l[i]);
   return make_pair8(h, l);
 }
 __device__ __forceinline__ f16v mma_small(const Pair& a, const Pair& b, f16v c) {
@@ -194,15 +184,23 @@ __device__ __forceinline__ float pair_max(float x) {
   const auto p = __builtin_amdgcn_permlane32_swap(u, u, false, false);
   return vmax(__uint_as_float(p[0]), __uint_as_float(p[1]));
 }
-// The max over each half of the wave.
-__device__ __forceinline__ float half_max(float x) {
-  x = fmaxf(x, dpp<0xB1>(x));
-  x = fmaxf(x, dpp<0x4E>(x));
-  x = fmaxf(x, dpp<0x141>(x));
-  x = fmaxf(x, dpp<0x140>(x));
-  const unsigned u = __float_as_uint(x);
-  const auto p = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  return vmax(__uint_as_float(p[0]), __uint_as_float(p[1]));
+// The max of magnitudes over each aligned group of N lanes (4, 8 or 16), as integers: one
+// instruction per step, where fmaxf quiets its inputs first.
+template <int CTRL>
+__device__ __forceinline__ unsigned max_dpp(unsigned x) {
+  return max(x, static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), CTRL, 0xF,
+                                                                  0xF, true)));
+}
+template <int N>
+__device__ __forceinline__ float group_max(float m) {
+  // (The mask is an instruction between an asm's result and the lane move that reads it: the compiler
+  // counts that wait from the instructions it knows.)
+  unsigned x = __float_as_uint(m) & 0x7fffffffu;
+  x = max_dpp<0xB1>(x);
+  x = max_dpp<0x4E>(x);
+  if constexpr (N >= 8) x = max_dpp<0x141>(x);
+  if constexpr (N >= 16) x = max_dpp<0x140>(x);
+  return __uint_as_float(x);
 }
 __device__ __forceinline__ float wave_sum(float x) {
 #pragma unroll
@@ -224,9 +222,6 @@ __device__ __forceinline__ float abs_max8(f4 x, f4 y, float m) {
 // No memory access moves across: a step's loads are issued before its LDS reads (left to itself the
 // compiler sinks them to their first use, at the end of the step).
 __device__ __forceinline__ void pin_loads() { asm volatile("" ::: "memory"); }
-// No instruction moves across: keeps the compiler from overlapping phases whose registers together
-// do not fit.
-__device__ __forceinline__ void fence_phase() { __builtin_amdgcn_sched_barrier(0); }
 // 0 where every value is finite, else NaN.
 template <int N>
 __device__ __forceinline__ float probe_finite(const f16v (&x)[N], float z) {
@@ -241,21 +236,18 @@ __device__ __forceinline__ float probe_finite(const f16v (&x)[N], float z) {
 // --- Staging -----------------------------------------------------------------------------------
 // Two operands' tiles of 32 rows through the registers of a workgroup of four waves: wave w takes
 // rows 8 w .. 8 w + 7 of both (D 32: operand a in lanes 0..31, b in the others), eight columns per
-// lane and access. A tile is loaded in one step of the walk, its maxima (one per wave and operand)
-// go to LDS at the end of that step, and after the step's barrier the next step scales, splits and
-// stores it.
+// lane and access. A tile is loaded in one step of the walk; the next step takes each row's largest
+// magnitude (over the lanes that hold the row), scales, splits and stores it.
 struct Operand {
   const char* p;  // row 0 of the (b, h)
   unsigned ss4;   // row stride in bytes
-};
-struct Maxima {
-  float m[2][2][4];  // by the step's parity, operand and wave
 };
 template <int D>
 struct Stage {
   static constexpr int kC = D / 8;                // chunks per row
   static constexpr int kN = D == 32 ? 1 : D / 32;  // accesses per lane: a's, then b's
   f4 x[kN][2];
+  int e[kN];  // the access's row's exponent (after store)
 
   static __device__ __forceinline__ int row(int i, int w, int lane) {
     if constexpr (D == 32) return 8 * w + (lane & 31) / kC;
@@ -275,34 +267,16 @@ struct Stage {
       x[i][1] = *reinterpret_cast<const f4*>(p + off + 16);
     }
   }
-  __device__ __forceinline__ void put_maxima(Maxima& mx, int parity, int w, int lane) const {
-    float m;
-    if constexpr (kN == 1) {
-      m = fmaxf(abs_max8(x[0][0], x[0][1], 0.0f), 0.0f);
-    } else {
-      float ma = 0.0f, mb = 0.0f;
-#pragma unroll
-      for (int i = 0; i < kN; ++i) {
-        float& t = i < kN / 2 ? ma : mb;
-        t = abs_max8(x[i][0], x[i][1], t);
-      }
-      // a's into the lower half, b's into the upper. (The swaps must not read an asm's result: the
-      // compiler counts their wait states from the instructions it knows.)
-      ma = fmaxf(ma, 0.0f), mb = fmaxf(mb, 0.0f);
-      const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(ma), __float_as_uint(mb),
-                                                      false, false);
-      m = vmax(__uint_as_float(p[0]), __uint_as_float(p[1]));
-    }
-    m = half_max(m);
-    if ((lane & 31) == 0) mx.m[parity][lane >> 5][w] = m;
-  }
-  __device__ __forceinline__ void store(Tile<D>& a, Tile<D>& b, float sa, float sb, int w,
-                                        int lane) const {
+  // The tiles and their rows' units (2^e).
+  __device__ __forceinline__ void store(Tile<D>& a, Tile<D>& b, float* ua, float* ub, int w,
+                                        int lane) {
 #pragma unroll
     for (int i = 0; i < kN; ++i) {
       const bool is_b = kN == 1 ? lane >= 32 : i >= kN / 2;
       const int r = row(i, w, lane);
-      const Pair s = split8(x[i][0], x[i][1], is_b ? sb : sa);
+      e[i] = exponent(group_max<kC>(abs_max8(x[i][0], x[i][1], 0.0f)));
+      if (lane % kC == 0) (is_b ? ub : ua)[r] = pow2(e[i]);
+      const Pair s = split8(x[i][0], x[i][1], pow2(kTop - e[i]));
       char* p = reinterpret_cast<char*>(is_b ? &b : &a) + r * (2 * D) +
                 (((lane % kC) ^ chunk_swz<D>(r)) << 4);
       *reinterpret_cast<h8*>(p) = s.h;
@@ -311,7 +285,7 @@ struct Stage {
   }
 };
 // Beside a Stage whose operand b is dO: O's rows in the same lanes, and D = rowsum(dO o O) of the
-// tile's 32 rows. O's offsets are in elements: its rows of one (b, h) may span more than 4 GiB (the
+// tile's 32 rows, in units of dO's rows. O's offsets are in elements: its rows of one (b, h) may span more than 4 GiB (the
 // views' may not).
 template <int D>
 struct RowDots {
@@ -338,16 +312,12 @@ struct RowDots {
       t += dpp<0x4E>(t);
       if constexpr (D >= 64) t += dpp<0x141>(t);
       if constexpr (D == 128) t += dpp<0x140>(t);
-      if (lane % kC == 0 && (D != 32 || lane >= 32)) dst[Stage<D>::row(i, w, lane)] = t;
+      if (lane % kC == 0 && (D != 32 || lane >= 32)) {
+        dst[Stage<D>::row(i, w, lane)] = t * pow2(-st.e[Stage<D>::kN / 2 + i]);
+      }
     }
   }
 };
-// The exponent of operand `o`'s staged tile (wave-uniform).
-__device__ __forceinline__ int tile_exponent(const Maxima& mx, int parity, int o) {
-  const f4 m = *reinterpret_cast<const f4*>(mx.m[parity][o]);
-  const float x = fmaxf(fmaxf(m.x, m.y), fmaxf(m.z, m.w));
-  return exponent(__int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))));
-}
 // A wave's own 32 rows as B operands: row j, columns 16 ks + 8 g .. + 7 of each step, scaled per
 // row (lanes j and j + 32 hold one row). Returns 1 / scale (without `sign`).
 template <int D>
@@ -380,13 +350,19 @@ struct OwnRows {
 //   O^T += V^T P^T (A = V transposed, B = P from S^T's registers).
 // Two LDS buffers, one barrier per tile: a step works on tile t, stores tile t + 1 and loads tile
 // t + 2.
-// The softmax: p = 2^(s c2 - m), c2 = |scale| log2 e and the two operands' scales, m a reference
-// that is kRefTop below the largest score seen when it was set. p is computed with the m in hand
-// and its row sum is what is tested: only where it exceeds kRowTop (or m is not set yet) is the
-// tile's max taken, m moved, O and the row sum rescaled and p computed again, so that an ordinary
-// tile pays neither a max nor a rescale, and every p stays below f16's limit.
+// The softmax: p = 2^(s c2 - m), c2 = |scale| log2 e and the two rows' scales, m a reference that is
+// kRefTop below the largest score seen when it was set. p is computed with the m in hand and its
+// row sum is what is tested: only where it exceeds kRowTop (or m is not set yet) is the tile's
+// largest score taken, m moved and p computed again, so that an ordinary tile pays no rescale.
+// What enters O's product is p times the unit of its V row and the query's running power of two
+// `wsc`, which puts the largest such weight at 2^kWTop when it is set, moves with m and falls where a
+// weight would pass f16's limit: a key of large weight and small V (an attention sink), or a large V
+// row of no weight, leaves the others' bits alone. (kWTop: 10 bits of room before a weight moves it.)
 constexpr float kRefTop = 3.0f;
 constexpr float kRowTop = 32768.0f;
+constexpr int kWTop = 6;
+constexpr float kMaxWeight = 61440.0f;  // of a scaled weight (f16 ends at 65504)
+constexpr float kMaxScale = 0x1p127f;   // of a running scale, and where it starts
 
 // One query's output row and L in plain fp32 by one wave: lanes take keys for the scores and dims
 // for the output.
@@ -455,7 +431,7 @@ fwd_pair_kernel(FwdArgs a) {
   };
   struct Smem {
     Tiles t;
-    Maxima mx;
+    float uk[2][kRows], uv[2][kRows];
   };
   __shared__ __attribute__((aligned(16))) Smem sm;
 
@@ -485,38 +461,31 @@ fwd_pair_kernel(FwdArgs a) {
   const bool wave_live = qw0 < S;
 
   // The first tile, the wave's queries (negated for a negative scale, so that the raw scores' max
-  // is the scaled scores'), and the second tile's loads. ek, ev: the exponents that tiles t, t + 1
-  // are scaled by; V's is the largest so far (its tiles are summed into one accumulator).
+  // is the scaled scores'), and the second tile's loads.
   Stage<D> st;
   Pair q[NQ][kKS];
-  float uq[NQ];  // 1 / the query's scale
-  int ek[2], ev[2];
+  float cq[NQ];  // |scale| log2 e over the scales of the query and kTop
   {
     OwnRows<D> own[NQ];
     st.load(kop, vop, 0, S - 1, w, lane);
 #pragma unroll
     for (int n = 0; n < NQ; ++n) own[n].load(qp + min(qw0 + kRows * n + j, S - 1) * a.q.ss, g);
-    st.put_maxima(sm.mx, 0, w, lane);
-    __syncthreads();
-    ek[0] = tile_exponent(sm.mx, 0, 0);
-    ev[0] = tile_exponent(sm.mx, 0, 1);
-    st.store(sm.t.kv[0].k, sm.t.kv[0].v, tile_scale(ek[0]), tile_scale(ev[0]), w, lane);
+    st.store(sm.t.kv[0].k, sm.t.kv[0].v, sm.uk[0], sm.uv[0], w, lane);
     st.load(kop, vop, kRows, S - 1, w, lane);
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
-      uq[n] = own[n].split(a.scale < 0.0f ? -1.0f : 1.0f, q[n]);
+      cq[n] = own[n].split(a.scale < 0.0f ? -1.0f : 1.0f, q[n]) *
+              (fabsf(a.scale) * kLog2e * pow2(-kTop));
     }
-    st.put_maxima(sm.mx, 1, w, lane);
-    ek[1] = ek[0], ev[1] = ev[0];
   }
 
-  f16v acc[NQ][kDT];  // O^T, in units of p and 2^(e_o - kTop)
-  int e_o = ev[0];
-  float m[NQ], lsum[NQ];
+  f16v acc[NQ][kDT];  // O^T, in units of p / wsc and 2^-kTop
+  float m[NQ], lsum[NQ], wsc[NQ];
 #pragma unroll
   for (int n = 0; n < NQ; ++n) {
     m[n] = kNegInf;
     lsum[n] = 0.0f;
+    wsc[n] = kMaxScale;
 #pragma unroll
     for (int dt = 0; dt < kDT; ++dt) acc[n][dt] = zero16();
   }
@@ -527,28 +496,19 @@ fwd_pair_kernel(FwdArgs a) {
   for (int dt = 0; dt < kDT; ++dt) coff[dt] = col_off<D>(lane, dt);
 
   // Stores tile t + 1 (loaded in the last step) and issues the loads of tile t + 2.
-  auto stage = [&](int t, Kv& put) {
-    ek[1] = tile_exponent(sm.mx, (t + 1) & 1, 0);
-    ev[1] = max(tile_exponent(sm.mx, (t + 1) & 1, 1), ev[0]);
-    st.store(put.k, put.v, tile_scale(ek[1]), tile_scale(ev[1]), w, lane);
+  auto stage = [&](int t) {
+    const int put = (t + 1) & 1;
+    st.store(sm.t.kv[put].k, sm.t.kv[put].v, sm.uk[put], sm.uv[put], w, lane);
     st.load(kop, vop, (t + 2) * kRows, S - 1, w, lane);
     pin_loads();
   };
   // One tile: kFull, one with no mask. (Past the walk's end a step stages rows that repeat the last
   // one and nothing reads: tested for, the loaded registers would live across the whole step.)
-  auto tile = [&](auto fullc, int t, const Kv& cur, Kv& put) {
+  auto tile = [&](auto fullc, int t) {
     constexpr bool kFull = decltype(fullc)::value != 0;
     const int kt0 = t * kRows;
-    if (ev[0] > e_o) {  // wave-uniform: V's largest exponent grows (by the tiles this wave uses)
-      const float f = e_o - ev[0] < -126 ? 0.0f : pow2(e_o - ev[0]);
-      e_o = ev[0];
-#pragma unroll
-      for (int n = 0; n < NQ; ++n) {
-#pragma unroll
-        for (int dt = 0; dt < kDT; ++dt) acc[n][dt] *= f;
-      }
-    }
-    stage(t, put);
+    const Kv& cur = sm.t.kv[t & 1];
+    stage(t);
     f16v s[NQ];
     {
       h8 kh[kKS];
@@ -571,42 +531,71 @@ fwd_pair_kernel(FwdArgs a) {
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
       const int qi = qw0 + kRows * n + j;
-      const float c2 = fabsf(a.scale) * kLog2e * (uq[n] * pow2(ek[0] - kTop));
       // Live: keys below S and, causal, not after the query.
       auto live = [&](int r) {
         const int key = kt0 + 8 * (r >> 2) + 4 * g + (r & 3);
         return kFull || (key < S && !(kCausal && key > qi));
       };
       f16v e;
-      float psum = 0.0f;
+      float psum = 0.0f, wmax = 0.0f;
+      // The weights (e) and their largest.
       auto exps = [&] {
+        wmax = 0.0f;
+        int r0 = 4 * g;
+        asm("" : "+v"(r0));  // (the units are read again the second time, not held)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float x = exp2_hw(fmaf(s[n][r], c2, -m[n]));
-          e[r] = live(r) ? x : 0.0f;
-          psum = r == 0 ? e[r] : psum + e[r];
+        for (int i = 0; i < 4; ++i) {
+          const f4 uk = ld4(&sm.uk[t & 1][8 * i + r0]), uv = ld4(&sm.uv[t & 1][8 * i + r0]);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const int r = 4 * i + c;
+            const float x = exp2_hw(fmaf(s[n][r], cq[n] * uk[c], -m[n]));
+            const float p = live(r) ? x : 0.0f;
+            psum = r == 0 ? p : psum + p;
+            e[r] = p * uv[c];
+          }
+          asm("v_max3_f32 %0, %1, %2, %0" : "+v"(wmax) : "v"(e[4 * i]), "v"(e[4 * i + 1]));
+          asm("v_max3_f32 %0, %1, %2, %0" : "+v"(wmax) : "v"(e[4 * i + 2]), "v"(e[4 * i + 3]));
         }
       };
       exps();
-      if (__builtin_amdgcn_ballot_w64(!(psum <= kRowTop)) != 0) {
+      if (__builtin_amdgcn_ballot_w64(!(psum <= kRowTop && wmax * wsc[n] <= kMaxWeight)) != 0) {
         float tmax = kNegInf;
+        int r0 = 4 * g;
+        asm("" : "+v"(r0));
 #pragma unroll
-        for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, live(r) ? s[n][r] : kNegInf);
-        tmax = pair_max(tmax);
-        // (c2 may be 0: a row with no live key keeps -inf.)
-        const float ref = tmax == kNegInf ? kNegInf : fmaf(tmax, c2, -kRefTop);
-        if (ref > m[n]) {
+        for (int r = 0; r < 16; ++r) {
+          const float x = s[n][r] * (cq[n] * sm.uk[t & 1][8 * (r >> 2) + r0 + (r & 3)]);
+          tmax = fmaxf(tmax, live(r) ? x : kNegInf);
+        }
+        // (-inf: a row with no live key.)
+        const float ref = pair_max(tmax) - kRefTop;
+        if (!(pair_sum(psum) <= kRowTop) && ref > m[n]) {
+          // O's unit is p / wsc: wsc rises as p falls, O stays as it is but for rounding.
           const float alpha = m[n] == kNegInf ? 0.0f : exp2_hw(m[n] - ref);
+          float to = kMaxScale, f = 0.0f;
+          if (alpha > 0x1p-100f) {
+            to = fminf(wsc[n] * pow2(-exponent(alpha)), kMaxScale);
+            f = alpha * (to / wsc[n]);
+          }
           m[n] = ref;
           lsum[n] *= alpha;
+          wsc[n] = to;
 #pragma unroll
-          for (int dt = 0; dt < kDT; ++dt) acc[n][dt] *= alpha;
+          for (int dt = 0; dt < kDT; ++dt) acc[n][dt] *= f;
+          exps();
         }
-        exps();
+        wmax = pair_max(fmaxf(wmax, 0.0f));
+        if (wmax * wsc[n] > kMaxWeight) {
+          const float to = pow2(kWTop - exponent(wmax));
+#pragma unroll
+          for (int dt = 0; dt < kDT; ++dt) acc[n][dt] *= to / wsc[n];
+          wsc[n] = to;
+        }
       }
       lsum[n] += psum;
-      p[n][0] = split_acc<0>(e);
-      p[n][1] = split_acc<1>(e);
+      p[n][0] = split_acc<0>(e, wsc[n]);
+      p[n][1] = split_acc<1>(e, wsc[n]);
     }
     const bool second = kFull || kt0 + 16 < kw_end;  // wave-uniform: the last 16 keys are live
 #pragma unroll
@@ -620,31 +609,25 @@ fwd_pair_kernel(FwdArgs a) {
         for (int n = 0; n < NQ; ++n) acc[n][dt] = mma3(v1, p[n][1], acc[n][dt]);
       }
     }
-    st.put_maxima(sm.mx, t & 1, w, lane);
-  };
-  auto advance = [&] {
-    __syncthreads();  // tile t + 1 is staged; every wave is done with tile t
-    ek[0] = ek[1], ev[0] = ev[1];
   };
   // Tiles wholly below S (and, causal, at or before the wave's first query) need no mask.
   const int full_end = (kCausal ? min(S, qw0 + 1) : S) / kRows;
   const int nfull = wave_live ? min(full_end, ntiles) : 0;
-  __syncthreads();  // tile 0, and tile 1's maxima
+  __syncthreads();  // tile 0
   int t = 0;
   for (; t < nfull; ++t) {
     if (!kCausal) prio_by_remaining(ntiles - t, ntiles);
-    tile(Const<1>{}, t, sm.t.kv[t & 1], sm.t.kv[(t + 1) & 1]);
-    advance();
+    tile(Const<1>{}, t);
+    __syncthreads();  // tile t + 1 is staged; every wave is done with tile t
   }
   for (; t < ntiles; ++t) {
     if (!kCausal) prio_by_remaining(ntiles - t, ntiles);
     if (wave_live && t * kRows < kw_end) {
-      tile(Const<0>{}, t, sm.t.kv[t & 1], sm.t.kv[(t + 1) & 1]);
+      tile(Const<0>{}, t);
     } else {
-      stage(t, sm.t.kv[(t + 1) & 1]);
-      st.put_maxima(sm.mx, t & 1, w, lane);
+      stage(t);
     }
-    advance();
+    __syncthreads();
   }
 
   // L = m / (log2 e as rounded into c2) + ln(l), to one rounding (in fp64, the logarithm of l's
@@ -665,7 +648,7 @@ fwd_pair_kernel(FwdArgs a) {
     }
     // O through LDS (the wave's own part; every wave is past its last tile), so that each row is
     // written as whole 128-byte lines.
-    const float inv = 1.0f / l, unit = pow2(e_o - kTop);  // (apart: inv unit may be subnormal)
+    const float inv = 1.0f / l, unit = pow2(-kTop) / wsc[n];  // (apart: the product may be subnormal)
     float* so = sm.t.o[w];
 #pragma unroll
     for (int c0 = 0; c0 < D; c0 += kOCols) {
@@ -725,9 +708,9 @@ fwd_pair_kernel(FwdArgs a) {
 // rounding) held per row and k about half of log2 s, so that the exponent stays near 0 whether a row
 // is flat (P about 1 / s) or peaked (P about 1): exp((S scale - L)) rounds its argument twice, at
 // -log2 s for a flat row, which was the largest error of the gradients.
-// Scales: P (at most 1) enters its product as P 2^kPTop; dS per lane (its key, or query) as dS times
-// a running power of two, lowered (and the sums with it) when a value would pass f16's limit; the
-// staged operands that are summed over tiles by their largest exponent so far, as V in the forward.
+// Weights: P 2^k and dS times the unit of the staged row enter their products times a running power
+// of two per lane (its key, or query), lowered (and the sums with it) when a weight would pass f16's
+// limit. D is staged in units of its dO row, so that the unit enters P alone: P u (dP / u - D / u).
 struct BwdPairArgs {
   View q, k, v, d_o;
   const float* o;
@@ -746,28 +729,36 @@ struct BwdPairArgs {
   int causal, defer, last, give_up_bh;
 };
 constexpr int kBwdRows = 128;  // rows per workgroup
-constexpr int kPTop = 15;
-constexpr float kDsMax = 61440.0f;  // of a scaled dS
-constexpr int kDsTop = 11;          // where a new scale puts the largest
+constexpr int kDsTop = 11;  // where a new scale puts the largest weight
 
-// The running scale of dS in one lane: raises nothing, lowers `sc` (and the accumulators by the same
-// factor) where a value would exceed kDsMax.
-template <int N>
-__device__ __forceinline__ void fit_scale(const f16v& ds, float& sc, f16v (&acc)[N]) {
+// The running scale of the weights in one lane: raises nothing, lowers `sc` (and the accumulators by
+// the same factor) where a weight would exceed kMaxWeight. First the largest, then the test.
+__device__ __forceinline__ float max_weight(const f16v& x) {
   float m = 0.0f;
 #pragma unroll
   for (int r = 0; r < 16; r += 2) {
-    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(ds[r]), "v"(ds[r + 1]));
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(x[r]), "v"(x[r + 1]));
   }
-  if (__builtin_amdgcn_ballot_w64(m * sc > kDsMax) != 0) {
-    m = pair_max(fmaxf(m, 0.0f));
-    if (m * sc > kDsMax) {
-      const float to = pow2(kDsTop - exponent(m));
-      const float f = to / sc;  // (a power of two, or 0)
-      sc = to;
+  return m;
+}
+template <int N>
+__device__ __forceinline__ void fit_scale(float m, float& sc, f16v (&acc)[N]) {
+  m = pair_max(fmaxf(m, 0.0f));
+  if (m * sc > kMaxWeight) {
+    const float to = pow2(kDsTop - exponent(m));
+    const float f = to / sc;  // (a power of two, or 0)
+    sc = to;
 #pragma unroll
-      for (int i = 0; i < N; ++i) acc[i] *= f;
-    }
+    for (int i = 0; i < N; ++i) acc[i] *= f;
+  }
+}
+// D 128: the sums stay in accumulation registers across a branch that rescales them (the compiler
+// otherwise keeps them, or what they displace, in memory).
+template <int N>
+__device__ __forceinline__ void pin_acc(f16v (&acc)[N]) {
+  if constexpr (N == 4) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm("" : "+a"(acc[i]));
   }
 }
 // k - L log2 e, log2 e in two terms.
@@ -776,10 +767,6 @@ __device__ __forceinline__ float shifted_l(float L, float k) {
   return fmaf(-L, kLog2eLow, fmaf(-L, kLog2e, k));
 }
 __device__ __forceinline__ int half_log2(int s) { return (32 - __builtin_clz(s)) / 2; }
-// A growing exponent of a staged operand: the factor its sums take.
-__device__ __forceinline__ float grown(int from, int to) {
-  return from - to < -126 ? 0.0f : pow2(from - to);
-}
 
 // dK and dV of one key, dQ of one query, in plain fp32 by one wave: lanes take the other side's rows
 // for the products and dims for the sums.
@@ -919,8 +906,7 @@ struct BwdSmem {
     } t[2];
     float o[4][kRows * ((D < 64 ? D : 64) + 4)];
   };
-  Maxima mx;
-  float l[2][kRows], d[2][kRows];
+  float ua[2][kRows], ub[2][kRows], l[2][kRows], d[2][kRows];  // (d over ub)
 };
 
 template <int D, bool kCausal, bool kSerial>
@@ -958,31 +944,25 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
   };
   Pair kB[kKS], vB[kKS];
   float uk, uv;  // 1 / the key's scales
-  int eq[2], eg[2];
   {
     OwnRows<D> ok, ov;
     load(0);
     load_o(0);
     ok.load(a.k.p + b * a.k.sb + h * a.k.sh + min(key, S - 1) * a.k.ss, g);
     ov.load(a.v.p + b * a.v.sb + h * a.v.sh + min(key, S - 1) * a.v.ss, g);
-    st.put_maxima(sm.mx, 1, w, lane);
     uk = ok.split(1.0f, kB);
     uv = ov.split(1.0f, vB);
-    __syncthreads();
-    eq[0] = eq[1] = tile_exponent(sm.mx, 1, 0);
-    eg[0] = eg[1] = tile_exponent(sm.mx, 1, 1);
-    st.store(sm.t[0].a, sm.t[0].b, tile_scale(eq[0]), tile_scale(eg[0]), w, lane);
+    st.store(sm.t[0].a, sm.t[0].b, sm.ua[0], sm.ub[0], w, lane);
     ro.put(st, sm.d[0], w, lane);
     if (w == 0 && g == 0) sm.l[0][j] = shifted_l(lreg, kp);
     load(1);
     load_o(1);
-    st.put_maxima(sm.mx, 0, w, lane);
   }
   f16v dk[kDT], dv[kDT];
 #pragma unroll
   for (int dt = 0; dt < kDT; ++dt) dk[dt] = zero16(), dv[dt] = zero16();
-  int e_k = eq[0], e_v = eg[0];
-  float dsc = pow2(kTop + 100);
+  const float cs = a.scale * kLog2e * uk * pow2(-kTop), cg = uv * pow2(-kTop);
+  float psc = kSerial ? 1.0f : kMaxScale, dsc = kMaxScale;
   int roff[kKS], coff[kDT];
 #pragma unroll
   for (int ks = 0; ks < kKS; ++ks) roff[ks] = row_off<D>(j, g, ks);
@@ -991,25 +971,13 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
 
   auto stage = [&](int u) {  // stores the next step's tile
     const int put = (u + 1) & 1;
-    eq[1] = max(tile_exponent(sm.mx, u & 1, 0), eq[0]);
-    eg[1] = max(tile_exponent(sm.mx, u & 1, 1), eg[0]);
-    st.store(sm.t[put].a, sm.t[put].b, tile_scale(eq[1]), tile_scale(eg[1]), w, lane);
+    st.store(sm.t[put].a, sm.t[put].b, sm.ua[put], sm.ub[put], w, lane);
     ro.put(st, sm.d[put], w, lane);
     if (w == 0 && g == 0) sm.l[put][j] = shifted_l(lreg, kp);
   };
   auto tile = [&](auto fullc, int u) {
     constexpr bool kFull = decltype(fullc)::value != 0;
     const int cur = u & 1, q0 = (t0 + u) * kRows;
-    if (eq[0] > e_k) {
-#pragma unroll
-      for (int dt = 0; dt < kDT; ++dt) dk[dt] *= grown(e_k, eq[0]);
-      e_k = eq[0];
-    }
-    if (eg[0] > e_v) {
-#pragma unroll
-      for (int dt = 0; dt < kDT; ++dt) dv[dt] *= grown(e_v, eg[0]);
-      e_v = eg[0];
-    }
     if (kFull) stage(u);
     const Tile<D>&Q = sm.t[cur].a, &G = sm.t[cur].b;
     f16v s = zero16(), dp = zero16();
@@ -1040,22 +1008,32 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
       load(u + 2);
       pin_loads();
     }
-    const float cs = a.scale * kLog2e * (uk * pow2(eq[0] - kTop)), cg = uv * pow2(eg[0] - kTop);
     // Live: register r's query, q0 + 4 g + 8 i + e, below S and, causal, not before the key.
     const int hi = key < S ? S - q0 - 4 * g : 0, lo = kCausal ? key - q0 - 4 * g : 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const f4 L = ld4(&sm.l[cur][8 * i + 4 * g]), Dv = ld4(&sm.d[cur][8 * i + 4 * g]);
+      const f4 uq = ld4(&sm.ua[cur][8 * i + 4 * g]), ug = ld4(&sm.ub[cur][8 * i + 4 * g]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int r = 4 * i + e;
-        const float x = exp2_hw(fmaf(s[r], cs, L[e]));
+        const float x = exp2_hw(fmaf(s[r], cs * uq[e], L[e])) * ug[e];
         const bool live = kFull || (8 * i + e < hi && !(kCausal && 8 * i + e < lo));
         const float p = live ? x : 0.0f;
-        const float y = p * fmaf(dp[r], cg, -Dv[e]);
+        const float y = p * fmaf(dp[r], cg, -Dv[e]) * uq[e];
         dp[r] = live ? y : 0.0f;
         s[r] = p;
       }
+    }
+    // (Both tests before either product: a second branch over accumulators spills at d 128.)
+    pin_acc(dv);
+    pin_acc(dk);
+    const float mp = kSerial ? 0.0f : max_weight(s), md = max_weight(dp);
+    if (__builtin_amdgcn_ballot_w64(mp * psc > kMaxWeight || md * dsc > kMaxWeight) != 0) {
+      if constexpr (!kSerial) fit_scale(mp, psc, dv);
+      fit_scale(md, dsc, dk);
+      pin_acc(dv);
+      pin_acc(dk);
     }
     if constexpr (kSerial) {
 #pragma unroll
@@ -1070,10 +1048,7 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
         }
       }
     } else {
-      unsigned hh[8], ll[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) split2(s[2 * i], s[2 * i + 1], pow2(kPTop - kp), hh[i], ll[i]);
-      const Pair p0 = make_pair8(hh, ll), p1 = make_pair8(hh + 4, ll + 4);
+      const Pair p0 = split_acc<0>(s, psc), p1 = split_acc<1>(s, psc);
 #pragma unroll
       for (int dt = 0; dt < kDT; ++dt) {
         dv[dt] = mma3(ld_col<D>(G, coff[dt], 0), p0, dv[dt]);
@@ -1084,23 +1059,14 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
       load_o(u + 2);
       pin_loads();
     }
-    fit_scale(dp, dsc, dk);
     {
-      unsigned hh[8], ll[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) split2(dp[2 * i], dp[2 * i + 1], dsc, hh[i], ll[i]);
-      const Pair p0 = make_pair8(hh, ll), p1 = make_pair8(hh + 4, ll + 4);
+      const Pair p0 = split_acc<0>(dp, dsc), p1 = split_acc<1>(dp, dsc);
 #pragma unroll
       for (int dt = 0; dt < kDT; ++dt) {
         dk[dt] = mma3(ld_col<D>(Q, coff[dt], 0), p0, dk[dt]);
         dk[dt] = mma3(ld_col<D>(Q, coff[dt], 1), p1, dk[dt]);
       }
     }
-    if (kFull) st.put_maxima(sm.mx, (u + 1) & 1, w, lane);
-  };
-  auto advance = [&] {
-    __syncthreads();
-    eq[0] = eq[1], eg[0] = eg[1];
   };
   // Steps with no mask: every query and key below S and, causal, past the diagonal. (In the others
   // the staging is outside the branch: in both its arms, the loaded registers and the accumulators
@@ -1112,8 +1078,7 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
     load_o(u + 2);
     pin_loads();
     if (wave_live && !(kCausal && (t0 + u) * kRows + kRows <= kw0)) tile(Const<0>{}, u);
-    st.put_maxima(sm.mx, (u + 1) & 1, w, lane);
-    advance();
+    __syncthreads();
   };
   __syncthreads();
   int u = 0;
@@ -1122,7 +1087,7 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
   }
   for (; u < full1; ++u) {
     tile(Const<1>{}, u);
-    advance();
+    __syncthreads();
   }
   for (; u < nsteps; ++u) masked(u);
   if (!wave_live) return;
@@ -1134,9 +1099,8 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
   }
   const int64_t part = static_cast<int64_t>(a.H) * D;
   float* row = a.dqkv + (static_cast<int64_t>(b) * S + kw0) * 3 * part + static_cast<int64_t>(h) * D;
-  store_rows<D>(dk, pow2(e_k - kTop), fk, sm.o[w], row + part, 3 * part, S - kw0, lane);
-  store_rows<D>(dv, pow2(e_v - kTop), pow2(kSerial ? -kp : -kPTop), sm.o[w], row + 2 * part,
-                3 * part, S - kw0, lane);
+  store_rows<D>(dk, pow2(-kTop), fk, sm.o[w], row + part, 3 * part, S - kw0, lane);
+  store_rows<D>(dv, pow2(-kTop - kp), 1.0f / psc, sm.o[w], row + 2 * part, 3 * part, S - kw0, lane);
 }
 
 template <int D, bool kCausal>
@@ -1169,7 +1133,6 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
   Pair qB[kKS], gB[kKS];
   const int kp = half_log2(S);
   float uq, ug, L, Dq;  // L: kp - L log2 e
-  int ek[2], ev[2];  // K's largest exponent so far, V's own
   {
     OwnRows<D> oq, og, oo;
     const int qc = min(qi, S - 1);
@@ -1178,7 +1141,6 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
     og.load(a.d_o.p + b * a.d_o.sb + h * a.d_o.sh + qc * a.d_o.ss, g);
     oo.load(a.o + ((static_cast<int64_t>(b) * S + qc) * a.H + h) * D, g);
     L = a.lse[static_cast<int64_t>(bh) * S + qc];
-    st.put_maxima(sm.mx, 1, w, lane);
     Dq = 0.0f;
 #pragma unroll
     for (int ks = 0; ks < kKS; ++ks) {
@@ -1191,18 +1153,14 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
     L = shifted_l(L, kp);
     uq = oq.split(1.0f, qB);
     ug = og.split(1.0f, gB);
-    __syncthreads();
-    ek[0] = ek[1] = tile_exponent(sm.mx, 1, 0);
-    ev[0] = ev[1] = tile_exponent(sm.mx, 1, 1);
-    st.store(sm.t[0].a, sm.t[0].b, tile_scale(ek[0]), tile_scale(ev[0]), w, lane);
+    st.store(sm.t[0].a, sm.t[0].b, sm.ua[0], sm.ub[0], w, lane);
     st.load(kop, vop, kRows, S - 1, w, lane);
-    st.put_maxima(sm.mx, 0, w, lane);
   }
   f16v dq[kDT];
 #pragma unroll
   for (int dt = 0; dt < kDT; ++dt) dq[dt] = zero16();
-  int e_q = ek[0];
-  float dsc = pow2(kTop + 100);
+  const float cs = a.scale * kLog2e * uq * pow2(-kTop), cg = ug * pow2(-kTop);
+  float dsc = kMaxScale;
   int roff[kKS], coff[kDT];
 #pragma unroll
   for (int ks = 0; ks < kKS; ++ks) roff[ks] = row_off<D>(j, g, ks);
@@ -1211,9 +1169,7 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
 
   auto stage = [&](int t) {
     const int put = (t + 1) & 1;
-    ek[1] = max(tile_exponent(sm.mx, t & 1, 0), ek[0]);
-    ev[1] = tile_exponent(sm.mx, t & 1, 1);
-    st.store(sm.t[put].a, sm.t[put].b, tile_scale(ek[1]), tile_scale(ev[1]), w, lane);
+    st.store(sm.t[put].a, sm.t[put].b, sm.ua[put], sm.ub[put], w, lane);
   };
   auto load = [&](int t) {
     st.load(kop, vop, (t + 2) * kRows, S - 1, w, lane);
@@ -1222,11 +1178,6 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
   auto tile = [&](auto fullc, int t) {
     constexpr bool kFull = decltype(fullc)::value != 0;
     const int cur = t & 1, kt0 = t * kRows;
-    if (ek[0] > e_q) {
-#pragma unroll
-      for (int dt = 0; dt < kDT; ++dt) dq[dt] *= grown(e_q, ek[0]);
-      e_q = ek[0];
-    }
     stage(t);
     const Tile<D>&K = sm.t[cur].a, &V = sm.t[cur].b;
     f16v s = zero16(), dp = zero16();
@@ -1252,28 +1203,29 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
       for (int ks = 0; ks < kKS; ++ks) dp = mma(x[ks], gB[ks].h, dp);
     }
     load(t);
-    const float cs = a.scale * kLog2e * (uq * pow2(ek[0] - kTop)), cg = ug * pow2(ev[0] - kTop);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int key = kt0 + 8 * (r >> 2) + 4 * g + (r & 3);
-      const float x = exp2_hw(fmaf(s[r], cs, L)) * fmaf(dp[r], cg, -Dq);
-      dp[r] = kFull || (key < S && !(kCausal && key > qi)) ? x : 0.0f;
+    for (int i = 0; i < 4; ++i) {
+      const f4 uk = ld4(&sm.ua[cur][8 * i + 4 * g]), uv = ld4(&sm.ub[cur][8 * i + 4 * g]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = 4 * i + e, key = kt0 + 8 * i + 4 * g + e;
+        const float x =
+            exp2_hw(fmaf(s[r], cs * uk[e], L)) * fmaf(dp[r], cg * uv[e], -Dq) * uk[e];
+        dp[r] = kFull || (key < S && !(kCausal && key > qi)) ? x : 0.0f;
+      }
     }
-    fit_scale(dp, dsc, dq);
-    unsigned hh[8], ll[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) split2(dp[2 * i], dp[2 * i + 1], dsc, hh[i], ll[i]);
-    const Pair p0 = make_pair8(hh, ll), p1 = make_pair8(hh + 4, ll + 4);
+    pin_acc(dq);
+    const float md = max_weight(dp);
+    if (__builtin_amdgcn_ballot_w64(md * dsc > kMaxWeight) != 0) {
+      fit_scale(md, dsc, dq);
+      pin_acc(dq);
+    }
+    const Pair p0 = split_acc<0>(dp, dsc), p1 = split_acc<1>(dp, dsc);
 #pragma unroll
     for (int dt = 0; dt < kDT; ++dt) {
       dq[dt] = mma3(ld_col<D>(K, coff[dt], 0), p0, dq[dt]);
       dq[dt] = mma3(ld_col<D>(K, coff[dt], 1), p1, dq[dt]);
     }
-    st.put_maxima(sm.mx, (t + 1) & 1, w, lane);
-  };
-  auto advance = [&] {
-    __syncthreads();
-    ek[0] = ek[1], ev[0] = ev[1];
   };
   const int full_end = (kCausal ? min(S, qw0 + 1) : S) / kRows;
   const int nfull = wave_live ? min(full_end, ntiles) : 0;
@@ -1281,7 +1233,7 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
   int t = 0;
   for (; t < nfull; ++t) {
     tile(Const<1>{}, t);
-    advance();
+    __syncthreads();
   }
   for (; t < ntiles; ++t) {
     if (wave_live && t * kRows < kw_end) {
@@ -1289,9 +1241,8 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
     } else {
       stage(t);
       load(t);
-      st.put_maxima(sm.mx, (t + 1) & 1, w, lane);
     }
-    advance();
+    __syncthreads();
   }
   // Where dQ goes (uniform): its rows, or the workspace for step 3.
   const bool gave_up = bh == a.give_up_bh;
@@ -1321,7 +1272,7 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
       bwd_query_fp32<D>(a, b, h, qw0 + i, lane, row + i * stride, factor);
     }
   } else {
-    store_rows<D>(dq, pow2(e_q - kTop), un * factor, sm.o[w], row, stride, S - qw0, lane);
+    store_rows<D>(dq, pow2(-kTop), un * factor, sm.o[w], row, stride, S - qw0, lane);
   }
 }
 

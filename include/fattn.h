@@ -29,10 +29,11 @@
  *     `fused_attention_qkv:`);
  *   - empty inputs (batch, heads or seq 0) are a successful no-op (empty outputs);
  *   - operands, sums and results are fp32: the products run on the f16 matrix cores with every
- *     fp32 operand held as the sum of two f16 under a power-of-two scale (22 bits or more of each
- *     value above 2^-17 of the largest of its 32-row tile, below that 2^-39 of that largest), and
- *     are summed in fp32; a 32-row group whose result is not finite is computed again in plain
- *     fp32. Results are bit-identical from run to run.
+ *     fp32 operand held as the sum of two f16 under a power-of-two scale of its row (head_dim
+ *     values: 22 bits or more of each above 2^-17 of the row's largest, below that 2^-39 of it),
+ *     and are summed in fp32. Softmax weights, and dS, times the scale of the row they weigh, are
+ *     held the same way under a scale of the sum they enter. A 32-row group whose result is not
+ *     finite is computed again in plain fp32. Results are bit-identical from run to run.
  */
 #ifndef FATTN_H
 #define FATTN_H
