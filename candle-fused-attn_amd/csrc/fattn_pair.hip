@@ -22,8 +22,8 @@
 // the staged rows, into the weights (P, dS). The weights of a lane's own row follow a power of two
 // of their own, so that they keep 22 bits down to about 2^-17 of the largest term of the sum, and no
 // term's error depends on a row that has no part in it. (One scale per tile, or the largest so far,
-// costs less: forward b64 h6 s240 33.5 us against 35.5, b16 h16 s1024 204 against 231, backward 104
-// against 106 and 787 against 807, d 128 227 against 248. But one large row, masked or not, or one
+// costs less: forward b64 h6 s240 34.6 us against 36.5, b16 h16 s1024 205 against 222, backward 105
+// against 107 and 779 against 798, d 128 229 against 236. But one large row, masked or not, or one
 // key of large weight, takes the bits of all the others.)
 //
 // For one v_mfma_f32_32x32x16_f16, lane l (j = l % 32, g = l / 32) supplies A[j][8 g + e] and
@@ -36,7 +36,7 @@
 // j, in the order above). 16-byte chunk c of row r sits at chunk c ^ chunk_swz(r).
 //
 // Values the split cannot carry (infinities, NaN) show as a non-finite result; a wave that finds
-// one computes its rows again in plain fp32.
+// one computes its 32 rows again on the fp32 matrix instruction.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stddef.h>
@@ -137,27 +137,30 @@ struct Tile {
 template <int D>
 constexpr int kPlane = kRows * D * 2;  // bytes
 
-// Row j = lane % 32's columns 16 ks + 8 g .. + 7.
+// Row j = lane % 32's columns 8 g .. + 7; those of step ks, 16 ks on, at this ^ row_step(ks).
 template <int D>
-__device__ __forceinline__ int row_off(int j, int g, int ks) {
-  return j * (2 * D) + (((2 * ks + g) ^ chunk_swz<D>(j)) << 4);
+__device__ __forceinline__ int row_off(int j, int g) {
+  return j * (2 * D) + ((g ^ chunk_swz<D>(j)) << 4);
 }
+__device__ constexpr int row_step(int ks) { return ks << 5; }
 template <int D>
 __device__ __forceinline__ Pair ld_row(const Tile<D>& t, int off) {
   const char* p = reinterpret_cast<const char*>(&t) + off;
   return Pair{*reinterpret_cast<const h8*>(p), *reinterpret_cast<const h8*>(p + kPlane<D>)};
 }
-// The lane's base offset of the transposed read of columns 32 dt + lane % 32: within each group of
+// The lane's base offset of the transposed read of columns lane % 32 (32 dt + those at this ^
+// col_step(dt)): within each group of
 // 16 lanes, lane i points at row i / 4 and columns 4 (i % 4) .. + 3 of a 4 x 16 block and receives
 // the block's column i. Rows 16 ks + 4 g + (0..3) at + 32 D ks bytes; 8 rows on, + 16 D bytes and
 // the chunk of the offset changed by kSwz8.
 template <int D>
-__device__ __forceinline__ int col_off(int lane, int dt) {
+__device__ __forceinline__ int col_off(int lane) {
   const int i = lane & 15, hi = (lane >> 4) & 1, g = lane >> 5;
   const int row = 4 * g + (i >> 2);
-  const int chunk = 4 * dt + 2 * hi + ((i & 3) >> 1);
+  const int chunk = 2 * hi + ((i & 3) >> 1);
   return row * (2 * D) + ((chunk ^ chunk_swz<D>(row)) << 4) + ((i & 1) << 3);
 }
+__device__ constexpr int col_step(int dt) { return dt << 6; }
 template <int D>
 __device__ __forceinline__ h8 ld_tr(const char* t, int off) {
   typedef __attribute__((address_space(3))) s4 lds_s4;
@@ -202,16 +205,6 @@ __device__ __forceinline__ float group_max(float m) {
   if constexpr (N >= 16) x = max_dpp<0x140>(x);
   return __uint_as_float(x);
 }
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int i = 1; i < 64; i <<= 1) x += __shfl_xor(x, i);
-  return x;
-}
-__device__ __forceinline__ float wave_max(float x) {
-#pragma unroll
-  for (int i = 1; i < 64; i <<= 1) x = fmaxf(x, __shfl_xor(x, i));
-  return x;
-}
 // max(m, |x|, |y|) over eight values: four v_max3_f32 with absolute operands (from fmaxf the
 // compiler makes eight and quiets every input first). For loaded values; NaN is passed over.
 __device__ __forceinline__ float abs_max8(f4 x, f4 y, float m) {
@@ -222,6 +215,12 @@ __device__ __forceinline__ float abs_max8(f4 x, f4 y, float m) {
 // No memory access moves across: a step's loads are issued before its LDS reads (left to itself the
 // compiler sinks them to their first use, at the end of the step).
 __device__ __forceinline__ void pin_loads() { asm volatile("" ::: "memory"); }
+// x, as the compiler finds it here: what is formed from it (a walk's offsets in each step, the
+// addresses used after it) is not formed earlier and held in registers, or memory, until then.
+__device__ __forceinline__ int late(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
 // 0 where every value is finite, else NaN.
 template <int N>
 __device__ __forceinline__ float probe_finite(const f16v (&x)[N], float z) {
@@ -342,6 +341,93 @@ struct OwnRows {
   }
 };
 
+// 32 rows x D of an accumulator (times f f2, per lane), through the wave's part of LDS, to rows of
+// `stride` floats. Two factors: their product may be below the least float, where it is 0 or, as a
+// pow2() out of range, anything, while a sum times it is not.
+template <int D, int N>
+__device__ __forceinline__ void store_rows(const f16v (&acc)[N], float f, float f2, float* so,
+                                           float* base, int64_t stride, int rows, int lane) {
+  constexpr int kCols = D < 64 ? D : 64, kPitch = kCols + 4, kLanes = kCols / 4;
+  const int j = lane & 31, g = lane >> 5;
+#pragma unroll
+  for (int c0 = 0; c0 < D; c0 += kCols) {
+#pragma unroll
+    for (int dt = c0 / 32; dt < (c0 + kCols) / 32; ++dt) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f4 x{acc[dt][4 * i], acc[dt][4 * i + 1], acc[dt][4 * i + 2], acc[dt][4 * i + 3]};
+        st4(so + j * kPitch + 32 * dt - c0 + 8 * i + 4 * g, x * f * f2);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kRows; i += 64 / kLanes) {
+      const int row = i + lane / kLanes, c = 4 * (lane % kLanes);
+      const f4 x = ld4(so + row * kPitch + c);
+      if (row < rows) st4_nt(base + row * stride + c0 + c, x);
+    }
+  }
+}
+// --- Rows in fp32 ------------------------------------------------------------------------------
+// A wave's 32 rows from memory, on v_mfma_f32_32x32x2_f32 and with no part of the workgroup's
+// staging (waves come here alone, past the last barrier). Lane (j, g) supplies A[j][g] and B[g][j]
+// and holds D as above, so a product over columns takes 8 i + 4 g + e in step (i, e), and a sum over
+// staged rows takes row 8 (r / 4) + 4 g + r % 4 in step r, with register r as its B operand. A row
+// that a lane's own row does not see must not meet its weight of 0 there (0 times an infinity): a
+// tile with masked rows sums its live ones row by row, the weights through the wave's part of LDS.
+// With a NaN in V of every head, forward / backward us (one row at a time, lanes over keys, before;
+// clean inputs in brackets): b64 h6 s240 132 / 477 (4186 / 19357; 36 / 106), b16 h16 s1024 1118 / 3939
+// (60518 / 262624; 222 / 798).
+__device__ __forceinline__ f16v mma32(float a, float b, f16v c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+// The tile's row of register r, for the half g.
+__device__ __forceinline__ int tile_row(int r, int g) { return 8 * (r >> 2) + 4 * g + (r & 3); }
+// The products of a tile's row (one per lane j) with the lane's own row.
+template <int D>
+__device__ __forceinline__ f16v dots_fp32(const float* row, const float* own, int g) {
+  f16v c = zero16();
+#pragma clang loop unroll_count(4)
+  for (int i = 4 * g; i < D; i += 8) {
+    const f4 x = ld4(row + i), y = ld4(own + i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c = mma32(x[e], y[e], c);
+  }
+  return c;
+}
+// acc^T += rows^T weights, over the tile's rows r0 .. (register r holds the weight of tile_row(r)).
+// kFull: all 32 are live for every lane. Else those below `end` that live(row) lets through.
+template <int D, bool kFull, typename Live>
+__device__ __forceinline__ void sum_fp32(const f16v& weights, const float* base, int64_t stride,
+                                         int r0, int end, Live live, float* so, f16v (&acc)[D / 32],
+                                         int j, int g) {
+  if constexpr (kFull) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float* row = base + (r0 + tile_row(r, g)) * stride + j;
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt) acc[dt] = mma32(row[32 * dt], weights[r], acc[dt]);
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) so[tile_row(r, g) * 32 + j] = weights[r];
+    const int n = min(kRows, end - r0);
+#pragma clang loop unroll(disable)
+    for (int i = 0; i < n; ++i) {
+      const float w = so[i * 32 + j];
+      const float* row = base + (r0 + i) * stride + 4 * g;
+      if (live(r0 + i)) {
+#pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            acc[dt][r] = fmaf(w, row[32 * dt + 8 * (r >> 2) + (r & 3)], acc[dt][r]);
+          }
+        }
+      }
+    }
+  }
+}
+
 // --- Forward -----------------------------------------------------------------------------------
 // One workgroup = 4 waves of one (b, h), NQ groups of 32 queries per wave; key tiles of 32 keys,
 // split into LDS by all four waves (each value split once per workgroup). Per wave, tile and group:
@@ -364,52 +450,50 @@ constexpr int kWTop = 6;
 constexpr float kMaxWeight = 61440.0f;  // of a scaled weight (f16 ends at 65504)
 constexpr float kMaxScale = 0x1p127f;   // of a running scale, and where it starts
 
-// One query's output row and L in plain fp32 by one wave: lanes take keys for the scores and dims
-// for the output.
-template <int D>
-__device__ void fwd_row_fp32(const FwdArgs& a, int b, int h, int qi, int lane) {
-  const float* qp = a.q.p + b * a.q.sb + h * a.q.sh + static_cast<int64_t>(qi) * a.q.ss;
+// O and L of 32 queries from qg in fp32. `store` takes O's sums and their factor.
+template <int D, bool kCausal, typename Store>
+__device__ __forceinline__ void fwd_rows_fp32(const FwdArgs& a, int b, int h, int qg, float* so,
+                                              int lane, Store store) {
+  const int j = lane & 31, g = lane >> 5, S = a.S, qi = qg + j;
+  const float* qp = a.q.p + b * a.q.sb + h * a.q.sh + min(qi, S - 1) * a.q.ss;
   const float* kp = a.k.p + b * a.k.sb + h * a.k.sh;
   const float* vp = a.v.p + b * a.v.sb + h * a.v.sh;
   const float sign = a.scale < 0.0f ? -1.0f : 1.0f, c2 = fabsf(a.scale) * kLog2e;
-  const int kend = a.causal ? qi + 1 : a.S;
-  constexpr int kND = (D + 63) / 64;
-  float m = kNegInf, l = 0.0f, o[kND] = {};
-  for (int k0 = 0; k0 < kend; k0 += 64) {
-    const int key = k0 + lane;
-    float s = kNegInf;
-    if (key < kend) {
-      const float* kr = kp + static_cast<int64_t>(key) * a.k.ss;
-      s = 0.0f;
-#pragma clang loop unroll(disable)
-      for (int c = 0; c < D; ++c) s = fmaf(sign * qp[c], kr[c], s);
+  f16v acc[D / 32];
+#pragma unroll
+  for (int dt = 0; dt < D / 32; ++dt) acc[dt] = zero16();
+  float m = kNegInf, l = 0.0f;
+  auto tile = [&](auto fullc, int k0) {
+    constexpr bool kFull = decltype(fullc)::value != 0;
+    auto live = [&](int key) { return kFull || (key < S && !(kCausal && key > qi)); };
+    f16v s = dots_fp32<D>(kp + min(k0 + j, S - 1) * a.k.ss, qp, g);
+    float mn = m;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = live(k0 + tile_row(r, g)) ? s[r] * sign : kNegInf;
+      mn = fmaxf(mn, s[r]);
     }
-    const float mn = fmaxf(m, wave_max(s));
+    mn = pair_max(fmaxf(mn, kNegInf));
     const float alpha = mn == m ? 1.0f : m == kNegInf ? 0.0f : exp2_hw((m - mn) * c2);
-    const float p = s == kNegInf ? 0.0f : exp2_hw(fmaf(s, c2, -(mn * c2)));
     m = mn;
-    l = l * alpha + wave_sum(p);
+    l *= alpha;
 #pragma unroll
-    for (int i = 0; i < kND; ++i) o[i] *= alpha;
-    const int n = min(64, kend - k0);
-#pragma clang loop unroll(disable)
-    for (int kk = 0; kk < n; ++kk) {
-      const float pk = __shfl(p, kk);
-      const float* vr = vp + static_cast<int64_t>(k0 + kk) * a.v.ss;
+    for (int dt = 0; dt < D / 32; ++dt) acc[dt] *= alpha;
 #pragma unroll
-      for (int i = 0; i < kND; ++i) {
-        const int c = 64 * i + lane;
-        if (c < D) o[i] = fmaf(pk, vr[c], o[i]);
-      }
+    for (int r = 0; r < 16; ++r) {
+      s[r] = s[r] == kNegInf ? 0.0f : exp2_hw(fmaf(s[r], c2, -(mn * c2)));
+      l += s[r];
     }
-  }
-#pragma unroll
-  for (int i = 0; i < kND; ++i) {
-    const int c = 64 * i + lane;
-    if (c < D) a.o[((static_cast<int64_t>(b) * a.S + qi) * a.H + h) * D + c] = o[i] / l;
-  }
-  if (lane == 0) {
-    a.lse[(static_cast<int64_t>(b) * a.H + h) * a.S + qi] = m * fabsf(a.scale) + logf(l);
+    sum_fp32<D, kFull>(s, vp, a.v.ss, k0, S, live, so, acc, j, g);
+  };
+  const int kend = kCausal ? min(S, qg + kRows) : S;
+  int k0 = 0;
+  for (; k0 + kRows <= (kCausal ? min(S, qg + 1) : S); k0 += kRows) tile(Const<1>{}, k0);
+  for (; k0 < kend; k0 += kRows) tile(Const<0>{}, k0);
+  l = pair_sum(l);
+  store(acc, 1.0f / l);
+  if (g == 0 && qi < S) {
+    a.lse[(static_cast<int64_t>(b) * a.H + h) * S + qi] = m * fabsf(a.scale) + logf(l);
   }
 }
 
@@ -489,11 +573,7 @@ fwd_pair_kernel(FwdArgs a) {
 #pragma unroll
     for (int dt = 0; dt < kDT; ++dt) acc[n][dt] = zero16();
   }
-  int roff[kKS], coff[kDT];
-#pragma unroll
-  for (int ks = 0; ks < kKS; ++ks) roff[ks] = row_off<D>(j, g, ks);
-#pragma unroll
-  for (int dt = 0; dt < kDT; ++dt) coff[dt] = col_off<D>(lane, dt);
+  const int roff0 = row_off<D>(j, g), coff0 = col_off<D>(lane);
 
   // Stores tile t + 1 (loaded in the last step) and issues the loads of tile t + 2.
   auto stage = [&](int t) {
@@ -506,7 +586,7 @@ fwd_pair_kernel(FwdArgs a) {
   // one and nothing reads: tested for, the loaded registers would live across the whole step.)
   auto tile = [&](auto fullc, int t) {
     constexpr bool kFull = decltype(fullc)::value != 0;
-    const int kt0 = t * kRows;
+    const int roff = late(roff0), coff = late(coff0), kt0 = t * kRows;
     const Kv& cur = sm.t.kv[t & 1];
     stage(t);
     f16v s[NQ];
@@ -516,7 +596,7 @@ fwd_pair_kernel(FwdArgs a) {
       for (int n = 0; n < NQ; ++n) s[n] = zero16();
 #pragma unroll
       for (int ks = 0; ks < kKS; ++ks) {
-        const Pair k = ld_row<D>(cur.k, roff[ks]);
+        const Pair k = ld_row<D>(cur.k, roff ^ row_step(ks));
         kh[ks] = k.h;
 #pragma unroll
         for (int n = 0; n < NQ; ++n) s[n] = mma_small(k, q[n][ks], s[n]);
@@ -600,11 +680,11 @@ fwd_pair_kernel(FwdArgs a) {
     const bool second = kFull || kt0 + 16 < kw_end;  // wave-uniform: the last 16 keys are live
 #pragma unroll
     for (int dt = 0; dt < kDT; ++dt) {
-      const Pair v0 = ld_col<D>(cur.v, coff[dt], 0);
+      const Pair v0 = ld_col<D>(cur.v, coff ^ col_step(dt), 0);
 #pragma unroll
       for (int n = 0; n < NQ; ++n) acc[n][dt] = mma3(v0, p[n][0], acc[n][dt]);
       if (second) {
-        const Pair v1 = ld_col<D>(cur.v, coff[dt], 1);
+        const Pair v1 = ld_col<D>(cur.v, coff ^ col_step(dt), 1);
 #pragma unroll
         for (int n = 0; n < NQ; ++n) acc[n][dt] = mma3(v1, p[n][1], acc[n][dt]);
       }
@@ -641,36 +721,22 @@ fwd_pair_kernel(FwdArgs a) {
     const int qg = qw0 + kRows * n, qi = qg + j;
     if (qg >= S) break;
     const float l = pair_sum(lsum[n]);
-    if (__builtin_amdgcn_ballot_w64(qi < S && !(probe_finite<kDT>(acc[n], l * 0.0f) == 0.0f)) !=
-        0) {
-      for (int i = 0; i < kRows && qg + i < S; ++i) fwd_row_fp32<D>(a, b, h, qg + i, lane);
-      continue;
-    }
     // O through LDS (the wave's own part; every wave is past its last tile), so that each row is
     // written as whole 128-byte lines.
-    const float inv = 1.0f / l, unit = pow2(-kTop) / wsc[n];  // (apart: the product may be subnormal)
     float* so = sm.t.o[w];
-#pragma unroll
-    for (int c0 = 0; c0 < D; c0 += kOCols) {
-#pragma unroll
-      for (int dt = c0 / 32; dt < (c0 + kOCols) / 32; ++dt) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const f4 x{acc[n][dt][4 * i], acc[n][dt][4 * i + 1], acc[n][dt][4 * i + 2],
-                     acc[n][dt][4 * i + 3]};
-          st4(so + j * kOPitch + 32 * dt - c0 + 8 * i + 4 * g, x * inv * unit);
-        }
-      }
-      constexpr int kLanes = kOCols / 4;  // lanes per row
-#pragma unroll
-      for (int i = 0; i < kRows; i += 64 / kLanes) {
-        const int row = i + lane / kLanes, c = 4 * (lane % kLanes);
-        const f4 x = ld4(so + row * kOPitch + c);
-        if (qg + row < S) {
-          st4_nt(a.o + ((static_cast<int64_t>(b) * S + qg + row) * a.H + h) * D + c0 + c, x);
-        }
-      }
+    const int lane_e = late(lane);
+    auto store = [&](const f16v (&x)[kDT], float f, float f2) {
+      store_rows<D>(x, f, f2, so, a.o + ((static_cast<int64_t>(b) * S + qg) * a.H + h) * D,
+                    static_cast<int64_t>(a.H) * D, S - qg, lane_e);
+    };
+    if (__builtin_amdgcn_ballot_w64(qi < S && !(probe_finite<kDT>(acc[n], l * 0.0f) == 0.0f)) !=
+        0) {
+      fwd_rows_fp32<D, kCausal>(a, b, h, qg, so, late(lane),
+                                [&](const f16v (&x)[kDT], float inv) { store(x, inv, 1.0f); });
+      continue;
     }
+    // (Two factors: their product may be subnormal.)
+    store(acc[n], 1.0f / l, pow2(-kTop) / wsc[n]);
     if (g == 0 && qi < S) {
       int le = exponent(l);
       float f = l * pow2(-le);  // [1, 2), then [0.75, 1.5)
@@ -768,135 +834,88 @@ __device__ __forceinline__ float shifted_l(float L, float k) {
 }
 __device__ __forceinline__ int half_log2(int s) { return (32 - __builtin_clz(s)) / 2; }
 
-// dK and dV of one key, dQ of one query, in plain fp32 by one wave: lanes take the other side's rows
-// for the products and dims for the sums.
-template <int D>
-__device__ void bwd_key_fp32(const BwdPairArgs& a, int b, int h, int key, int lane) {
-  const float* kr = a.k.p + b * a.k.sb + h * a.k.sh + static_cast<int64_t>(key) * a.k.ss;
-  const float* vr = a.v.p + b * a.v.sb + h * a.v.sh + static_cast<int64_t>(key) * a.v.ss;
+// dK and dV of 32 keys from kw0, dQ of 32 queries from qw0, in fp32 (without the scale).
+template <int D, bool kCausal>
+__device__ __forceinline__ void bwd_keys_fp32(const BwdPairArgs& a, int b, int h, int kw0, float* so,
+                                              f16v (&dk)[D / 32], f16v (&dv)[D / 32], int lane) {
+  const int j = lane & 31, g = lane >> 5, S = a.S, key = kw0 + j;
+  const float* kr = a.k.p + b * a.k.sb + h * a.k.sh + min(key, S - 1) * a.k.ss;
+  const float* vr = a.v.p + b * a.v.sb + h * a.v.sh + min(key, S - 1) * a.v.ss;
   const float* qp = a.q.p + b * a.q.sb + h * a.q.sh;
   const float* gp = a.d_o.p + b * a.d_o.sb + h * a.d_o.sh;
-  const float* op = a.o + (static_cast<int64_t>(b) * a.S * a.H + h) * D;
-  const float* lp = a.lse + (static_cast<int64_t>(b) * a.H + h) * a.S;
-  constexpr int kND = (D + 63) / 64;
-  float dk[kND] = {}, dv[kND] = {};
-  for (int q0 = a.causal ? key : 0; q0 < a.S; q0 += 64) {
-    const int qi = q0 + lane;
-    float p = 0.0f, ds = 0.0f;
-    if (qi < a.S) {
-      const float* qr = qp + static_cast<int64_t>(qi) * a.q.ss;
-      const float* gr = gp + static_cast<int64_t>(qi) * a.d_o.ss;
-      const float* orow = op + static_cast<int64_t>(qi) * a.H * D;
-      float s = 0.0f, t = 0.0f, dd = 0.0f;
-#pragma clang loop unroll(disable)
-      for (int c = 0; c < D; ++c) {
-        s = fmaf(qr[c], kr[c], s);
-        t = fmaf(gr[c], vr[c], t);
-        dd = fmaf(gr[c], orow[c], dd);
-      }
-      p = exp2_hw(fmaf(s, a.scale, -lp[qi]) * kLog2e);
-      ds = p * (t - dd);
-    }
-    const int n = min(64, a.S - q0);
-#pragma clang loop unroll(disable)
-    for (int i = 0; i < n; ++i) {
-      const float pi = __shfl(p, i), di = __shfl(ds, i);
-      const float* qr = qp + static_cast<int64_t>(q0 + i) * a.q.ss;
-      const float* gr = gp + static_cast<int64_t>(q0 + i) * a.d_o.ss;
+  const float* op = a.o + (static_cast<int64_t>(b) * S * a.H + h) * D;
+  const float* lp = a.lse + (static_cast<int64_t>(b) * a.H + h) * S;
 #pragma unroll
-      for (int e = 0; e < kND; ++e) {
-        const int c = 64 * e + lane;
-        if (c < D) {
-          dv[e] = fmaf(pi, gr[c], dv[e]);
-          dk[e] = fmaf(di, qr[c], dk[e]);
-        }
-      }
-    }
-  }
-  float* row = a.dqkv + (static_cast<int64_t>(b) * a.S + key) * 3 * a.H * D +
-               static_cast<int64_t>(h) * D;
+  for (int dt = 0; dt < D / 32; ++dt) dk[dt] = zero16(), dv[dt] = zero16();
+  auto tile = [&](auto fullc, int q0) {
+    constexpr bool kFull = decltype(fullc)::value != 0;
+    auto live = [&](int qi) { return kFull || (qi < S && !(kCausal && qi < key)); };
+    const int64_t qr = min(q0 + j, S - 1);
+    f16v s = dots_fp32<D>(qp + qr * a.q.ss, kr, g), dp = dots_fp32<D>(gp + qr * a.d_o.ss, vr, g);
+    float dd = 0.0f;
+#pragma clang loop unroll(disable)
+    for (int c = 4 * g; c < D; c += 8) {
+      const f4 x = ld4(gp + qr * a.d_o.ss + c), y = ld4(op + qr * a.H * D + c);
 #pragma unroll
-  for (int e = 0; e < kND; ++e) {
-    const int c = 64 * e + lane;
-    if (c < D) {
-      row[static_cast<int64_t>(a.H) * D + c] = dk[e] * a.scale;
-      row[static_cast<int64_t>(2) * a.H * D + c] = dv[e];
+      for (int e = 0; e < 4; ++e) dd = fmaf(x[e], y[e], dd);
     }
-  }
+    dd = pair_sum(dd);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int t = tile_row(r, g), qi = min(q0 + t, S - 1);
+      const float p = exp2_hw(fmaf(s[r], a.scale, -lp[qi]) * kLog2e);
+      const float y = p * (dp[r] - __shfl(dd, t));  // (every lane takes part in the shuffle)
+      s[r] = live(q0 + t) ? p : 0.0f;
+      dp[r] = live(q0 + t) ? y : 0.0f;
+    }
+    sum_fp32<D, kFull>(s, gp, a.d_o.ss, q0, S, live, so, dv, j, g);
+    sum_fp32<D, kFull>(dp, qp, a.q.ss, q0, S, live, so, dk, j, g);
+  };
+  int q0 = kCausal ? kw0 : 0;
+  if (kCausal) tile(Const<0>{}, q0), q0 += kRows;
+  for (; q0 + kRows <= S; q0 += kRows) tile(Const<1>{}, q0);
+  if (q0 < S) tile(Const<0>{}, q0);
 }
-template <int D>
-__device__ void bwd_query_fp32(const BwdPairArgs& a, int b, int h, int qi, int lane, float* row,
-                               float factor) {
-  const float* qr = a.q.p + b * a.q.sb + h * a.q.sh + static_cast<int64_t>(qi) * a.q.ss;
-  const float* gr = a.d_o.p + b * a.d_o.sb + h * a.d_o.sh + static_cast<int64_t>(qi) * a.d_o.ss;
+template <int D, bool kCausal>
+__device__ __forceinline__ void bwd_queries_fp32(const BwdPairArgs& a, int b, int h, int qw0,
+                                                 float* so, f16v (&dq)[D / 32], int lane) {
+  const int j = lane & 31, g = lane >> 5, S = a.S, qi = qw0 + j;
+  const int64_t qc = min(qi, S - 1);
+  const float* qr = a.q.p + b * a.q.sb + h * a.q.sh + qc * a.q.ss;
+  const float* gr = a.d_o.p + b * a.d_o.sb + h * a.d_o.sh + qc * a.d_o.ss;
   const float* kp = a.k.p + b * a.k.sb + h * a.k.sh;
   const float* vp = a.v.p + b * a.v.sb + h * a.v.sh;
-  const float* orow = a.o + ((static_cast<int64_t>(b) * a.S + qi) * a.H + h) * D;
-  const float L = a.lse[(static_cast<int64_t>(b) * a.H + h) * a.S + qi];
-  constexpr int kND = (D + 63) / 64;
-  float dq[kND] = {}, dd = 0.0f;
+  const float* orow = a.o + ((static_cast<int64_t>(b) * S + qc) * a.H + h) * D;
+  const float L = a.lse[(static_cast<int64_t>(b) * a.H + h) * S + qc];
+  float dd = 0.0f;
 #pragma clang loop unroll(disable)
-  for (int c = 0; c < D; ++c) dd = fmaf(gr[c], orow[c], dd);
-  const int kend = a.causal ? qi + 1 : a.S;
-  for (int k0 = 0; k0 < kend; k0 += 64) {
-    const int key = k0 + lane;
-    float ds = 0.0f;
-    if (key < kend) {
-      const float* kr = kp + static_cast<int64_t>(key) * a.k.ss;
-      const float* vr = vp + static_cast<int64_t>(key) * a.v.ss;
-      float s = 0.0f, t = 0.0f;
-#pragma clang loop unroll(disable)
-      for (int c = 0; c < D; ++c) {
-        s = fmaf(qr[c], kr[c], s);
-        t = fmaf(gr[c], vr[c], t);
-      }
-      ds = exp2_hw(fmaf(s, a.scale, -L) * kLog2e) * (t - dd);
-    }
-    const int n = min(64, kend - k0);
-#pragma clang loop unroll(disable)
-    for (int i = 0; i < n; ++i) {
-      const float di = __shfl(ds, i);
-      const float* kr = kp + static_cast<int64_t>(k0 + i) * a.k.ss;
+  for (int c = 4 * g; c < D; c += 8) {
+    const f4 x = ld4(gr + c), y = ld4(orow + c);
 #pragma unroll
-      for (int e = 0; e < kND; ++e) {
-        const int c = 64 * e + lane;
-        if (c < D) dq[e] = fmaf(di, kr[c], dq[e]);
-      }
-    }
+    for (int e = 0; e < 4; ++e) dd = fmaf(x[e], y[e], dd);
   }
+  dd = pair_sum(dd);
 #pragma unroll
-  for (int e = 0; e < kND; ++e) {
-    const int c = 64 * e + lane;
-    if (c < D) row[c] = dq[e] * factor;
-  }
+  for (int dt = 0; dt < D / 32; ++dt) dq[dt] = zero16();
+  auto tile = [&](auto fullc, int k0) {
+    constexpr bool kFull = decltype(fullc)::value != 0;
+    auto live = [&](int key) { return kFull || (key < S && !(kCausal && key > qi)); };
+    const int64_t kr = min(k0 + j, S - 1);
+    const f16v s = dots_fp32<D>(kp + kr * a.k.ss, qr, g);
+    f16v dp = dots_fp32<D>(vp + kr * a.v.ss, gr, g);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float x = exp2_hw(fmaf(s[r], a.scale, -L) * kLog2e) * (dp[r] - dd);
+      dp[r] = live(k0 + tile_row(r, g)) ? x : 0.0f;
+    }
+    sum_fp32<D, kFull>(dp, kp, a.k.ss, k0, S, live, so, dq, j, g);
+  };
+  const int kend = kCausal ? min(S, qw0 + kRows) : S;
+  int k0 = 0;
+  for (; k0 + kRows <= (kCausal ? min(S, qw0 + 1) : S); k0 += kRows) tile(Const<1>{}, k0);
+  for (; k0 < kend; k0 += kRows) tile(Const<0>{}, k0);
 }
 
-// 32 rows x D of an accumulator (times f f2, per lane), through the wave's part of LDS, to rows of
-// `stride` floats. Two factors: their product may be below the least float, where it is 0 or, as a
-// pow2() out of range, anything, while a sum times it is not.
-template <int D, int N>
-__device__ __forceinline__ void store_rows(const f16v (&acc)[N], float f, float f2, float* so,
-                                           float* base, int64_t stride, int rows, int lane) {
-  constexpr int kCols = D < 64 ? D : 64, kPitch = kCols + 4, kLanes = kCols / 4;
-  const int j = lane & 31, g = lane >> 5;
-#pragma unroll
-  for (int c0 = 0; c0 < D; c0 += kCols) {
-#pragma unroll
-    for (int dt = c0 / 32; dt < (c0 + kCols) / 32; ++dt) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const f4 x{acc[dt][4 * i], acc[dt][4 * i + 1], acc[dt][4 * i + 2], acc[dt][4 * i + 3]};
-        st4(so + j * kPitch + 32 * dt - c0 + 8 * i + 4 * g, x * f * f2);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < kRows; i += 64 / kLanes) {
-      const int row = i + lane / kLanes, c = 4 * (lane % kLanes);
-      const f4 x = ld4(so + row * kPitch + c);
-      if (row < rows) st4_nt(base + row * stride + c0 + c, x);
-    }
-  }
-}
 // LDS of a backward workgroup.
 template <int D>
 struct BwdSmem {
@@ -963,11 +982,7 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
   for (int dt = 0; dt < kDT; ++dt) dk[dt] = zero16(), dv[dt] = zero16();
   const float cs = a.scale * kLog2e * uk * pow2(-kTop), cg = uv * pow2(-kTop);
   float psc = kSerial ? 1.0f : kMaxScale, dsc = kMaxScale;
-  int roff[kKS], coff[kDT];
-#pragma unroll
-  for (int ks = 0; ks < kKS; ++ks) roff[ks] = row_off<D>(j, g, ks);
-#pragma unroll
-  for (int dt = 0; dt < kDT; ++dt) coff[dt] = col_off<D>(lane, dt);
+  const int roff0 = row_off<D>(j, g), coff0 = col_off<D>(lane);
 
   auto stage = [&](int u) {  // stores the next step's tile
     const int put = (u + 1) & 1;
@@ -977,7 +992,7 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
   };
   auto tile = [&](auto fullc, int u) {
     constexpr bool kFull = decltype(fullc)::value != 0;
-    const int cur = u & 1, q0 = (t0 + u) * kRows;
+    const int roff = late(roff0), coff = late(coff0), cur = u & 1, q0 = (t0 + u) * kRows;
     if (kFull) stage(u);
     const Tile<D>&Q = sm.t[cur].a, &G = sm.t[cur].b;
     f16v s = zero16(), dp = zero16();
@@ -985,7 +1000,7 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
       h8 x[kKS];
 #pragma unroll
       for (int ks = 0; ks < kKS; ++ks) {
-        const Pair q = ld_row<D>(Q, roff[ks]);
+        const Pair q = ld_row<D>(Q, roff ^ row_step(ks));
         x[ks] = q.h;
         // (The forward's order: its A operand is this B.)
         s = mma(q.l, kB[ks].h, s);
@@ -995,7 +1010,7 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
       for (int ks = 0; ks < kKS; ++ks) s = mma(x[ks], kB[ks].h, s);
 #pragma unroll
       for (int ks = 0; ks < kKS; ++ks) {
-        const Pair y = ld_row<D>(G, roff[ks]);
+        const Pair y = ld_row<D>(G, roff ^ row_step(ks));
         x[ks] = y.h;
         dp = mma_small(y, vB[ks], dp);
       }
@@ -1038,21 +1053,20 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
     if constexpr (kSerial) {
 #pragma unroll
       for (int dt = 0; dt < kDT; ++dt) {
-        const Pair g0 = ld_col<D>(G, coff[dt], 0), g1 = ld_col<D>(G, coff[dt], 1);
+        const Pair g0 = ld_col<D>(G, coff ^ col_step(dt), 0), g1 = ld_col<D>(G, coff ^ col_step(dt), 1);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const Pair& y = r < 8 ? g0 : g1;
-          dv[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-              static_cast<float>(y.h[r % 8]) + static_cast<float>(y.l[r % 8]), s[r], dv[dt], 0, 0,
-              0);
+          dv[dt] = mma32(static_cast<float>(y.h[r % 8]) + static_cast<float>(y.l[r % 8]), s[r],
+                         dv[dt]);
         }
       }
     } else {
       const Pair p0 = split_acc<0>(s, psc), p1 = split_acc<1>(s, psc);
 #pragma unroll
       for (int dt = 0; dt < kDT; ++dt) {
-        dv[dt] = mma3(ld_col<D>(G, coff[dt], 0), p0, dv[dt]);
-        dv[dt] = mma3(ld_col<D>(G, coff[dt], 1), p1, dv[dt]);
+        dv[dt] = mma3(ld_col<D>(G, coff ^ col_step(dt), 0), p0, dv[dt]);
+        dv[dt] = mma3(ld_col<D>(G, coff ^ col_step(dt), 1), p1, dv[dt]);
       }
     }
     if (kFull) {
@@ -1063,8 +1077,8 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
       const Pair p0 = split_acc<0>(dp, dsc), p1 = split_acc<1>(dp, dsc);
 #pragma unroll
       for (int dt = 0; dt < kDT; ++dt) {
-        dk[dt] = mma3(ld_col<D>(Q, coff[dt], 0), p0, dk[dt]);
-        dk[dt] = mma3(ld_col<D>(Q, coff[dt], 1), p1, dk[dt]);
+        dk[dt] = mma3(ld_col<D>(Q, coff ^ col_step(dt), 0), p0, dk[dt]);
+        dk[dt] = mma3(ld_col<D>(Q, coff ^ col_step(dt), 1), p1, dk[dt]);
       }
     }
   };
@@ -1091,16 +1105,18 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
   }
   for (; u < nsteps; ++u) masked(u);
   if (!wave_live) return;
-  const float fk = pow2(-kp) / dsc * a.scale;
-  const float z = probe_finite<kDT>(dk, probe_finite<kDT>(dv, fk * 0.0f));
+  // The two factors of dK and of dV.
+  float fk = pow2(-kTop), fk2 = pow2(-kp) / dsc * a.scale, fv = pow2(-kTop - kp), fv2 = 1.0f / psc;
+  const float z = probe_finite<kDT>(dk, probe_finite<kDT>(dv, fk2 * 0.0f));
   if (__builtin_amdgcn_ballot_w64(key < S && !(z == 0.0f)) != 0) {
-    for (int i = 0; i < kRows && kw0 + i < S; ++i) bwd_key_fp32<D>(a, b, h, kw0 + i, lane);
-    return;
+    bwd_keys_fp32<D, kCausal>(a, b, h, kw0, sm.o[w], dk, dv, late(lane));
+    fk = a.scale, fk2 = fv = fv2 = 1.0f;
   }
   const int64_t part = static_cast<int64_t>(a.H) * D;
   float* row = a.dqkv + (static_cast<int64_t>(b) * S + kw0) * 3 * part + static_cast<int64_t>(h) * D;
-  store_rows<D>(dk, pow2(-kTop), fk, sm.o[w], row + part, 3 * part, S - kw0, lane);
-  store_rows<D>(dv, pow2(-kTop - kp), 1.0f / psc, sm.o[w], row + 2 * part, 3 * part, S - kw0, lane);
+  const int lane_e = late(lane);
+  store_rows<D>(dk, fk, fk2, sm.o[w], row + part, 3 * part, S - kw0, lane_e);
+  store_rows<D>(dv, fv, fv2, sm.o[w], row + 2 * part, 3 * part, S - kw0, lane_e);
 }
 
 template <int D, bool kCausal>
@@ -1161,11 +1177,7 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
   for (int dt = 0; dt < kDT; ++dt) dq[dt] = zero16();
   const float cs = a.scale * kLog2e * uq * pow2(-kTop), cg = ug * pow2(-kTop);
   float dsc = kMaxScale;
-  int roff[kKS], coff[kDT];
-#pragma unroll
-  for (int ks = 0; ks < kKS; ++ks) roff[ks] = row_off<D>(j, g, ks);
-#pragma unroll
-  for (int dt = 0; dt < kDT; ++dt) coff[dt] = col_off<D>(lane, dt);
+  const int roff0 = row_off<D>(j, g), coff0 = col_off<D>(lane);
 
   auto stage = [&](int t) {
     const int put = (t + 1) & 1;
@@ -1177,7 +1189,7 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
   };
   auto tile = [&](auto fullc, int t) {
     constexpr bool kFull = decltype(fullc)::value != 0;
-    const int cur = t & 1, kt0 = t * kRows;
+    const int roff = late(roff0), coff = late(coff0), cur = t & 1, kt0 = t * kRows;
     stage(t);
     const Tile<D>&K = sm.t[cur].a, &V = sm.t[cur].b;
     f16v s = zero16(), dp = zero16();
@@ -1185,7 +1197,7 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
       h8 x[kKS];
 #pragma unroll
       for (int ks = 0; ks < kKS; ++ks) {
-        const Pair k = ld_row<D>(K, roff[ks]);
+        const Pair k = ld_row<D>(K, roff ^ row_step(ks));
         x[ks] = k.h;
         s = mma_small(k, qB[ks], s);
       }
@@ -1193,7 +1205,7 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
       for (int ks = 0; ks < kKS; ++ks) s = mma(x[ks], qB[ks].h, s);
 #pragma unroll
       for (int ks = 0; ks < kKS; ++ks) {
-        const Pair v = ld_row<D>(V, roff[ks]);
+        const Pair v = ld_row<D>(V, roff ^ row_step(ks));
         x[ks] = v.h;
         // (The key blocks' order: their A operand is this B.)
         dp = mma(v.l, gB[ks].h, dp);
@@ -1223,8 +1235,8 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
     const Pair p0 = split_acc<0>(dp, dsc), p1 = split_acc<1>(dp, dsc);
 #pragma unroll
     for (int dt = 0; dt < kDT; ++dt) {
-      dq[dt] = mma3(ld_col<D>(K, coff[dt], 0), p0, dq[dt]);
-      dq[dt] = mma3(ld_col<D>(K, coff[dt], 1), p1, dq[dt]);
+      dq[dt] = mma3(ld_col<D>(K, coff ^ col_step(dt), 0), p0, dq[dt]);
+      dq[dt] = mma3(ld_col<D>(K, coff ^ col_step(dt), 1), p1, dq[dt]);
     }
   };
   const int full_end = (kCausal ? min(S, qw0 + 1) : S) / kRows;
@@ -1258,22 +1270,19 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
                             static_cast<int64_t>(h) * D
                       : a.part + (static_cast<int64_t>(bh) * ntile16 * kBwdQueryTile + qw0) * D;
   const float factor = direct ? a.scale : 1.0f;
-  const float un = pow2(-kp) / dsc;
-  const bool bad = __builtin_amdgcn_ballot_w64(
-                       qi < S && !(probe_finite<kDT>(dq, un * 0.0f) == 0.0f)) != 0;
+  float f = pow2(-kTop), f2 = pow2(-kp) / dsc * factor;
   if (gave_up && direct) {
     // (The test hook, as a wait that ran out would: NaN and the guard word.)
     if (lane == 0) {
       __hip_atomic_store(a.ctrl + kCtrlGuard, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    store_rows<D>(dq, __builtin_nanf(""), 1.0f, sm.o[w], row, stride, S - qw0, lane);
-  } else if (bad) {
-    for (int i = 0; i < kRows && qw0 + i < S; ++i) {
-      bwd_query_fp32<D>(a, b, h, qw0 + i, lane, row + i * stride, factor);
-    }
-  } else {
-    store_rows<D>(dq, pow2(-kTop), un * factor, sm.o[w], row, stride, S - qw0, lane);
+    f = __builtin_nanf("");
+  } else if (__builtin_amdgcn_ballot_w64(
+                 qi < S && !(probe_finite<kDT>(dq, f2 * 0.0f) == 0.0f)) != 0) {
+    bwd_queries_fp32<D, kCausal>(a, b, h, qw0, sm.o[w], dq, late(lane));
+    f = factor, f2 = 1.0f;
   }
+  store_rows<D>(dq, f, f2, sm.o[w], row, stride, S - qw0, late(lane));
 }
 
 template <int D, bool kCausal, bool kSerial, int WAVES>

@@ -263,3 +263,31 @@ def test_tiny_magnitudes(cuda, f, causal):
     for name, a, w in zip(("dq", "dk", "dv"), got, want[1:]):
         check(name, a, w)
     check("o", forward(q, k, v * f, 0.125, causal), reference(q, k, v * f, 0.125, causal)[0])
+
+
+@pytest.mark.parametrize("s", [64, 150, 333])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_causal_non_finite_stays_in_its_rows(cuda, d, s):
+    """Causal, a NaN or infinity in one row: the rows that do not see it are those of the same call
+    with that row zero; queries and keys next to it in its tile among them."""
+    at, scale = s // 2 + 3, 0.125
+    x = [normal(180 + i, 1, s, d) for i in range(4)]
+    before, after = slice(0, at), slice(at + 1, s)
+    # (The infinite V reaches O, hence D, of every query from `at` on, but no P: dV stays whole.)
+    unaffected = {"k": {"o": before, "dq": before}, "v": {"o": before, "dq": before, "dv": slice(0, s)},
+                  "q": {"o": before, "dq": before, "dk": after, "dv": after},
+                  "dO": {"dq": before, "dk": after, "dv": after}}
+    for (name, rows), which, bad in zip(unaffected.items(), (1, 2, 0, 3),
+                                        (math.nan, math.inf, math.inf, -math.inf)):
+        y, z = [t.clone() for t in x], [t.clone() for t in x]
+        y[which][0, at, 3] = bad
+        z[which][0, at] = 0
+        want = dict(zip(("o", "dq", "dk", "dv"), reference(*z[:3], scale, True, z[3])))
+        got = dict(zip(("o", "dq", "dk", "dv"), [forward(*y[:3], scale, True),
+                                                 *gradients(*y, scale, True)]))
+        if name == "v":
+            want["dv"] = reference(*x[:3], scale, True, x[3])[3]
+        for out, r in rows.items():
+            e = rel(got[out][:, r], want[out][:, r])
+            print(f"{name} s{s} d{d} {out}: {e:.2e}", flush=True)
+            assert e <= REL_TOL, (name, out)
