@@ -1329,14 +1329,17 @@ const void* bwd_pair_fn(int causal, bool serial) {
 int launch_forward(View q, View k, View v, float* o, float* lse, int b, int h, int s, int d,
                    float scale, int causal, void* stream) {
   // 64 queries per wave (256 per workgroup) halve what a query pays for reading, splitting and
-  // waiting for the key tiles, but hold 2 waves per SIMD instead of 3 (D 64) and halve the
-  // workgroups: taken where they make two rounds of the two a CU holds and every workgroup walks
-  // all keys. Measured, 64 against 32 queries per wave: D 64, b 16 h 16 s 1024 (1024 workgroups)
-  // 194 against 223 us, b 64 h 6 s 240 (384) 33.6 against 30.2; causal b 8 h 12 s 2048 180 against
-  // 176; D 32, b 16 h 16 s 1024 127 against 134, b 64 h 6 s 240 19.9 against 18.1. At D 128 their
-  // registers do not fit.
+  // waiting for the key tiles, but hold 2 waves per SIMD instead of 3 (D 64; 3 instead of 4 at D 32)
+  // and halve the workgroups. Taken where every workgroup walks all keys, 1024 of them keep every CU
+  // busy for two rounds or more, and no more than an eighth of their queries is padding that 128 per
+  // workgroup would not have. Measured, 64 against 32 queries per wave, us: D 64, b h 256 s 1024
+  // (1024 workgroups) 224 / 247, 512 x 512 121 / 131, 1024 x 256 77 / 83; too few, 64 x 1280 (320)
+  // 119 / 108, 256 x 256 26 / 23; padded, 1024 x 300 140 / 121, 1024 x 640 425 / 419, and below s 128
+  // half of it is (1536 x 32: 29 / 17). D 32, 256 x 1024 145 / 150, 512 x 512 81 / 81, but 1024 x 200
+  // 46 / 43: from s 257 on. At D 128 their registers do not fit.
   const int64_t wide = static_cast<int64_t>((s + 255) / 256) * b * h;
-  const int nq = d != 128 && !causal && wide >= 1024 ? 2 : 1;
+  const bool filled = 8 * 2 * ((s + 255) / 256) <= 9 * ((s + 127) / 128) && (d == 64 || s > 256);
+  const int nq = d != 128 && !causal && wide >= 1024 && filled ? 2 : 1;
   const int qb = 128 * nq, nqb = (s + qb - 1) / qb;
   FwdArgs a{q, k, v, o, lse, b, h, s, nqb, scale, causal ? 1 : 0};
   void* args[] = {&a};

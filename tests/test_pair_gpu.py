@@ -74,6 +74,21 @@ def test_forward_wide_workgroups(cuda, s, d):
         assert e <= REL_TOL
 
 
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("n,s", [(1536, 32), (1024, 128), (1024, 129), (1024, 250), (511, 512),
+                                 (512, 511), (512, 385), (512, 384), (205, 1153), (205, 1152)])
+def test_forward_query_groups_rule(cuda, n, s, d):
+    """One or two groups of 32 queries per wave, on either side of each condition of the choice (256
+    queries per workgroup: how many of them, how many of their queries are padding)."""
+    q, k, v = (normal(19 * s + i, n, s, d) for i in range(3))
+    o = forward(q, k, v, 0.125, False)
+    for i in (0, n // 2 + 1, n - 1):
+        at = slice(i, i + 1)
+        e = rel(o[at], reference(q[at], k[at], v[at], 0.125, False)[0])
+        print(f"{n} x s{s} d{d} pair {i}: {e:.2e}", flush=True)
+        assert e <= REL_TOL
+
+
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("qs,ks,vs,grow", [(1e-9, 1e9, 1e-12, 0), (1e6, 1e-7, 1e15, 0),
                                            (1.0, 1.0, 1e-3, 3), (1.0, 1.0, 1e3, -3)])
