@@ -233,31 +233,34 @@ __device__ __forceinline__ float probe_finite(const f16v (&x)[N], float z) {
 }
 
 // --- Staging -----------------------------------------------------------------------------------
-// Two operands' tiles of 32 rows through the registers of a workgroup of four waves: wave w takes
-// rows 8 w .. 8 w + 7 of both (D 32: operand a in lanes 0..31, b in the others), eight columns per
-// lane and access. A tile is loaded in one step of the walk; the next step takes each row's largest
+// Two operands' tiles of 32 rows through the registers of a workgroup of W waves: wave w takes rows
+// 32 / W w .. of both (D 32 with four waves: operand a in lanes 0..31, b in the others), eight
+// columns per lane and access. A tile is loaded in one step of the walk; the next step takes each row's largest
 // magnitude (over the lanes that hold the row), scales, splits and stores it.
 struct Operand {
   const char* p;  // row 0 of the (b, h)
   unsigned ss4;   // row stride in bytes
 };
-template <int D>
+template <int D, int W>
 struct Stage {
-  static constexpr int kC = D / 8;                // chunks per row
-  static constexpr int kN = D == 32 ? 1 : D / 32;  // accesses per lane: a's, then b's
+  static constexpr int kC = D / 8;             // chunks per row
+  static constexpr int kWaveRows = kRows / W;
+  static constexpr bool kHalves = kWaveRows * kC == 32;  // one access holds both operands
+  static constexpr int kPer = kHalves ? 1 : kWaveRows * kC / 64;  // accesses per lane and operand
+  static constexpr int kN = kHalves ? 1 : 2 * kPer;               // in all: a's, then b's
   f4 x[kN][2];
   int e[kN];  // the access's row's exponent (after store)
 
   static __device__ __forceinline__ int row(int i, int w, int lane) {
-    if constexpr (D == 32) return 8 * w + (lane & 31) / kC;
-    return 8 * w + (64 / kC) * (i % (kN / 2)) + lane / kC;
+    if constexpr (kHalves) return kWaveRows * w + (lane & 31) / kC;
+    return kWaveRows * w + (64 / kC) * (i % kPer) + lane / kC;
   }
   // Rows past `last` repeat it (finite where the operand is; masked by the reader).
   __device__ __forceinline__ void load(const Operand& a, const Operand& b, int r0, int last, int w,
                                        int lane) {
 #pragma unroll
     for (int i = 0; i < kN; ++i) {
-      const bool is_b = kN == 1 ? lane >= 32 : i >= kN / 2;
+      const bool is_b = kHalves ? lane >= 32 : i >= kPer;
       const unsigned r = static_cast<unsigned>(min(r0 + row(i, w, lane), last));
       const char* p = is_b ? b.p : a.p;
       const unsigned off =
@@ -271,7 +274,7 @@ struct Stage {
                                         int lane) {
 #pragma unroll
     for (int i = 0; i < kN; ++i) {
-      const bool is_b = kN == 1 ? lane >= 32 : i >= kN / 2;
+      const bool is_b = kHalves ? lane >= 32 : i >= kPer;
       const int r = row(i, w, lane);
       e[i] = exponent(group_max<kC>(abs_max8(x[i][0], x[i][1], 0.0f)));
       if (lane % kC == 0) (is_b ? ub : ua)[r] = pow2(e[i]);
@@ -286,24 +289,25 @@ struct Stage {
 // Beside a Stage whose operand b is dO: O's rows in the same lanes, and D = rowsum(dO o O) of the
 // tile's 32 rows, in units of dO's rows. O's offsets are in elements: its rows of one (b, h) may span more than 4 GiB (the
 // views' may not).
-template <int D>
+template <int D, int W>
 struct RowDots {
-  static constexpr int kC = D / 8, kN = D == 128 ? 2 : 1;
+  using S = Stage<D, W>;
+  static constexpr int kC = S::kC, kN = S::kPer;
   f4 x[kN][2];
   __device__ __forceinline__ void load(const float* o, unsigned ss, int r0, int last, int w,
                                        int lane) {
 #pragma unroll
     for (int i = 0; i < kN; ++i) {
-      const unsigned r = static_cast<unsigned>(min(r0 + Stage<D>::row(i, w, lane), last));
+      const unsigned r = static_cast<unsigned>(min(r0 + S::row(i, w, lane), last));
       const unsigned off = r * ss + 8u * static_cast<unsigned>(lane % kC);
       x[i][0] = ld4(o + off);
       x[i][1] = ld4(o + off + 4);
     }
   }
-  __device__ __forceinline__ void put(const Stage<D>& st, float* dst, int w, int lane) const {
+  __device__ __forceinline__ void put(const S& st, float* dst, int w, int lane) const {
 #pragma unroll
     for (int i = 0; i < kN; ++i) {
-      const f4(&y)[2] = st.x[Stage<D>::kN / 2 + i];
+      const f4(&y)[2] = st.x[S::kN / 2 + i];
       float t = x[i][0][0] * y[0][0];
 #pragma unroll
       for (int e = 1; e < 8; ++e) t = fmaf(x[i][e / 4][e % 4], y[e / 4][e % 4], t);
@@ -311,8 +315,8 @@ struct RowDots {
       t += dpp<0x4E>(t);
       if constexpr (D >= 64) t += dpp<0x141>(t);
       if constexpr (D == 128) t += dpp<0x140>(t);
-      if (lane % kC == 0 && (D != 32 || lane >= 32)) {
-        dst[Stage<D>::row(i, w, lane)] = t * pow2(-st.e[Stage<D>::kN / 2 + i]);
+      if (lane % kC == 0 && (!S::kHalves || lane >= 32)) {
+        dst[S::row(i, w, lane)] = t * pow2(-st.e[S::kN / 2 + i]);
       }
     }
   }
@@ -429,13 +433,13 @@ __device__ __forceinline__ void sum_fp32(const f16v& weights, const float* base,
 }
 
 // --- Forward -----------------------------------------------------------------------------------
-// One workgroup = 4 waves of one (b, h), NQ groups of 32 queries per wave; key tiles of 32 keys,
-// split into LDS by all four waves (each value split once per workgroup). Per wave, tile and group:
+// One workgroup = W waves of one (b, h), NQ groups of 32 queries per wave; key tiles of 32 keys,
+// split into LDS by all its waves (each value split once per workgroup). Per wave, tile and group:
 //   S^T = K Q^T (A = K rows, B = Q in registers): lane (j, g), register r holds the score of query
 //   j and key 8 (r / 4) + 4 g + r % 4, so a query's online softmax is one lane's and lane ^ 32's;
 //   O^T += V^T P^T (A = V transposed, B = P from S^T's registers).
 // Two LDS buffers, one barrier per tile: a step works on tile t, stores tile t + 1 and loads tile
-// t + 2.
+// t + 2. (Fewer than four waves have at most one tile each, and all are staged before the walk.)
 // The softmax: p = 2^(s c2 - m), c2 = |scale| log2 e and the two rows' scales, m a reference that is
 // kRefTop below the largest score seen when it was set. p is computed with the m in hand and its
 // row sum is what is tested: only where it exceeds kRowTop (or m is not set yet) is the tile's
@@ -497,25 +501,24 @@ __device__ __forceinline__ void fwd_rows_fp32(const FwdArgs& a, int b, int h, in
   }
 }
 
-template <int D, bool kCausal, int NQ, int WAVES>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))
+template <int D, bool kCausal, int NQ, int W, int WAVES>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))
 fwd_pair_kernel(FwdArgs a) {
   a.causal = kCausal ? 1 : 0;
   constexpr int kKS = D / 16;              // contraction steps of S
   constexpr int kDT = D / 32;              // 32-dim tiles of O
-  constexpr int kOCols = D < 64 ? D : 64;  // columns per pass of the output's transpose
-  constexpr int kOPitch = kOCols + 4;
-  constexpr int kWaveQ = kRows * NQ, kQ = 4 * kWaveQ;
+  constexpr int kOPitch = (D < 64 ? D : 64) + 4;  // store_rows'
+  constexpr int kWaveQ = kRows * NQ, kQ = W * kWaveQ, kBufs = W == 1 ? 1 : 2;
   struct Kv {
     Tile<D> k, v;
   };
   union Tiles {
-    Kv kv[2];
-    float o[4][kRows * kOPitch];
+    Kv kv[kBufs];
+    float o[W][kRows * kOPitch];
   };
   struct Smem {
     Tiles t;
-    float uk[2][kRows], uv[2][kRows];
+    float uk[kBufs][kRows], uv[kBufs][kRows];
   };
   __shared__ __attribute__((aligned(16))) Smem sm;
 
@@ -546,7 +549,7 @@ fwd_pair_kernel(FwdArgs a) {
 
   // The first tile, the wave's queries (negated for a negative scale, so that the raw scores' max
   // is the scaled scores'), and the second tile's loads.
-  Stage<D> st;
+  Stage<D, W> st;
   Pair q[NQ][kKS];
   float cq[NQ];  // |scale| log2 e over the scales of the query and kTop
   {
@@ -555,12 +558,13 @@ fwd_pair_kernel(FwdArgs a) {
 #pragma unroll
     for (int n = 0; n < NQ; ++n) own[n].load(qp + min(qw0 + kRows * n + j, S - 1) * a.q.ss, g);
     st.store(sm.t.kv[0].k, sm.t.kv[0].v, sm.uk[0], sm.uv[0], w, lane);
-    st.load(kop, vop, kRows, S - 1, w, lane);
+    if (W > 1) st.load(kop, vop, kRows, S - 1, w, lane);
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
       cq[n] = own[n].split(a.scale < 0.0f ? -1.0f : 1.0f, q[n]) *
               (fabsf(a.scale) * kLog2e * pow2(-kTop));
     }
+    if constexpr (W == 2) st.store(sm.t.kv[1].k, sm.t.kv[1].v, sm.uk[1], sm.uv[1], w, lane);
   }
 
   f16v acc[NQ][kDT];  // O^T, in units of p / wsc and 2^-kTop
@@ -577,6 +581,7 @@ fwd_pair_kernel(FwdArgs a) {
 
   // Stores tile t + 1 (loaded in the last step) and issues the loads of tile t + 2.
   auto stage = [&](int t) {
+    if (W != 4) return;
     const int put = (t + 1) & 1;
     st.store(sm.t.kv[put].k, sm.t.kv[put].v, sm.uk[put], sm.uv[put], w, lane);
     st.load(kop, vop, (t + 2) * kRows, S - 1, w, lane);
@@ -586,8 +591,8 @@ fwd_pair_kernel(FwdArgs a) {
   // one and nothing reads: tested for, the loaded registers would live across the whole step.)
   auto tile = [&](auto fullc, int t) {
     constexpr bool kFull = decltype(fullc)::value != 0;
-    const int roff = late(roff0), coff = late(coff0), kt0 = t * kRows;
-    const Kv& cur = sm.t.kv[t & 1];
+    const int roff = late(roff0), coff = late(coff0), kt0 = t * kRows, cur = W == 1 ? 0 : t & 1;
+    const Kv& kv = sm.t.kv[cur];
     stage(t);
     f16v s[NQ];
     {
@@ -596,7 +601,7 @@ fwd_pair_kernel(FwdArgs a) {
       for (int n = 0; n < NQ; ++n) s[n] = zero16();
 #pragma unroll
       for (int ks = 0; ks < kKS; ++ks) {
-        const Pair k = ld_row<D>(cur.k, roff ^ row_step(ks));
+        const Pair k = ld_row<D>(kv.k, roff ^ row_step(ks));
         kh[ks] = k.h;
 #pragma unroll
         for (int n = 0; n < NQ; ++n) s[n] = mma_small(k, q[n][ks], s[n]);
@@ -625,7 +630,7 @@ fwd_pair_kernel(FwdArgs a) {
         asm("" : "+v"(r0));  // (the units are read again the second time, not held)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const f4 uk = ld4(&sm.uk[t & 1][8 * i + r0]), uv = ld4(&sm.uv[t & 1][8 * i + r0]);
+          const f4 uk = ld4(&sm.uk[cur][8 * i + r0]), uv = ld4(&sm.uv[cur][8 * i + r0]);
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
             const int r = 4 * i + c;
@@ -645,7 +650,7 @@ fwd_pair_kernel(FwdArgs a) {
         asm("" : "+v"(r0));
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const float x = s[n][r] * (cq[n] * sm.uk[t & 1][8 * (r >> 2) + r0 + (r & 3)]);
+          const float x = s[n][r] * (cq[n] * sm.uk[cur][8 * (r >> 2) + r0 + (r & 3)]);
           tmax = fmaxf(tmax, live(r) ? x : kNegInf);
         }
         // (-inf: a row with no live key.)
@@ -680,11 +685,11 @@ fwd_pair_kernel(FwdArgs a) {
     const bool second = kFull || kt0 + 16 < kw_end;  // wave-uniform: the last 16 keys are live
 #pragma unroll
     for (int dt = 0; dt < kDT; ++dt) {
-      const Pair v0 = ld_col<D>(cur.v, coff ^ col_step(dt), 0);
+      const Pair v0 = ld_col<D>(kv.v, coff ^ col_step(dt), 0);
 #pragma unroll
       for (int n = 0; n < NQ; ++n) acc[n][dt] = mma3(v0, p[n][0], acc[n][dt]);
       if (second) {
-        const Pair v1 = ld_col<D>(cur.v, coff ^ col_step(dt), 1);
+        const Pair v1 = ld_col<D>(kv.v, coff ^ col_step(dt), 1);
 #pragma unroll
         for (int n = 0; n < NQ; ++n) acc[n][dt] = mma3(v1, p[n][1], acc[n][dt]);
       }
@@ -748,10 +753,11 @@ fwd_pair_kernel(FwdArgs a) {
 }
 
 // --- Backward ----------------------------------------------------------------------------------
-// One launch of two kinds of workgroup, four waves x 32 rows each, which share no sum, so that no
+// One launch of two kinds of workgroup, W waves x 32 rows each, which share no sum, so that no
 // workgroup waits for another and the results depend on nothing but the shape:
-//   key blocks of 128 keys walk 32-query tiles and hold dK, dV (S, dP, dV, dK: four products);
-//   query blocks of 128 queries walk 32-key tiles and hold dQ (S, dP, dQ: three products).
+//   key blocks (of 128 keys with four waves) walk 32-query tiles and hold dK, dV (S, dP, dV, dK: four
+//   products);
+//   query blocks walk 32-key tiles and hold dQ (S, dP, dQ: three products).
 // S and dP are computed in both: seven products where one kind of workgroup would need five, but
 // then dQ's partial sums (4 s^2 b h bytes) would go through memory and dS through LDS, between
 // barriers. Backward, against that scheme on the fp32 matrix instruction (five products): b64 h6 s240
@@ -790,11 +796,10 @@ struct BwdPairArgs {
   unsigned long long* epoch_slot;
   unsigned long long epoch;
   int* ctrl;
-  int B, H, S, nkv, nblk;  // nkv: key blocks in the grid; nblk: blocks of 128 rows per (b, h)
+  int B, H, S, nkv, nblk;  // nkv: key blocks in the grid; nblk: blocks of 32 W rows per (b, h)
   float scale;
   int causal, defer, last, give_up_bh;
 };
-constexpr int kBwdRows = 128;  // rows per workgroup
 constexpr int kDsTop = 11;  // where a new scale puts the largest weight
 
 // The running scale of the weights in one lane: raises nothing, lowers `sc` (and the accumulators by
@@ -917,29 +922,26 @@ __device__ __forceinline__ void bwd_queries_fp32(const BwdPairArgs& a, int b, in
 }
 
 // LDS of a backward workgroup.
-template <int D>
+template <int D, int W>
 struct BwdSmem {
+  static constexpr int kBufs = W == 1 ? 1 : 2;  // (one wave has at most one tile, two have two)
   union {
     struct {
       Tile<D> a, b;
-    } t[2];
-    float o[4][kRows * ((D < 64 ? D : 64) + 4)];
+    } t[kBufs];
+    float o[W][kRows * ((D < 64 ? D : 64) + 4)];
   };
-  float ua[2][kRows], ub[2][kRows], l[2][kRows], d[2][kRows];  // (d over ub)
+  float ua[kBufs][kRows], ub[kBufs][kRows], l[kBufs][kRows], d[kBufs][kRows];  // (d over ub)
 };
 
-template <int D, bool kCausal, bool kSerial>
-__device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, int id) {
+template <int D, bool kCausal, bool kSerial, int W>
+__device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D, W>& sm, int item) {
   constexpr int kKS = D / 16, kDT = D / 32;
   const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, g = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int S = a.S, BH = a.B * a.H;
-  // Causal: the low blocks (they see every later query) first.
-  const int item = kCausal ? id : xcd_remap(id, a.nkv);
-  const int bh = kCausal ? item % BH : item / a.nblk;
-  const int kb = kCausal ? item / BH : item % a.nblk;
+  const int S = a.S, bh = item / a.nblk, kb = item % a.nblk;
   const int b = bh / a.H, h = bh % a.H;
-  const int k0 = kb * kBwdRows, kw0 = k0 + w * kRows, key = kw0 + j;
+  const int k0 = kb * (W * kRows), kw0 = k0 + w * kRows, key = kw0 + j;
   const bool wave_live = kw0 < S;
   const Operand qop{reinterpret_cast<const char*>(a.q.p + b * a.q.sb + h * a.q.sh),
                     static_cast<unsigned>(a.q.ss) * 4u};
@@ -947,19 +949,24 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
                     static_cast<unsigned>(a.d_o.ss) * 4u};
   const float* op = a.o + (static_cast<int64_t>(b) * S * a.H + h) * D;
   const float* lp = a.lse + static_cast<int64_t>(bh) * S;
-  // The walk: step u takes tile t0 + u (causal: from the block's diagonal, four tiles, on).
+  // The walk: step u takes tile t0 + u (causal: from the block's diagonal, W tiles, on).
   const int ntiles = (S + kRows - 1) / kRows, t0 = kCausal ? k0 / kRows : 0;
   const int nsteps = ntiles - t0;
 
   const int kp = half_log2(S);
-  Stage<D> st;
-  RowDots<D> ro;
+  Stage<D, W> st;
+  RowDots<D, W> ro;
   float lreg;
   auto load = [&](int u) { st.load(qop, gop, (t0 + u) * kRows, S - 1, w, lane); };
   auto load_o = [&](int u) {
     const int r0 = (t0 + u) * kRows;
     ro.load(op, static_cast<unsigned>(a.H) * D, r0, S - 1, w, lane);
     lreg = lp[min(r0 + j, S - 1)];
+  };
+  auto store = [&](int put) {
+    st.store(sm.t[put].a, sm.t[put].b, sm.ua[put], sm.ub[put], w, lane);
+    ro.put(st, sm.d[put], w, lane);
+    if (w == 0 && g == 0) sm.l[put][j] = shifted_l(lreg, kp);
   };
   Pair kB[kKS], vB[kKS];
   float uk, uv;  // 1 / the key's scales
@@ -971,11 +978,12 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
     ov.load(a.v.p + b * a.v.sb + h * a.v.sh + min(key, S - 1) * a.v.ss, g);
     uk = ok.split(1.0f, kB);
     uv = ov.split(1.0f, vB);
-    st.store(sm.t[0].a, sm.t[0].b, sm.ua[0], sm.ub[0], w, lane);
-    ro.put(st, sm.d[0], w, lane);
-    if (w == 0 && g == 0) sm.l[0][j] = shifted_l(lreg, kp);
-    load(1);
-    load_o(1);
+    store(0);
+    if (W > 1) {
+      load(1);
+      load_o(1);
+    }
+    if (W == 2) store(1);
   }
   f16v dk[kDT], dv[kDT];
 #pragma unroll
@@ -984,16 +992,13 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
   float psc = kSerial ? 1.0f : kMaxScale, dsc = kMaxScale;
   const int roff0 = row_off<D>(j, g), coff0 = col_off<D>(lane);
 
-  auto stage = [&](int u) {  // stores the next step's tile
-    const int put = (u + 1) & 1;
-    st.store(sm.t[put].a, sm.t[put].b, sm.ua[put], sm.ub[put], w, lane);
-    ro.put(st, sm.d[put], w, lane);
-    if (w == 0 && g == 0) sm.l[put][j] = shifted_l(lreg, kp);
-  };
+  // The next step's tile, and the loads of the one after it (four waves; fewer have at most two
+  // tiles, and both are staged).
+  constexpr bool kWalk = W == 4;
   auto tile = [&](auto fullc, int u) {
     constexpr bool kFull = decltype(fullc)::value != 0;
-    const int roff = late(roff0), coff = late(coff0), cur = u & 1, q0 = (t0 + u) * kRows;
-    if (kFull) stage(u);
+    const int roff = late(roff0), coff = late(coff0), cur = W == 1 ? 0 : u & 1, q0 = (t0 + u) * kRows;
+    if (kFull && kWalk) store((u + 1) & 1);
     const Tile<D>&Q = sm.t[cur].a, &G = sm.t[cur].b;
     f16v s = zero16(), dp = zero16();
     {
@@ -1019,7 +1024,7 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
     }
     // The loads of the step after next from here on (its O later still): held across the products
     // above as well, they do not fit.
-    if (kFull) {
+    if (kFull && kWalk) {
       load(u + 2);
       pin_loads();
     }
@@ -1069,7 +1074,7 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
         dv[dt] = mma3(ld_col<D>(G, coff ^ col_step(dt), 1), p1, dv[dt]);
       }
     }
-    if (kFull) {
+    if (kFull && kWalk) {
       load_o(u + 2);
       pin_loads();
     }
@@ -1087,17 +1092,19 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
   // spill where they join.)
   const int full1 = kw0 + kRows <= S ? S / kRows - t0 : 0;
   auto masked = [&](int u) {
-    stage(u);
-    load(u + 2);
-    load_o(u + 2);
-    pin_loads();
+    if (kWalk) {
+      store((u + 1) & 1);
+      load(u + 2);
+      load_o(u + 2);
+      pin_loads();
+    }
     if (wave_live && !(kCausal && (t0 + u) * kRows + kRows <= kw0)) tile(Const<0>{}, u);
     __syncthreads();
   };
   __syncthreads();
   int u = 0;
   if (kCausal) {
-    for (; u < min(4, nsteps); ++u) masked(u);
+    for (; u < min(W, nsteps); ++u) masked(u);
   }
   for (; u < full1; ++u) {
     tile(Const<1>{}, u);
@@ -1119,33 +1126,24 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D>& sm, i
   store_rows<D>(dv, fv, fv2, sm.o[w], row + 2 * part, 3 * part, S - kw0, lane_e);
 }
 
-template <int D, bool kCausal>
-__device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm, int id) {
+template <int D, bool kCausal, int W>
+__device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D, W>& sm, int item) {
   constexpr int kKS = D / 16, kDT = D / 32;
   const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, g = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int S = a.S, BH = a.B * a.H;
-  int qb, bh;
-  if (kCausal) {
-    qb = a.nblk - 1 - id / BH;
-    bh = id % BH;
-  } else {
-    const int item = xcd_remap(id, a.nblk * BH);
-    qb = item % a.nblk;
-    bh = item / a.nblk;
-  }
+  const int S = a.S, bh = item / a.nblk, qb = item % a.nblk;
   const int b = bh / a.H, h = bh % a.H;
-  const int q0 = qb * kBwdRows, qw0 = q0 + w * kRows, qi = qw0 + j;
+  const int q0 = qb * (W * kRows), qw0 = q0 + w * kRows, qi = qw0 + j;
   const bool wave_live = qw0 < S;
   const Operand kop{reinterpret_cast<const char*>(a.k.p + b * a.k.sb + h * a.k.sh),
                     static_cast<unsigned>(a.k.ss) * 4u};
   const Operand vop{reinterpret_cast<const char*>(a.v.p + b * a.v.sb + h * a.v.sh),
                     static_cast<unsigned>(a.v.ss) * 4u};
-  const int k_end = kCausal ? min(S, q0 + kBwdRows) : S;
+  const int k_end = kCausal ? min(S, q0 + W * kRows) : S;
   const int ntiles = (k_end + kRows - 1) / kRows;
   const int kw_end = kCausal ? min(S, qw0 + kRows) : S;
 
-  Stage<D> st;
+  Stage<D, W> st;
   Pair qB[kKS], gB[kKS];
   const int kp = half_log2(S);
   float uq, ug, L, Dq;  // L: kp - L log2 e
@@ -1170,7 +1168,8 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
     uq = oq.split(1.0f, qB);
     ug = og.split(1.0f, gB);
     st.store(sm.t[0].a, sm.t[0].b, sm.ua[0], sm.ub[0], w, lane);
-    st.load(kop, vop, kRows, S - 1, w, lane);
+    if (W > 1) st.load(kop, vop, kRows, S - 1, w, lane);
+    if constexpr (W == 2) st.store(sm.t[1].a, sm.t[1].b, sm.ua[1], sm.ub[1], w, lane);
   }
   f16v dq[kDT];
 #pragma unroll
@@ -1179,17 +1178,19 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
   float dsc = kMaxScale;
   const int roff0 = row_off<D>(j, g), coff0 = col_off<D>(lane);
 
-  auto stage = [&](int t) {
+  auto stage = [&](int t) {  // (four waves, as above)
+    if (W != 4) return;
     const int put = (t + 1) & 1;
     st.store(sm.t[put].a, sm.t[put].b, sm.ua[put], sm.ub[put], w, lane);
   };
   auto load = [&](int t) {
+    if (W != 4) return;
     st.load(kop, vop, (t + 2) * kRows, S - 1, w, lane);
     pin_loads();
   };
   auto tile = [&](auto fullc, int t) {
     constexpr bool kFull = decltype(fullc)::value != 0;
-    const int roff = late(roff0), coff = late(coff0), cur = t & 1, kt0 = t * kRows;
+    const int roff = late(roff0), coff = late(coff0), cur = W == 1 ? 0 : t & 1, kt0 = t * kRows;
     stage(t);
     const Tile<D>&K = sm.t[cur].a, &V = sm.t[cur].b;
     f16v s = zero16(), dp = zero16();
@@ -1260,7 +1261,7 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
   const bool gave_up = bh == a.give_up_bh;
   const bool direct = a.part == nullptr || !(a.defer || (gave_up && !a.last));
   const int ntile16 = (S + kBwdQueryTile - 1) / kBwdQueryTile;
-  if (a.done != nullptr && direct && tid < kBwdRows / kBwdQueryTile) {
+  if (a.done != nullptr && direct && tid < W * kRows / kBwdQueryTile) {
     const int j16 = q0 / kBwdQueryTile + tid;
     if (j16 < ntile16) a.done[static_cast<int64_t>(bh) * ntile16 + j16] = a.epoch;
   }
@@ -1285,27 +1286,60 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D>& sm
   store_rows<D>(dq, f, f2, sm.o[w], row, stride, S - qw0, late(lane));
 }
 
-template <int D, bool kCausal, bool kSerial, int WAVES>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))
+template <int D, bool kCausal, bool kSerial, int W, int WAVES>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))
 bwd_pair_kernel(BwdPairArgs a) {
   a.causal = kCausal ? 1 : 0;
-  __shared__ __attribute__((aligned(16))) BwdSmem<D> sm;
-  const int id = static_cast<int>(blockIdx.x);
+  __shared__ __attribute__((aligned(16))) BwdSmem<D, W> sm;
+  const int id = static_cast<int>(blockIdx.x), BH = a.B * a.H;
   if (id == 0 && threadIdx.x == 0) {
     __hip_atomic_store(a.ctrl + kCtrlGuard, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (a.epoch_slot != nullptr) *a.epoch_slot = a.epoch;
   }
-  if (id < a.nkv) {
-    bwd_keys<D, kCausal, kSerial>(a, sm, id);
+  if (W < 4) {
+    // One workgroup of each kind per (b, h): side by side on one XCD, so that what both read comes
+    // from memory once.
+    const int item = xcd_remap(id, 2 * a.nkv);
+    if (item & 1) {
+      bwd_queries<D, kCausal, W>(a, sm, item >> 1);
+    } else {
+      bwd_keys<D, kCausal, kSerial, W>(a, sm, item >> 1);
+    }
+  } else if (id < a.nkv) {
+    // Causal: the low blocks (they see every later query) first.
+    bwd_keys<D, kCausal, kSerial, W>(a, sm, kCausal ? id % BH * a.nblk + id / BH : xcd_remap(id, a.nkv));
   } else {
-    bwd_queries<D, kCausal>(a, sm, id - a.nkv);
+    const int i = id - a.nkv;
+    bwd_queries<D, kCausal, W>(a, sm, kCausal ? i % BH * a.nblk + a.nblk - 1 - i / BH : xcd_remap(i, a.nkv));
   }
 }
 
-template <int D, int NQ, int WAVES>
-const void* fwd_pair_fn(int causal) {
-  return causal ? reinterpret_cast<const void*>(fwd_pair_kernel<D, true, NQ, WAVES>)
-                : reinterpret_cast<const void*>(fwd_pair_kernel<D, false, NQ, WAVES>);
+template <int D, int WAVES>
+const void* fwd_pair_fn(int causal, int waves) {
+  auto fn = [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    constexpr int kOcc = W == 2 && D == 64 ? 2 : WAVES;  // (two waves share two tiles' LDS)
+    return causal ? reinterpret_cast<const void*>(fwd_pair_kernel<D, true, 1, W, kOcc>)
+                  : reinterpret_cast<const void*>(fwd_pair_kernel<D, false, 1, W, kOcc>);
+  };
+  if constexpr (D != 128) {
+    if (waves == 2) return fn(Const<2>{});
+  }
+  return waves == 1 ? fn(Const<1>{}) : fn(Const<4>{});
+}
+
+// Waves per workgroup, each of 32 rows. Four share the staging of a tile, but over a short sequence
+// those past its end only stage and wait, and the tiles ahead of the walk are staged for nothing:
+// where there are workgroups enough for every CU without them, one wave takes s <= 32 and two
+// s <= 64, with every tile staged before the walk (and, backward, the two kinds of workgroup of one
+// (b, h) side by side). Fewer waves against four, us, 1536 (b, h), forward / backward: D 64, s 16
+// 9.5 / 18 (16.0 / 41), s 32 11.5 / 22 (17.0 / 47), s 64 22.8 / 47 (24.4 / 66), causal s 64 25.3 / 49
+// (25.2 / 72); D 128 s 32 27 / 56 (31 / 148), s 64 backward 122 (209), forward 46 (44: four);
+// D 32 s 64 13.4 / 27 (15.9 / 39). With 64 (b, h), where the time is one workgroup's: D 64 s 64
+// 8.1 / 11.4 (7.2 / 10.1), D 128 s 32 9.2 / 14.1 (8.1 / 13.4).
+int workgroup_waves(int bh, int s, bool two) {
+  if (bh <= 256 || s > 64) return 4;
+  return s <= 32 ? 1 : two ? 2 : 4;
 }
 
 // Causal, up to this many key blocks: dV summed over the queries one at a time, on the fp32 matrix
@@ -1318,10 +1352,14 @@ const void* fwd_pair_fn(int causal) {
 // sum.
 constexpr int kSerialBlocks = 64;
 template <int D, int WAVES>
-const void* bwd_pair_fn(int causal, bool serial) {
-  return !causal  ? reinterpret_cast<const void*>(bwd_pair_kernel<D, false, false, WAVES>)
-         : serial ? reinterpret_cast<const void*>(bwd_pair_kernel<D, true, true, WAVES>)
-                  : reinterpret_cast<const void*>(bwd_pair_kernel<D, true, false, WAVES>);
+const void* bwd_pair_fn(int causal, bool serial, int waves) {
+  auto fn = [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    return !causal  ? reinterpret_cast<const void*>(bwd_pair_kernel<D, false, false, W, WAVES>)
+           : serial ? reinterpret_cast<const void*>(bwd_pair_kernel<D, true, true, W, WAVES>)
+                    : reinterpret_cast<const void*>(bwd_pair_kernel<D, true, false, W, WAVES>);
+  };
+  return waves == 1 ? fn(Const<1>{}) : waves == 2 ? fn(Const<2>{}) : fn(Const<4>{});
 }
 
 }  // namespace
@@ -1340,20 +1378,20 @@ int launch_forward(View q, View k, View v, float* o, float* lse, int b, int h, i
   const int64_t wide = static_cast<int64_t>((s + 255) / 256) * b * h;
   const bool filled = 8 * 2 * ((s + 255) / 256) <= 9 * ((s + 127) / 128) && (d == 64 || s > 256);
   const int nq = d != 128 && !causal && wide >= 1024 && filled ? 2 : 1;
-  const int qb = 128 * nq, nqb = (s + qb - 1) / qb;
+  const int waves = workgroup_waves(b * h, s, d != 128), qb = kRows * waves * nq, nqb = (s + qb - 1) / qb;
   FwdArgs a{q, k, v, o, lse, b, h, s, nqb, scale, causal ? 1 : 0};
   void* args[] = {&a};
   const void* fn;
   if (nq == 2) {
-    fn = d == 32 ? reinterpret_cast<const void*>(fwd_pair_kernel<32, false, 2, 3>)
-                 : reinterpret_cast<const void*>(fwd_pair_kernel<64, false, 2, 2>);
+    fn = d == 32 ? reinterpret_cast<const void*>(fwd_pair_kernel<32, false, 2, 4, 3>)
+                 : reinterpret_cast<const void*>(fwd_pair_kernel<64, false, 2, 4, 2>);
   } else {
-    fn = d == 32    ? fwd_pair_fn<32, 1, 4>(causal)
-         : d == 128 ? fwd_pair_fn<128, 1, 2>(causal)
-                    : fwd_pair_fn<64, 1, 3>(causal);
+    fn = d == 32    ? fwd_pair_fn<32, 4>(causal, waves)
+         : d == 128 ? fwd_pair_fn<128, 2>(causal, waves)
+                    : fwd_pair_fn<64, 3>(causal, waves);
   }
   return static_cast<int>(hipLaunchKernel(fn, dim3(static_cast<unsigned>(nqb) * b * h),
-                                          dim3(kThreads), args, 0,
+                                          dim3(64u * waves), args, 0,
                                           static_cast<hipStream_t>(stream)));
 }
 
@@ -1361,7 +1399,7 @@ int launch_backward(View q, View k, View v, View d_o, const float* o, const floa
                     float* part, unsigned long long* done, unsigned long long* epoch_slot,
                     unsigned long long epoch, int* ctrl, int b, int h, int s, int d, float scale,
                     int causal, int defer, int last, int give_up_bh, void* stream) {
-  const int nblk = (s + kBwdRows - 1) / kBwdRows;
+  const int waves = workgroup_waves(b * h, s, true), rows = kRows * waves, nblk = (s + rows - 1) / rows;
   BwdPairArgs a{q, k, v, d_o, o, lse, dqkv, part, done, epoch_slot, epoch, ctrl, b, h, s,
                 nblk * b * h, nblk, scale, causal ? 1 : 0, defer, last, give_up_bh};
   void* args[] = {&a};
@@ -1369,11 +1407,11 @@ int launch_backward(View q, View k, View v, View d_o, const float* o, const floa
   // Waves per SIMD: what the registers allow without spills to the loop. At d 32 the third fits once
   // the fp32 fallback's loops are not unrolled (they set the register count); with it b64 h6 s240
   // takes 63 us (67 with two), causal b8 h12 s2048 352 (375).
-  const void* fn = d == 32    ? bwd_pair_fn<32, 3>(causal, serial)
-                   : d == 128 ? bwd_pair_fn<128, 1>(causal, serial)
-                              : bwd_pair_fn<64, 2>(causal, serial);
+  const void* fn = d == 32    ? bwd_pair_fn<32, 3>(causal, serial, waves)
+                   : d == 128 ? bwd_pair_fn<128, 1>(causal, serial, waves)
+                              : bwd_pair_fn<64, 2>(causal, serial, waves);
   return static_cast<int>(hipLaunchKernel(fn, dim3(2u * static_cast<unsigned>(a.nkv)),
-                                          dim3(kThreads), args, 0,
+                                          dim3(64u * waves), args, 0,
                                           static_cast<hipStream_t>(stream)));
 }
 

@@ -306,3 +306,38 @@ def test_causal_non_finite_stays_in_its_rows(cuda, d, s):
             e = rel(got[out][:, r], want[out][:, r])
             print(f"{name} s{s} d{d} {out}: {e:.2e}", flush=True)
             assert e <= REL_TOL, (name, out)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("n,s", [(257, 1), (257, 31), (257, 32), (257, 33), (257, 63), (300, 64),
+                                 (257, 65), (256, 32), (256, 64)])
+def test_short_sequences_over_many_pairs(cuda, n, s, d, causal):
+    """One, two or four waves per workgroup, on either side of s 32, s 64 and 256 (b, h): O and
+    the gradients."""
+    scale = 0.125
+    q, k, v, g = (normal(23 * s + i, n, s, d) for i in range(4))
+    o, got = forward(q, k, v, scale, causal), gradients(q, k, v, g, scale, causal)
+    for i in (0, n // 2, n - 1):
+        at = slice(i, i + 1)
+        want = reference(q[at], k[at], v[at], scale, causal, g[at])
+        e = rel(o[at], want[0])
+        assert e <= REL_TOL
+        check_gradients([t[at] for t in got], want[1:], f"{n} x s{s} d{d} causal={causal} o {e:.2e}")
+
+
+@pytest.mark.parametrize("s", [32, 64])
+def test_short_sequences_non_finite(cuda, s):
+    """The fp32 rows in workgroups of one and two waves: one pair with an infinity, the others' bits
+    those of a clean call."""
+    n, d = 300, 64
+    q, k, v, g = (normal(29 * s + i, n, s, d) for i in range(4))
+    clean = [forward(q, k, v, 0.125, True), *gradients(q, k, v, g, 0.125, True)]
+    v[5, s // 2, 3] = math.inf
+    got = [forward(q, k, v, 0.125, True), *gradients(q, k, v, g, 0.125, True)]
+    others = torch.arange(n, device="cuda:0") != 5
+    for a, c in zip(got, clean):
+        assert torch.equal(a[others], c[others])
+    want = reference(q[5:6], k[5:6], v[5:6].nan_to_num(posinf=0.0), 0.125, True, g[5:6])
+    assert rel(got[0][5:6, :s // 2], want[0][:, :s // 2]) <= REL_TOL
+    assert rel(got[3][5:6], want[3]) <= REL_TOL
