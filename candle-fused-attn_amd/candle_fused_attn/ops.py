@@ -38,7 +38,6 @@ HIP_HEAD_DIM = CUDA_HEAD_DIM
 # torch.cuda.current_stream, 1 to the arrays and the rest of the difference to wrapping pointers:
 # 12.0 us now.
 _A3, _A4 = ctypes.c_int64 * 3, ctypes.c_int64 * 4
-_raw_stream = torch._C._cuda_getCurrentRawStream
 
 
 def _a4(values) -> ctypes.Array:
@@ -46,8 +45,9 @@ def _a4(values) -> ctypes.Array:
 
 
 def _stream(t: torch.Tensor) -> int:
-    """torch's current HIP stream of the tensor's device, as a hipStream_t."""
-    return _raw_stream(t.get_device())
+    """torch's current HIP stream of the tensor's device, as a hipStream_t. (Looked up in the call: a
+    torch built without GPU support has no such function and still imports this module.)"""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _storage(t: torch.Tensor):

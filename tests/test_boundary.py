@@ -470,3 +470,20 @@ def test_test_hooks_need_the_opt_in(opt_in):
         assert "FATTN_TEST_HOOKS" in r["err"]
         assert r["state"] == [1, 0, -1]
         assert r["grid"] == default_grid          # the schedule is unchanged
+
+
+def test_imports_on_a_torch_without_gpu_support():
+    """The package imports (and refuses a CPU tensor) where torch has no stream query of its own."""
+    import subprocess
+    import sys
+    code = (f"import sys; sys.path.insert(0, {str(REPO / 'candle-fused-attn_amd')!r})\n"
+            "import torch\n"
+            "del torch._C._cuda_getCurrentRawStream\n"
+            "import candle_fused_attn as cfa\n"
+            "try:\n"
+            "    cfa.fused_attention_qkv(torch.zeros(1, 2, 192), 1, 0.125, False)\n"
+            "except cfa.FusedAttentionError as e:\n"
+            "    print(e)\n")
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert res.returncode == 0, res.stderr
+    assert "not on a HIP device" in res.stdout
