@@ -1342,22 +1342,26 @@ int workgroup_waves(int bh, int s, bool two) {
   return s <= 32 ? 1 : two ? 2 : 4;
 }
 
-// Causal, up to this many key blocks: dV summed over the queries one at a time, on the fp32 matrix
-// instruction (kSerial). The first keys of a causal row sum hundreds of terms of one sign, and there
-// a sum of one rounding per query, as the composed fp32 path makes, and one of three per 16 queries
-// drift apart by more than the reference's band around that path (5e-6; tests/parity.rs:218): at
-// b 2 h 6 s 240 the composed path's dV is 6.0e-6 from fp64, so a correctly rounded one misses the
-// band too. The small grids, whose time is a workgroup's latency, keep to the band: backward at that
-// shape 25 us without, 31 with (the fp32 kernels' 35); larger ones take the faster and more accurate
-// sum.
-constexpr int kSerialBlocks = 64;
+// Causal, s up to kSerialLength and up to kSerialBlocks key blocks: dV summed over the queries one at a
+// time, on the fp32 matrix instruction (kSerial). The first keys of a causal row sum hundreds of terms
+// of one sign, and there a sum of one rounding per query, as the composed fp32 path makes, and one of
+// three per 16 queries drift apart by more than the reference's band around that path (5e-6;
+// tests/parity.rs:218): at b 2 h 6 s 240 the composed path's dV is 6.0e-6 from fp64, so a correctly
+// rounded one misses the band too. Small grids of the lengths for which the reference states the band
+// (up to 240; here two blocks) keep to it, at a few us per call; all others take the faster and more
+// accurate sum. With it / without, backward us: s 64 12.3 / 10.7, s 128 19.3 / 16.1, s 240 30.5 / 23.5
+// (b 2 h 6: 31.0 / 24.0), and what longer walks would pay: s 512 51.5 / 36.9, s 2048 179 / 119, s 8192
+// 689 / 447; D 128 s 1024 180 / 125.
+constexpr int kSerialBlocks = 64, kSerialLength = 256;
 template <int D, int WAVES>
 const void* bwd_pair_fn(int causal, bool serial, int waves) {
   auto fn = [&](auto w) {
     constexpr int W = decltype(w)::value;
-    return !causal  ? reinterpret_cast<const void*>(bwd_pair_kernel<D, false, false, W, WAVES>)
-           : serial ? reinterpret_cast<const void*>(bwd_pair_kernel<D, true, true, W, WAVES>)
-                    : reinterpret_cast<const void*>(bwd_pair_kernel<D, true, false, W, WAVES>);
+    if constexpr (W == 4) {  // (fewer waves: more than 256 (b, h))
+      if (serial) return reinterpret_cast<const void*>(bwd_pair_kernel<D, true, true, W, WAVES>);
+    }
+    return causal ? reinterpret_cast<const void*>(bwd_pair_kernel<D, true, false, W, WAVES>)
+                  : reinterpret_cast<const void*>(bwd_pair_kernel<D, false, false, W, WAVES>);
   };
   return waves == 1 ? fn(Const<1>{}) : waves == 2 ? fn(Const<2>{}) : fn(Const<4>{});
 }
@@ -1403,7 +1407,7 @@ int launch_backward(View q, View k, View v, View d_o, const float* o, const floa
   BwdPairArgs a{q, k, v, d_o, o, lse, dqkv, part, done, epoch_slot, epoch, ctrl, b, h, s,
                 nblk * b * h, nblk, scale, causal ? 1 : 0, defer, last, give_up_bh};
   void* args[] = {&a};
-  const bool serial = causal && a.nkv <= kSerialBlocks;
+  const bool serial = causal && s <= kSerialLength && a.nkv <= kSerialBlocks;
   // Waves per SIMD: what the registers allow without spills to the loop. At d 32 the third fits once
   // the fp32 fallback's loops are not unrolled (they set the register count); with it b64 h6 s240
   // takes 63 us (67 with two), causal b8 h12 s2048 352 (375).

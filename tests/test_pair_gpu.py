@@ -6,10 +6,12 @@ from __future__ import annotations
 
 import math
 
+import numpy as np
 import pytest
 import torch
 
 import candle_fused_attn as cfa
+import test_parity_gpu as parity
 
 pytestmark = pytest.mark.gpu
 
@@ -341,3 +343,36 @@ def test_short_sequences_non_finite(cuda, s):
     want = reference(q[5:6], k[5:6], v[5:6].nan_to_num(posinf=0.0), 0.125, True, g[5:6])
     assert rel(got[0][5:6, :s // 2], want[0][:, :s // 2]) <= REL_TOL
     assert rel(got[3][5:6], want[3]) <= REL_TOL
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("n,s", [(21, 257), (1, 640), (1, 2100)])
+def test_backward_long_walks_of_small_grids(cuda, n, s, d):
+    """Causal, few key blocks and walks past the serial rule's length: the same sum as in large grids,
+    to the bit."""
+    q, k, v, g = (normal(31 * s + i, n, s, d) for i in range(4))
+    got = gradients(q, k, v, g, 0.125, True)
+    check_gradients([t[:1] for t in got], reference(q[:1], k[:1], v[:1], 0.125, True, g[:1])[1:],
+                    f"{n} x s{s} d{d}")
+    more = -(-65 // ((s + 127) // 128))  # pairs of more than 64 key blocks
+    many = gradients(*(t[:1].expand(more, s, d).contiguous() for t in (q, k, v, g)), 0.125, True)
+    for a, w in zip(got, many):
+        assert torch.equal(a[0], w[0])
+
+
+@pytest.mark.parametrize("shape", [(2, 7, 3, 64), (2, 240, 6, 64), (1, 97, 2, 64), (1, 33, 2, 64),
+                                   (2, 70, 3, 32), (1, 128, 2, 128), (2, 240, 3, 128)])
+def test_closed_form_in_large_causal_grids(orc, cuda, shape):
+    """The closed-form inputs of the reference's test in a batch of more than 64 key blocks, where the
+    causal dV is not summed one query at a time: no component less accurate than 1.5 times the
+    composed fp32 path against fp64."""
+    b, s, h, d = shape
+    x, w = orc.closed_form_inputs(b, s, h, d)
+    want = parity.oracle_qkv(orc, x, w, h, d, True, np.float64)
+    floor, cmax = parity.composed_floor(orc, x, w, h, d, True, want[0], want[2])
+    copies = -(-65 // (b * h * ((s + 127) // 128)))
+    qkv, wt = (torch.from_numpy(np.tile(t, (copies, 1, 1))).to(cuda) for t in (x, w))
+    out, grad = (t[-b:] for t in parity.run("fused_qkv", qkv, wt, h, d, True))
+    parity.check_errors(orc, out, grad, want[0], want[2], f"{copies} copies", floor, d=d)
+    e = orc.max_abs(grad.cpu().numpy(), want[2])
+    assert e <= max(parity.zero_band(d), 1.5 * cmax), f"max-abs {e:.3e}"
