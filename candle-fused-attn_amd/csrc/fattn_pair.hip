@@ -1112,9 +1112,9 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D, W>& sm
   }
   for (; u < nsteps; ++u) masked(u);
   if (!wave_live) return;
-  // The two factors of dK and of dV.
-  float fk = pow2(-kTop), fk2 = pow2(-kp) / dsc * a.scale, fv = pow2(-kTop - kp), fv2 = 1.0f / psc;
-  const float z = probe_finite<kDT>(dk, probe_finite<kDT>(dv, fk2 * 0.0f));
+  // The two factors of dK and of dV: the second is a power of two, exact where it is subnormal.
+  float fk = pow2(-kTop) * a.scale, fk2 = pow2(-kp) / dsc, fv = pow2(-kTop - kp), fv2 = 1.0f / psc;
+  const float z = probe_finite<kDT>(dk, probe_finite<kDT>(dv, fk * 0.0f));
   if (__builtin_amdgcn_ballot_w64(key < S && !(z == 0.0f)) != 0) {
     bwd_keys_fp32<D, kCausal>(a, b, h, kw0, sm.o[w], dk, dv, late(lane));
     fk = a.scale, fk2 = fv = fv2 = 1.0f;
@@ -1271,7 +1271,7 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D, W>&
                             static_cast<int64_t>(h) * D
                       : a.part + (static_cast<int64_t>(bh) * ntile16 * kBwdQueryTile + qw0) * D;
   const float factor = direct ? a.scale : 1.0f;
-  float f = pow2(-kTop), f2 = pow2(-kp) / dsc * factor;
+  float f = pow2(-kTop) * factor, f2 = pow2(-kp) / dsc;
   if (gave_up && direct) {
     // (The test hook, as a wait that ran out would: NaN and the guard word.)
     if (lane == 0) {
@@ -1279,7 +1279,7 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D, W>&
     }
     f = __builtin_nanf("");
   } else if (__builtin_amdgcn_ballot_w64(
-                 qi < S && !(probe_finite<kDT>(dq, f2 * 0.0f) == 0.0f)) != 0) {
+                 qi < S && !(probe_finite<kDT>(dq, f * 0.0f) == 0.0f)) != 0) {
     bwd_queries_fp32<D, kCausal>(a, b, h, qw0, sm.o[w], dq, late(lane));
     f = factor, f2 = 1.0f;
   }

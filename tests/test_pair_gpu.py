@@ -376,3 +376,18 @@ def test_closed_form_in_large_causal_grids(orc, cuda, shape):
     parity.check_errors(orc, out, grad, want[0], want[2], f"{copies} copies", floor, d=d)
     e = orc.max_abs(grad.cpu().numpy(), want[2])
     assert e <= max(parity.zero_band(d), 1.5 * cmax), f"max-abs {e:.3e}"
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("f", [1e-33, 1e-35])
+@pytest.mark.parametrize("scale", [0.1, 0.003])
+def test_tiny_gradients_under_any_scale(cuda, scale, f, causal):
+    """As above with a scale that is no power of two: dQ and dK keep their bits where the factor that
+    takes their sums back is subnormal."""
+    s, d = 200, 64
+    q, k, v, g = (normal(160 + i, 2, s, d) for i in range(4))
+    got, want = gradients(q, k, v, g * f, scale, causal), reference(q, k, v, scale, causal, g * f)[1:]
+    for name, a, w in zip(("dq", "dk", "dv"), got, want):
+        diff = (a.double().cpu() - w).norm().item()
+        print(f"{f:g} scale {scale} causal={causal} {name}: {diff / w.norm().item():.2e}", flush=True)
+        assert diff <= REL_TOL * w.norm().item() + 2.0 ** -149 * math.sqrt(w.numel()), name
