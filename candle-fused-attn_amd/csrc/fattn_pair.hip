@@ -269,7 +269,9 @@ struct Stage {
       x[i][1] = *reinterpret_cast<const f4*>(p + off + 16);
     }
   }
-  // The tiles and their rows' units (2^e).
+  // The tiles and their rows' units: 2^(e - kTop) of operand a's, 2^e of b's. (a's meet the unit of a
+  // wave's own row, 2^(e - kTop) too, in the factor of the scores: the product of a tiny and a huge row
+  // passes through no subnormal, which 2^(-2 kTop) on one side would be from 2^-98 down.)
   __device__ __forceinline__ void store(Tile<D>& a, Tile<D>& b, float* ua, float* ub, int w,
                                         int lane) {
 #pragma unroll
@@ -277,7 +279,7 @@ struct Stage {
       const bool is_b = kHalves ? lane >= 32 : i >= kPer;
       const int r = row(i, w, lane);
       e[i] = exponent(group_max<kC>(abs_max8(x[i][0], x[i][1], 0.0f)));
-      if (lane % kC == 0) (is_b ? ub : ua)[r] = pow2(e[i]);
+      if (lane % kC == 0) (is_b ? ub : ua)[r] = pow2(is_b ? e[i] : e[i] - kTop);
       const Pair s = split8(x[i][0], x[i][1], pow2(kTop - e[i]));
       char* p = reinterpret_cast<char*>(is_b ? &b : &a) + r * (2 * D) +
                 (((lane % kC) ^ chunk_swz<D>(r)) << 4);
@@ -287,8 +289,8 @@ struct Stage {
   }
 };
 // Beside a Stage whose operand b is dO: O's rows in the same lanes, and D = rowsum(dO o O) of the
-// tile's 32 rows, in units of dO's rows. O's offsets are in elements: its rows of one (b, h) may span more than 4 GiB (the
-// views' may not).
+// tile's 32 rows, in units of dO's rows and times 2^kTop (dS meets Q's unit). O's offsets are in
+// elements: its rows of one (b, h) may span more than 4 GiB (the views' may not).
 template <int D, int W>
 struct RowDots {
   using S = Stage<D, W>;
@@ -316,7 +318,7 @@ struct RowDots {
       if constexpr (D >= 64) t += dpp<0x141>(t);
       if constexpr (D == 128) t += dpp<0x140>(t);
       if (lane % kC == 0 && (!S::kHalves || lane >= 32)) {
-        dst[S::row(i, w, lane)] = t * pow2(-st.e[S::kN / 2 + i]);
+        dst[S::row(i, w, lane)] = t * pow2(kTop - st.e[S::kN / 2 + i]);
       }
     }
   }
@@ -551,7 +553,7 @@ fwd_pair_kernel(FwdArgs a) {
   // is the scaled scores'), and the second tile's loads.
   Stage<D, W> st;
   Pair q[NQ][kKS];
-  float cq[NQ];  // |scale| log2 e over the scales of the query and kTop
+  float cq[NQ];  // |scale| log2 e over the query's scale
   {
     OwnRows<D> own[NQ];
     st.load(kop, vop, 0, S - 1, w, lane);
@@ -562,7 +564,7 @@ fwd_pair_kernel(FwdArgs a) {
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
       cq[n] = own[n].split(a.scale < 0.0f ? -1.0f : 1.0f, q[n]) *
-              (fabsf(a.scale) * kLog2e * pow2(-kTop));
+              (fabsf(a.scale) * kLog2e);
     }
     if constexpr (W == 2) st.store(sm.t.kv[1].k, sm.t.kv[1].v, sm.uk[1], sm.uv[1], w, lane);
   }
@@ -988,7 +990,7 @@ __device__ __forceinline__ void bwd_keys(const BwdPairArgs& a, BwdSmem<D, W>& sm
   f16v dk[kDT], dv[kDT];
 #pragma unroll
   for (int dt = 0; dt < kDT; ++dt) dk[dt] = zero16(), dv[dt] = zero16();
-  const float cs = a.scale * kLog2e * uk * pow2(-kTop), cg = uv * pow2(-kTop);
+  const float cs = a.scale * kLog2e * uk, cg = uv;
   float psc = kSerial ? 1.0f : kMaxScale, dsc = kMaxScale;
   const int roff0 = row_off<D>(j, g), coff0 = col_off<D>(lane);
 
@@ -1163,7 +1165,7 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D, W>&
         Dq = fmaf(og.x[ks][e / 4][e % 4], oo.x[ks][e / 4][e % 4], Dq);
       }
     }
-    Dq = pair_sum(Dq);
+    Dq = pair_sum(Dq) * pow2(kTop);  // (dP and D times 2^kTop meet K's unit)
     L = shifted_l(L, kp);
     uq = oq.split(1.0f, qB);
     ug = og.split(1.0f, gB);
@@ -1174,7 +1176,7 @@ __device__ __forceinline__ void bwd_queries(const BwdPairArgs& a, BwdSmem<D, W>&
   f16v dq[kDT];
 #pragma unroll
   for (int dt = 0; dt < kDT; ++dt) dq[dt] = zero16();
-  const float cs = a.scale * kLog2e * uq * pow2(-kTop), cg = ug * pow2(-kTop);
+  const float cs = a.scale * kLog2e * uq, cg = ug;
   float dsc = kMaxScale;
   const int roff0 = row_off<D>(j, g), coff0 = col_off<D>(lane);
 

@@ -391,3 +391,19 @@ def test_tiny_gradients_under_any_scale(cuda, scale, f, causal):
         diff = (a.double().cpu() - w).norm().item()
         print(f"{f:g} scale {scale} causal={causal} {name}: {diff / w.norm().item():.2e}", flush=True)
         assert diff <= REL_TOL * w.norm().item() + 2.0 ** -149 * math.sqrt(w.numel()), name
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("f", [1e-33, 1e33])
+def test_tiny_against_huge(cuda, f, d, causal):
+    """Queries and keys, values and output gradients of 1e-33 against 1e33: scores, and dP, of ordinary
+    size."""
+    s = 150
+    q, k, v, g = (normal(300 + i, 2, s, d) * x for i, x in enumerate((f, 1 / f, f, 1 / f)))
+    want = reference(q, k, v, 0.125, causal, g)
+    got = [forward(q, k, v, 0.125, causal), *gradients(q, k, v, g, 0.125, causal)]
+    for name, a, w in zip(("o", "dq", "dk", "dv"), got, want):
+        e = rel(a, w)
+        print(f"{f:g} d{d} causal={causal} {name}: {e:.2e}", flush=True)
+        assert e <= REL_TOL, name
