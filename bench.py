@@ -60,9 +60,10 @@ SCALE = 0.125
 TRAFFIC = REPO / "profiles" / "traffic.json"
 LIB = REPO / "candle-fused-attn_amd" / "lib" / "libfattn.so"
 COPY_KIB = 256 * 1024            # the --calibrate-copy kernel moves 256 MiB each way
-KERNEL_NAMES = {"fwd": "fwd_pair_kernel<64, false, 1, 3>",
-                "bwd_main": "bwd_pair_kernel<64, false, false, 2>", "bwd_dq": "dq_kernel<64>"}
-CAUSAL_FWD_NAME = "fwd_pair_kernel<64, true, 1, 3>"   # config 3's forward
+KERNEL_NAMES = {"fwd": "fwd_pair_kernel<64, false, 1, 4, 3>",
+                "bwd_main": "bwd_pair_kernel<64, false, false, 4, 2>", "bwd_dq": "dq_kernel<64>"}
+CAUSAL_FWD_NAME = "fwd_pair_kernel<64, true, 1, 4, 3>"   # config 3's forward
+WIDE_FWD_NAME = "fwd_pair_kernel<64, false, 2, 4, 2>"    # config 5's: 64 queries per wave
 # (The second names: traces of libraries with the fp32-instruction kernels.)
 FWD_PREFIXES = ("fwd_pair_kernel", "fwd_kernel")
 MAIN_PREFIXES = ("bwd_pair_kernel", "bwd_split_kernel", "bwd_kernel")
@@ -325,6 +326,17 @@ def _kernel_label(raw: str) -> str:
     return name.split("(", 1)[0].replace("void ", "")
 
 
+def forward_launch(cfg: int) -> tuple[str, int]:
+    """A config's forward launch at d 64: kernel and workgroups (four waves of 32 queries each, or of
+    64 where 1024 such workgroups are filled; none of the configs is short enough for fewer waves)."""
+    _, _, b, h, s, causal, _, _ = CONFIGS[cfg]
+    if causal:
+        return CAUSAL_FWD_NAME, -(-s // 128) * b * h
+    if -(-s // 256) * b * h >= 1024 and 16 * -(-s // 256) <= 9 * -(-s // 128):
+        return WIDE_FWD_NAME, -(-s // 256) * b * h
+    return KERNEL_NAMES["fwd"], -(-s // 128) * b * h
+
+
 def _headline_windows(rows: list, warmup: int, steps: int, cfg: int) -> dict | None:
     """The headline's windows from a time-ordered list of (start, kernel, workgroups, payload)
     dispatches of `bench.py --warmup W --steps K`: {"timed", "fwds", "kern", "bwds", "idle"}, each
@@ -333,10 +345,7 @@ def _headline_windows(rows: list, warmup: int, steps: int, cfg: int) -> dict | N
     starts at a forward launch, or at a step-2 launch in a step that already holds one) and the
     main config's steps picked by the forward's name and grid; the headline's are the run of them
     after configs 3-5, its K forwards, K kernel-level steps and K backwards the steps after it."""
-    b, h, s = CONFIGS[cfg][2], CONFIGS[cfg][3], CONFIGS[cfg][4]
-    qb = 64 if CONFIGS[cfg][5] else 128
-    main_fwd = (CAUSAL_FWD_NAME if CONFIGS[cfg][5] else KERNEL_NAMES["fwd"],
-                ((s + qb - 1) // qb) * b * h)
+    main_fwd = forward_launch(cfg)
     steps_seq: list[list] = []
 
     def step2(name):
@@ -800,7 +809,7 @@ def main() -> int:
                        "step": round(kus["step"], 2)},
         "dq_sum": "split" if w.split else "turns",
         "roofline": {
-            "kernel": "bwd_pair_kernel<64, false, false, 2> (fattn_bwd_main_f32_d64)",
+            "kernel": f"{KERNEL_NAMES['bwd_main']} (fattn_bwd_main_f32_d64)",
             "bound": "mfma",
             "achieved": round(step2_tflops, 3),
             "peak": PEAK_FP32_MFMA_TFLOPS,

@@ -16,7 +16,23 @@ import pytest  # noqa: E402
 PREFIX = "void fattn::(anonymous namespace)::"
 FWD, MAIN, DQ = (bench.KERNEL_NAMES[k] for k in ("fwd", "bwd_main", "bwd_dq"))
 CAUSAL_FWD = bench.CAUSAL_FWD_NAME
-D32_FWD = "fwd_kernel<32, 128, 64, 3, false>"
+D32_FWD = "fwd_pair_kernel<32, false, 1, 4, 4>"
+
+
+def test_kernel_names_are_the_librarys():
+    """The kernels that the summaries look for exist in the built library, under these names."""
+    lib = bench.LIB.read_bytes()
+    for name in (*bench.KERNEL_NAMES.values(), CAUSAL_FWD, bench.WIDE_FWD_NAME, D32_FWD):
+        kernel, args = name.rstrip(">").split("<")
+        mangled = kernel + "I" + "".join(
+            f"Lb{int(a == 'true')}E" if a in ("true", "false") else f"Li{a}E"
+            for a in args.split(", ")) + "E"
+        assert mangled.encode() in lib, name
+
+
+@pytest.mark.parametrize("cfg,grid", [(2, 768), (3, 768), (4, 1536), (5, 1024)])
+def test_forward_launch(cfg, grid):
+    assert bench.forward_launch(cfg)[1] == grid
 
 
 def write_trace(path, w, k, cfg=2):
@@ -26,7 +42,7 @@ def write_trace(path, w, k, cfg=2):
     (fwd 52, main 135, dq 4), backwards (main 137), then config 2 at d 32."""
     b, h, s = bench.CONFIGS[2][2], bench.CONFIGS[2][3], bench.CONFIGS[2][4]
     grid = ((s + 127) // 128) * b * h
-    head, other = (FWD, grid), (CAUSAL_FWD, ((s + 63) // 64) * b * h)
+    head, other = (FWD, grid), (CAUSAL_FWD, grid)
     if cfg == 3:  # config 3 as the headline (bench.py --causal); config 2 is then the other
         head, other = other, head
     FWD_, grid = head
