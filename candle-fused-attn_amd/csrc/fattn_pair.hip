@@ -20,11 +20,12 @@
 // wave's own rows hold theirs in a register; a staged row's is in LDS beside the tile (`unit`, 2^e)
 // and multiplies back per accumulator row: into the scores' factor, and, where the product sums over
 // the staged rows, into the weights (P, dS). The weights of a lane's own row follow a power of two
-// of their own, so that they keep 22 bits down to about 2^-17 of the largest term of the sum, and no
-// term's error depends on a row that has no part in it. (One scale per tile, or the largest so far,
-// costs less: forward b64 h6 s240 34.6 us against 36.5, b16 h16 s1024 205 against 222, backward 105
-// against 107 and 779 against 798, d 128 229 against 236. But one large row, masked or not, or one
-// key of large weight, takes the bits of all the others.)
+// of their own, which puts the largest term of the sum at 2^6 or more: 22 bits down to 2^-9 of it,
+// below that an error of 2^-31 of it, and none that depends on a row that has no part in the sum. (One
+// scale per tile, or the largest so far, costs less: forward b64 h6 s240 28.9 us against 30.3, b16 h16
+// s1024 200 against 220, with inputs of deviation 2, whose weights move the scales more often, 203
+// against 242; backward 92 against 94 and 792 against 808, d 128 228 against 235. But one large row,
+// masked or not, or one key of large weight, takes the bits of all the others.)
 //
 // For one v_mfma_f32_32x32x16_f16, lane l (j = l % 32, g = l / 32) supplies A[j][8 g + e] and
 // B[8 g + e][j], e = 0..7, and holds D[8 (r / 4) + 4 g + r % 4][j], r = 0..15. As the contraction
@@ -657,28 +658,21 @@ fwd_pair_kernel(FwdArgs a) {
         }
         // (-inf: a row with no live key.)
         const float ref = pair_max(tmax) - kRefTop;
+        // O's unit is p / wsc: where p falls by alpha, wsc rises and O stays as it is but for rounding.
+        float to = wsc[n], alpha = 1.0f;
         if (!(pair_sum(psum) <= kRowTop) && ref > m[n]) {
-          // O's unit is p / wsc: wsc rises as p falls, O stays as it is but for rounding.
-          const float alpha = m[n] == kNegInf ? 0.0f : exp2_hw(m[n] - ref);
-          float to = kMaxScale, f = 0.0f;
-          if (alpha > 0x1p-100f) {
-            to = fminf(wsc[n] * pow2(-exponent(alpha)), kMaxScale);
-            f = alpha * (to / wsc[n]);
-          }
+          alpha = m[n] == kNegInf ? 0.0f : exp2_hw(m[n] - ref);
+          to = alpha > 0x1p-100f ? fminf(to * pow2(-exponent(alpha)), kMaxScale) : kMaxScale;
           m[n] = ref;
           lsum[n] *= alpha;
-          wsc[n] = to;
-#pragma unroll
-          for (int dt = 0; dt < kDT; ++dt) acc[n][dt] *= f;
           exps();
         }
         wmax = pair_max(fmaxf(wmax, 0.0f));
-        if (wmax * wsc[n] > kMaxWeight) {
-          const float to = pow2(kWTop - exponent(wmax));
+        if (wmax * to > kMaxWeight) to = pow2(kWTop - exponent(wmax));
+        const float f = alpha > 0x1p-100f ? alpha * (to / wsc[n]) : 0.0f;
+        wsc[n] = to;
 #pragma unroll
-          for (int dt = 0; dt < kDT; ++dt) acc[n][dt] *= to / wsc[n];
-          wsc[n] = to;
-        }
+        for (int dt = 0; dt < kDT; ++dt) acc[n][dt] *= f;
       }
       lsum[n] += psum;
       p[n][0] = split_acc<0>(e, wsc[n]);
@@ -802,7 +796,10 @@ struct BwdPairArgs {
   float scale;
   int causal, defer, last, give_up_bh;
 };
-constexpr int kDsTop = 11;  // where a new scale puts the largest weight
+// Where a new scale puts the largest weight: 9 bits of room before the next one moves it, which costs
+// a pass over the sums (with 5, inputs of deviation 2: d 128 b64 h6 s240 259 us against 242, d 32 56.0 /
+// 54.4, b16 h16 s1024 851 / 839), and no row error above 1.01 of that over 1580 checks.
+constexpr int kDsTop = 7;
 
 // The running scale of the weights in one lane: raises nothing, lowers `sc` (and the accumulators by
 // the same factor) where a weight would exceed kMaxWeight. First the largest, then the test.
