@@ -170,7 +170,7 @@ hipMemPool_t device_pool(hipStream_t stream) {
 
 WorkspaceCache::Lease WorkspaceCache::take(std::size_t b, std::size_t h, std::size_t s,
                                            std::size_t d, hipStream_t stream) {
-  const std::size_t bytes = fattn_bwd_workspace_bytes(
+  const std::size_t bytes = fattn_bwd_workspace_min_bytes(
       static_cast<int64_t>(b), static_cast<int64_t>(h), static_cast<int64_t>(s),
       static_cast<int64_t>(d));
   Lease kept;
@@ -179,7 +179,7 @@ WorkspaceCache::Lease WorkspaceCache::take(std::size_t b, std::size_t h, std::si
     std::swap(kept, kept_);
   }
   if (kept.ws && kept.stream == stream && kept.bytes >= bytes) {
-    kept.bytes = bytes;  // the size this backward asks for (its chunks follow from it)
+    kept.bytes = bytes;  // the size this backward asks for
     return kept;
   }
   Lease fresh;

@@ -132,7 +132,7 @@ class WorkspaceCache {
     std::size_t bytes = 0;
     hipStream_t stream = nullptr;
   };
-  // The workspace for a (b, h, s, d) backward on `stream` (fattn_bwd_workspace_bytes).
+  // The workspace for a (b, h, s, d) backward on `stream` (the minimum: all the kernels use).
   Lease take(std::size_t b, std::size_t h, std::size_t s, std::size_t d, hipStream_t stream);
   // Keeps `lease` for the next backward (the larger one, if one was given back meanwhile).
   void give_back(Lease lease);
