@@ -619,8 +619,7 @@ def main() -> int:
     ap.add_argument("--warmup", type=int, default=200)
     ap.add_argument("--causal", action="store_true", help="config 3 as the main workload")
     ap.add_argument("--config", type=int, choices=sorted(CONFIGS), default=None,
-                    help="the main workload's config (default 2; --causal is config 3); the "
-                         "driver's line is config 2's")
+                    help="the main workload's config (default 2; --causal is config 3)")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
     ap.add_argument("--no-accuracy", action="store_true", help="skip the fp64 scoring")
     ap.add_argument("--no-extra", action="store_true",

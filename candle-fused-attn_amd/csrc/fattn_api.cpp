@@ -50,13 +50,10 @@ int64_t split_slots(int keys, int64_t d) {
   return (keys > kBwdKeys && d > 32 ? 2 : 3) * int64_t{256};
 }
 
-// The (b, h) pairs per chunk of the split dQ sum that a workspace of ws_bytes holds: b h when it
-// holds the whole split; else, at d <= 64, from the most pairs whose split partials, arrival
-// slots and done flags fit:
-//   causal: equal chunks (the key blocks' own sums read the partials at device scope, so the
-//     XCDs a chunk's key blocks run on do not matter);
-//   non-causal: the most pairs whose key blocks fill whole rounds of the chip's workgroup slots
-//     (every key block walks all query tiles, so a partial round idles slots; the last chunk
+// The (b, h) pairs per chunk of a workspace of ws_bytes: b h when it holds the whole split size; else,
+// at d <= 64, from the most pairs whose split size fits:
+//   causal: equal chunks;
+//   non-causal: the most pairs whose key blocks fill whole rounds of workgroup slots (the last chunk
 //     takes the rest);
 // 0 when that is fewer than min_pairs. A chunk's size is workspace_layout(1, chunk, s, d).
 int64_t split_chunk(int64_t b, int64_t h, int64_t s, int64_t d, size_t ws_bytes,
@@ -95,10 +92,9 @@ int64_t min_chunk_pairs(int64_t b, int64_t h, int64_t s, int64_t d, bool causal)
   return (blocks + nkb - 1) / nkb;
 }
 
-// The workspace the library asks for within `limit` bytes: the whole split, else the split of the
-// larger of the chunks each mask's rule takes (the size takes no mask; a run applies its own rule
-// to the workspace it is given, and each rule's chunk fits in the larger one), else the turn
-// hand-over's minimum (possibly over the limit: the caller decides).
+// The workspace the library asks for within `limit` bytes: the whole split size, else that of the
+// larger of the chunks each mask's rule takes (the size takes no mask), else the minimum (possibly
+// over the limit: the caller decides).
 size_t workspace_within(int64_t b, int64_t h, int64_t s, int64_t d, size_t limit) {
   const Workspace l = workspace_layout(b, h, s, d);
   if (l.bytes_split <= limit) return l.bytes_split;
@@ -315,7 +311,7 @@ int run_bwd_main(const char* who, View q, View k, View v, const float* o, View d
   return ok();
 }
 
-// Step 3: in split mode (the workspace holds the partials) dQ from the partials; else nothing.
+// Step 3: with a split-size workspace, the dQ tiles that step 2 left there (a test hook); else nothing.
 int run_bwd_dq(const char* who, float* dqkv, void* ws, size_t ws_bytes, int64_t b, int64_t h,
                int64_t s, int64_t d, float scale, int causal, void* stream) {
   if (int rc = check_range(who, b, h, s, d)) return rc;
@@ -533,8 +529,7 @@ int fattn_bwd_f32_noalloc(const float* q, const float* k, const float* v, const 
     return fail(FATTN_EINVAL, "fused_attention: null strides");
   }
   if (int rc = check_range(who, b, h, s, d)) return rc;
-  // dQ summed as fattn_bwd_f32 sums it with a workspace of the scratch's size: the whole split
-  // when it fits, else (d <= 64) the split by chunks of (b, h) pairs, else the turn hand-over.
+  // The size that fattn_bwd_f32 would be given within the scratch; what it refuses is refused.
   const size_t need = fattn::workspace_within(b, h, s, d, FATTN_STATIC_SCRATCH_BYTES);
   if (need > FATTN_STATIC_SCRATCH_BYTES) {
     return fail(FATTN_EWORKSPACE,

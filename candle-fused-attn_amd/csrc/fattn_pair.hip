@@ -150,9 +150,8 @@ __device__ __forceinline__ Pair ld_row(const Tile<D>& t, int off) {
   return Pair{*reinterpret_cast<const h8*>(p), *reinterpret_cast<const h8*>(p + kPlane<D>)};
 }
 // The lane's base offset of the transposed read of columns lane % 32 (32 dt + those at this ^
-// col_step(dt)): within each group of
-// 16 lanes, lane i points at row i / 4 and columns 4 (i % 4) .. + 3 of a 4 x 16 block and receives
-// the block's column i. Rows 16 ks + 4 g + (0..3) at + 32 D ks bytes; 8 rows on, + 16 D bytes and
+// col_step(dt)): within each group of 16 lanes, lane i points at row i / 4 and columns 4 (i % 4) .. + 3
+// of a 4 x 16 block and receives the block's column i. Rows 16 ks + 4 g + (0..3) at + 32 D ks bytes; 8 rows on, + 16 D bytes and
 // the chunk of the offset changed by kSwz8.
 template <int D>
 __device__ __forceinline__ int col_off(int lane) {

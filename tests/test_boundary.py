@@ -64,13 +64,12 @@ def test_workspace_size_is_aligned_and_monotone():
     assert L.fattn_bwd_workspace_bytes(-1, 6, 240, 64) == 0
     assert L.fattn_bwd_workspace_min_bytes(-1, 6, 240, 64) == 0
     assert L.fattn_bwd_workspace_bytes(64, 6, 240, 48) == 0      # head_dim not built
-    # Past FATTN_SPLIT_MAX_BYTES (4 GiB), at d <= 64: the split sum of equal chunks of (b, h),
-    # each chunk's state in a workspace laid out for that many pairs (split_bytes(1, chunk, ...));
-    # at d 128 the minimum (the turn hand-over).
+    # Past FATTN_SPLIT_MAX_BYTES (4 GiB), at d <= 64: the split size of a chunk of (b, h) pairs
+    # (split_bytes(1, chunk, ...)); at d 128 the minimum.
     cap = 4 << 30
     assert L.fattn_bwd_workspace_split_bytes(1, 64, 16384, 64) > cap
     # 1 GiB of partials per pair: 3 fit, but their 3 x 128 key blocks (of 128 keys) fill less than
-    # one round of the 512 workgroup slots: the minimum (turns)
+    # one round of the 512 workgroup slots: the minimum
     assert L.fattn_bwd_workspace_split_bytes(1, 3, 16384, 64) <= cap
     assert L.fattn_bwd_workspace_split_bytes(1, 4, 16384, 64) > cap
     assert (L.fattn_bwd_workspace_bytes(1, 64, 16384, 64)
@@ -350,9 +349,9 @@ def expected_keys(bh, s, d, causal):
 
 
 def expected_sum_bh(bh, s, causal, keys=64):
-    """Restated from the schedule's definition: every (b, h) has its tiles summed in step 2 while
-    a (b, h) has at most 256 key blocks (the summing units read the partials at device scope, so
-    where the key blocks ran does not matter)."""
+    """Restated from the plan's definition: every (b, h) has its tiles summed in step 2 while a (b, h)
+    has at most 256 key blocks. (The plan is what the size and audit queries answer by; the kernels
+    sum nothing across workgroups.)"""
     nkb = -(-s // keys)
     return 0 if nkb > 256 else bh
 
@@ -374,8 +373,8 @@ def expected_sum_grid(bh, s, keys=64):
 
 @pytest.mark.parametrize("causal", [False, True])
 def test_step2_dq_sum_schedule(causal):
-    """Step 2's dQ sums, over many shapes (the kernel's own scheduling functions, run on the
-    host): a causal unit waits only for key blocks earlier in the grid; a non-causal unit of XCD x
+    """The plan of dQ sums that the size and audit queries answer by, over many shapes (no launch
+    runs it: the kernels keep dQ in registers): a causal unit waits only for key blocks earlier in the grid; a non-causal unit of XCD x
     takes a (b, h) whose last key block runs on x (or, after those, one whose last key block is
     dealt round robin: the plan's order); no target lies past b h (the case a rounded-up per-XCD
     count once produced: nkb = 1, b h not a multiple of 8, e.g. h 17 s 50); no tile is summed
@@ -404,7 +403,7 @@ def test_step2_dq_sum_schedule(causal):
                     assert a["grid"] == want_grid, (s, bh, d, a, want_grid)
                 n += 1
     assert n > 1000
-    # The advisor's case: b 1, h 17, s 50 (one key block per (b, h)): no target past b h; all 17
+    # The smallest such case: b 1, h 17, s 50 (one key block per (b, h)): no target past b h; all 17
     # heads summed in step 2 (16 by the XCDs' ranges, the 17th by the round-robin rest).
     if not causal:
         a = sum_audit(1, 17, 50, 64, False)

@@ -1,7 +1,6 @@
 """fattn_bwd_f32_noalloc (the backward with the library's static scratch as its workspace) against
-fattn_bwd_f32 with a caller's workspace of the scratch's size, FATTN_STATIC_SCRATCH_BYTES (so the
-same way of summing dQ: the whole split when it fits, else the split by chunks of (b, h) at
-d <= 64, else turns): bit-identical dQ, dK, dV on two calls in a row, the second on a smaller
+fattn_bwd_f32 with a caller's workspace of the scratch's size, FATTN_STATIC_SCRATCH_BYTES (the split
+size where it fits, else at d <= 64 that of some (b, h) pairs, else the minimum): bit-identical dQ, dK, dV on two calls in a row, the second on a smaller
 shape, causal and not, the first and last (b, h) pair of every call against the fp64 oracle
 (normwise 2e-6, as every parity test), and the refusal of a shape whose minimum workspace exceeds
 the scratch (before any launch)."""
@@ -82,8 +81,8 @@ def check_against_oracle(orc, got, io, h, d, causal, pairs):
 @pytest.mark.parametrize("causal", [False, True])
 def test_noalloc_matches_workspace_entry(orc, cuda, causal):
     # (b, h, s, d): split fits the scratch, then a smaller split shape; the config-2 shape (its
-    # split workspace exceeds the scratch: split by chunks), then a smaller one; head_dim 32 and
-    # 128 (the latter past the scratch: turns).
+    # split size exceeds the scratch: that of some pairs), then a smaller one; head_dim 32 and 128
+    # (the latter past the scratch: the minimum).
     cases = [((4, 6, 240, 64), (2, 3, 97, 64)),
              ((64, 6, 240, 64), (8, 6, 200, 64)),
              ((2, 4, 333, 32), (1, 2, 65, 32)),
@@ -117,8 +116,7 @@ def test_noalloc_under_graph_capture(cuda, shape):
     """The no-alloc backward is for callers under HIP graph capture: the forward and
     fattn_bwd_f32_noalloc captured in one graph and replayed on new inputs (with eager work and
     synchronisations between replays) equal eager fattn_bwd_f32 runs with a workspace of the
-    scratch's size (config 2's shape: the split by chunks, several launches captured; the smaller
-    one: the whole split), bit for bit."""
+    scratch's size (the first shape's split size exceeds it, the other's does not), bit for bit."""
     b, h, s = shape
     d = 64
     L = _lib.lib()
