@@ -459,7 +459,7 @@ def summarize_counters(csvs: list[str], warmup: int, steps: int, cfg: int = 2) -
     against that; waves per SIMD = 4 SQ_WAVE_CYCLES (quad-cycles) / (GPU-busy cycles x 1024
     SIMDs); non-MFMA VALU issue (4 cycles an instruction) as a share of SIMD cycles; per MFMA
     instruction: other VALU, SALU, LDS, transcendental instructions; executed MFMA GFLOP (512 FLOP
-    per F32 MOPS unit); wave time waiting on a dependency (SQ_WAIT_ANY: memory, LDS, barrier),
+    per F16 or F32 MOPS unit); wave time waiting on a dependency (SQ_WAIT_ANY: memory, LDS, barrier),
     waiting to issue (SQ_WAIT_INST_ANY: its pipe busy with other waves) and issuing
     (SQ_ACTIVE_INST_ANY) as shares of the waves' cycles. Printed as a markdown table."""
     per: dict[str, dict[str, list[float]]] = {}
@@ -516,8 +516,9 @@ def summarize_counters(csvs: list[str], warmup: int, steps: int, cfg: int = 2) -
                              ("SQ_INSTS_VMEM", "vector memory per MFMA")):
                 if k in c:
                     out[label] = c[k] / mfma
-        if "SQ_INSTS_VALU_MFMA_MOPS_F32" in c:
-            out["MFMA GFLOP executed"] = c["SQ_INSTS_VALU_MFMA_MOPS_F32"] * 512 / 1e9
+        mops = [c[k] for k in ("SQ_INSTS_VALU_MFMA_MOPS_F16", "SQ_INSTS_VALU_MFMA_MOPS_F32") if k in c]
+        if mops:
+            out["MFMA GFLOP executed"] = sum(mops) * 512 / 1e9
         if c.get("SQ_WAVE_CYCLES"):
             for k, label in (("SQ_WAIT_ANY", "wave cycles waiting (%)"),
                              ("SQ_WAIT_INST_ANY", "wave cycles waiting to issue (%)"),

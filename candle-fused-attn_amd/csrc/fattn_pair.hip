@@ -756,8 +756,11 @@ fwd_pair_kernel(FwdArgs a) {
 // S and dP are computed in both: seven products where one kind of workgroup would need five, but
 // then dQ's partial sums (4 s^2 b h bytes) would go through memory and dS through LDS, between
 // barriers. Backward, against that scheme on the fp32 matrix instruction (five products): b64 h6 s240
-// 97 us (147), causal 86 (93), causal b8 h12 s2048 611 (1096), b16 h16 s1024 796 (1373), d 128
-// b64 h6 s240 231 (319).
+// 92 us (147), causal 81 (93), causal b8 h12 s2048 630 (1096), b16 h16 s1024 808 (1373), d 128
+// b64 h6 s240 234 (319). Where walks are short and the blocks many it loses at d 128: one wave per SIMD,
+// so that nothing runs beside a block's first loads and last stores: causal, 1024 (b, h), s 65
+// 192 us (132), s 128 277 (228), s 200 572 (466), even at s 400; without a mask even at s 65.
+// (Workgroups of two waves that walk need 124 registers more than there are: s 200 669.)
 // Bounds, b64 h6 s240 (per call): 8.8 us per 32-row step of the walk, about half of it the matrix
 // cores, the rest the softmax, the splits and the staging between them; 35 us for the own rows in,
 // the first tiles and the gradients out (past the L2s 239 MB are read, each operand by both kinds of
