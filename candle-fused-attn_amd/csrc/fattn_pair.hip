@@ -661,14 +661,14 @@ fwd_pair_kernel(FwdArgs a) {
         float to = wsc[n], alpha = 1.0f;
         if (!(pair_sum(psum) <= kRowTop) && ref > m[n]) {
           alpha = m[n] == kNegInf ? 0.0f : exp2_hw(m[n] - ref);
-          to = alpha > 0x1p-100f ? fminf(to * pow2(-exponent(alpha)), kMaxScale) : kMaxScale;
+          to = alpha > 0.0f ? fminf(to * pow2(-exponent(alpha)), kMaxScale) : kMaxScale;
           m[n] = ref;
           lsum[n] *= alpha;
           exps();
         }
         wmax = pair_max(fmaxf(wmax, 0.0f));
         if (wmax * to > kMaxWeight) to = pow2(kWTop - exponent(wmax));
-        const float f = alpha > 0x1p-100f ? alpha * (to / wsc[n]) : 0.0f;
+        const float f = alpha > 0.0f ? alpha * (to / wsc[n]) : 0.0f;
         wsc[n] = to;
 #pragma unroll
         for (int dt = 0; dt < kDT; ++dt) acc[n][dt] *= f;

@@ -124,3 +124,17 @@ def test_rows_of_every_size(cuda, d, grow):
     for causal in (False, True):
         for name, r in everything(q, k, v, g, scale, causal).items():
             check_rows(f"sizes {grow} d{d} causal={causal} {name}", r, bar(8))
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("logit", [60.0, 76.0])
+def test_late_sink(cuda, logit, d, causal):
+    """A sink of value zero after tiles of ordinary keys, which its weight makes as small as 2^-110: what
+    was summed before it is not dropped."""
+    s, at, scale = 300, 130, 1.0 / math.sqrt(d)
+    q, k, v, g = (normal(280 + i, 2, s, d) for i in range(4))
+    with_logit(q, k, at, logit, scale)
+    v[:, at] = 0
+    for name, r in everything(q, k, v, g, scale, causal).items():
+        check_rows(f"late sink {logit} d{d} causal={causal} {name}", r, bar(logit + math.log(s)))
