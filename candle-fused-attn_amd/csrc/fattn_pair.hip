@@ -22,10 +22,12 @@
 // the staged rows, into the weights (P, dS). The weights of a lane's own row follow a power of two
 // of their own, which puts the largest term of the sum at 2^6 or more: 22 bits down to 2^-9 of it,
 // below that an error of 2^-31 of it, and none that depends on a row that has no part in the sum. (One
-// scale per tile, or the largest so far, costs less: forward b64 h6 s240 28.9 us against 30.3, b16 h16
-// s1024 200 against 220, with inputs of deviation 2, whose weights move the scales more often, 203
+// scale serves all D columns of it: where the heavy rows are exactly 0 in a column, the light ones' sum
+// there has the error too. More range would take the low terms' products into sums of their own.)
+// One scale per tile, or the largest so far, costs less: forward b64 h6 s240 28.9 us against 30.3, b16
+// h16 s1024 200 against 220, with inputs of deviation 2, whose weights move the scales more often, 203
 // against 242; backward 92 against 94 and 792 against 808, d 128 228 against 235. But one large row,
-// masked or not, or one key of large weight, takes the bits of all the others.)
+// masked or not, or one key of large weight, takes the bits of all the others.
 //
 // For one v_mfma_f32_32x32x16_f16, lane l (j = l % 32, g = l / 32) supplies A[j][8 g + e] and
 // B[8 g + e][j], e = 0..7, and holds D[8 (r / 4) + 4 g + r % 4][j], r = 0..15. As the contraction

@@ -32,7 +32,9 @@
  *     fp32 operand held as the sum of two f16 under a power-of-two scale of its row (head_dim
  *     values: 22 bits or more of each above 2^-17 of the row's largest, below that 2^-39 of it),
  *     and are summed in fp32. Softmax weights, and dS, times the scale of the row they weigh, are
- *     held the same way under a scale of the sum they enter. A 32-row group whose result is not
+ *     held the same way under a scale of the sum they enter (22 bits of each above 2^-9 of the
+ *     largest, below that 2^-31 of it; one scale for all head_dim columns, so a column in which the
+ *     heavily weighted rows are exactly 0 has that error too). A 32-row group whose result is not
  *     finite is computed again in plain fp32. Results are bit-identical from run to run.
  */
 #ifndef FATTN_H
