@@ -23,7 +23,7 @@
 // of their own, which puts the largest term of the sum at 2^6 or more: 22 bits down to 2^-9 of it,
 // below that an error of 2^-31 of it, and none that depends on a row that has no part in the sum. (One
 // scale serves all D columns of it: where the heavy rows are exactly 0 in a column, the light ones' sum
-// there has the error too. More range would take the low terms' products into sums of their own.)
+// there has the error too.)
 // One scale per tile, or the largest so far, costs less: forward b64 h6 s240 28.9 us against 30.3, b16
 // h16 s1024 200 against 220, with inputs of deviation 2, whose weights move the scales more often, 203
 // against 242; backward 92 against 94 and 792 against 808, d 128 228 against 235. But one large row,
